@@ -29,8 +29,8 @@ HBM_PEAK_GBPS = 8000.0
 MEASURED_TRAFFIC_BYTES = {
     ("cfg3", "direct"): (536914021, "direct_allreduce_bisect_8x32MiB_hbm_traffic.md"),
     ("cfg4", "direct"): (167799218, "direct_allreduce_bisect_8x32MiB_hbm_traffic.md"),
-    ("cfg5_32MiB", "wire"): (1498284599, "wire_allreduce_flag_words_8x32MiB.md"),
-    ("cfg3", "wire"): (1501431833, "wire_allreduce_flag_words_8x32MiB.md"),
+    ("cfg5_32MiB", "wire"): (536903576, "wire_allreduce_through_lds_8x32MiB.md"),
+    ("cfg3", "wire"): (536909720, "wire_allreduce_through_lds_8x32MiB.md"),
 }
 
 

@@ -332,7 +332,7 @@ hipError_t launch_xcc_probe(hipStream_t s, uint32_t blocks, uint32_t *out_device
 // Residency cap of a one-trip grid.  The hardware places as many work-groups on a
 // CU as registers and LDS allow; a launch that wants at most `wgs` there asks for
 // so much dynamic LDS (never touched) that one more would not fit.  0 = no cap.
-static uint32_t lds_cap_bytes(const DeviceInfo &dev, int wgs) {
+uint32_t lds_cap_bytes(const DeviceInfo &dev, int wgs) {
   if (wgs <= 0 || dev.lds_per_cu == 0) return 0;
   if (wgs > 12) wgs = 12;
   // 15/16 of an equal share: `wgs` shares fit with room for allocation granules,
@@ -344,7 +344,7 @@ static uint32_t lds_cap_bytes(const DeviceInfo &dev, int wgs) {
 
 // A kernel may ask for more than 48 KiB of dynamic LDS only after its limit has been
 // raised, once per kernel and device.
-static hipError_t allow_dynamic_lds(const void *kernel, const DeviceInfo &dev, uint32_t bytes) {
+hipError_t allow_dynamic_lds(const void *kernel, const DeviceInfo &dev, uint32_t bytes) {
   const int device = dev.device;
   if (bytes <= 48u * 1024u) return hipSuccess;
   static std::mutex lock;

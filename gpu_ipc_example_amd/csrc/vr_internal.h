@@ -83,6 +83,12 @@ hipError_t launch_copy(hipStream_t s, const DeviceInfo &dev, const Tuning &t, vo
                        const void *src, size_t bytes, int mode = 0);
 
 
+// Residency cap of a launch: bytes of dynamic LDS (never touched) with which at most `wgs`
+// work-groups share a compute unit; 0 = no cap.  And the allowance a kernel needs before
+// it may ask for more than 48 KiB.
+uint32_t lds_cap_bytes(const DeviceInfo &dev, int wgs);
+hipError_t allow_dynamic_lds(const void *kernel, const DeviceInfo &dev, uint32_t bytes);
+
 hipError_t launch_xcc_probe(hipStream_t s, uint32_t blocks, uint32_t *out_device);
 
 // Wire transport ------------------------------------------------------------------
@@ -133,6 +139,21 @@ uint32_t wire_slot_bytes(WireFormat fmt, int vec_halves);
 // and `flag_bytes` bytes of flag words at `flag_off`.
 hipError_t launch_wire_clear_sinks(hipStream_t s, const PtrTable &scatter, const PtrTable &gather, int nranks,
                                    size_t slot_bytes, size_t flag_off, size_t flag_bytes);
+// A launch that holds all ranks: the messages of a column travel through one compute
+// unit's LDS (vr_wire_group.hip).  How inputs are loaded and outputs stored:
+enum GroupPolicy : int {
+  GROUP_RESIDENT = 0,  // cached loads, cached stores
+  GROUP_MIXED = 1,     // cached loads, streaming stores written through at agent scope
+  GROUP_STREAM = 2,    // streaming loads, streaming stores written through
+};
+struct GroupPlan {
+  GroupPolicy policy;
+  int unroll;       // 16-byte vectors per lane and message: 1, or 2 at 8 and 16 ranks
+  int wgs_per_cu;   // residency cap, 0 = none
+};
+hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow, int nranks, DType dtype,
+                             const PtrTable &in, const PtrTable &out, size_t chunk_bytes, const GroupPlan &plan,
+                             uint32_t spin_limit, uint32_t *status);
 // The library's own fixed scratch region in device memory (one per GPU, held
 // until the process ends): its device address on the current device and its size.
 constexpr uint32_t kStaticWiresPerRank = 32;

@@ -1,4 +1,6 @@
-// Wire transport: the reference's message-passing stage structure on one GPU.
+// Wire transport: the reference's message-passing stage structure on one GPU, sinks in
+// memory.  (A call that holds all ranks and asks for nothing special keeps its messages
+// in LDS instead: vr_wire_group.hip.)
 //
 // One persistent kernel holds the work-groups of ALL virtual ranks (block b
 // belongs to rank b % N), or of a group of consecutive ranks (WireArgs::rank_first,

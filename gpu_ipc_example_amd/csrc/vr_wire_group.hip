@@ -1,0 +1,430 @@
+// Wire transport, launches that hold all ranks: messages through a compute unit's LDS.
+//
+// The waves of one wire column talk to nobody but each other: one wave per rank,
+// N waves.  When a launch holds all N ranks those N waves are made ONE work-group,
+// so they share a compute unit and its LDS, and the sinks of the column's ranks
+// live there: message slots and flag words at work-group scope, no scratch in
+// device memory, no polling across the chip, no co-residency demand on the grid.
+// The stages stay the reference's: every wave loads its own rank's input only,
+// scatters messages into the owners' sinks, the owner polls the flags, adds in the
+// protocol's order and gathers the sum into its peers' sinks, and every wave stores
+// its own rank's output only (parallel_transmit.hpp:63-131, sequential_transmit.hpp:
+// 83-207, 429-516, simple_transmit.hpp:16-179, bisect_transmit.hpp:286-424).
+// Launches that hold some of the ranks keep their sinks in memory (vr_wire.hip).
+//
+// What bounds it: HBM, like the direct transport.  Messages through memory cost 2.75
+// times the algorithmic bytes at the L2 / fabric boundary, which carries about
+// 8 TB/s however much of it the memory-side cache serves; here only inputs and
+// outputs cross it.  ParallelTransmit, 8 ranks in place: 256 MiB per rank
+// 2196 -> 688 us (6.2 TB/s), 1 MiB per rank 14.4 -> 5.6 us (the host's pace);
+// RingTransmit, 4 x 8 MB: 39.3 -> 11.4 us; ring all-gather, 8 x 1 MB: 51 -> 13 us.
+//
+// One wire per work-group and no loop: the hardware starts work-groups in index
+// order, so a launch sweeps the chunks front to back with all compute units close
+// together (as the direct transport's one-trip grids).  A wave's message is U x 16
+// bytes per lane; the host picks U and the cache policies (group_plan).
+//
+// Polls are bounded as there: after `spin_limit` unsuccessful polls (or once another
+// wave has given up) a wave records a time-out in the status word and runs to its
+// end without waiting again.
+
+#include <hip/hip_ext.h>
+
+#include "vr_internal.h"
+
+namespace vr {
+
+namespace {
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// Cache policies of the accesses to inputs and outputs (see vr_direct.hip).
+constexpr int kStreamLoad = 2;        // nt
+constexpr int kStreamStore = 2 | 16;  // nt sc1
+
+struct Args {
+  PtrTable in, out;
+  size_t chunk_bytes;     // bytes per rank-chunk (all-gather: of one slice)
+  uint32_t spin_limit;
+  uint32_t *status;       // non-zero once any poll gave up
+};
+
+struct Poll {
+  uint32_t limit;
+  uint32_t *status;
+  bool dead;
+  // Waits until `ready` holds in every lane.
+  template <typename F>
+  __device__ __forceinline__ void until(F &&ready) {
+    if (dead) return;
+    uint32_t polls = 0;
+    while (!__all(ready())) {
+      ++polls;
+      if (polls >= limit || ((polls & 63u) == 0 &&
+                             __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+        dead = true;
+        __hip_atomic_store(status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  }
+};
+
+// One message: U x 16 bytes per lane.
+template <int U>
+struct Msg {
+  u32x4 d[U];
+};
+
+// A wave's piece of a rank's buffer: the bytes that remain of the chunk at the
+// wire's offset, behind a buffer resource (accesses beyond it return zero / are
+// dropped, dword by dword, so a chunk may end inside a lane's 16 bytes).
+template <int U>
+static __device__ __forceinline__ __amdgpu_buffer_rsrc_t piece(const void *base, size_t at, size_t off, size_t chunk) {
+  const size_t left = chunk - off;
+  const uint32_t n = left < 1024u * U ? (uint32_t)left : 1024u * U;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(static_cast<const char *>(base) + at + off), 0, (int)n,
+                                           0x00020000);
+}
+template <int U, int LD>
+static __device__ __forceinline__ Msg<U> load(__amdgpu_buffer_rsrc_t rs, uint32_t lane) {
+  Msg<U> m;
+#pragma unroll
+  for (int u = 0; u < U; ++u) m.d[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, (u * 64u + lane) * 16u, 0, LD);
+  return m;
+}
+template <int U, int ST>
+static __device__ __forceinline__ void store(__amdgpu_buffer_rsrc_t rs, uint32_t lane, const Msg<U> &m) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) __builtin_amdgcn_raw_buffer_store_b128(m.d[u], rs, (u * 64u + lane) * 16u, 0, ST);
+}
+// v = m + v, the received message on the left (rt64_128.hpp:947-957)
+template <int DT, int U>
+static __device__ __forceinline__ void add(Msg<U> &v, const Msg<U> &m) {
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    v.d[u] = __builtin_bit_cast(u32x4, vadd<DT>(__builtin_bit_cast(h8, m.d[u]), __builtin_bit_cast(h8, v.d[u])));
+}
+
+// The sinks of a column: SLOTS message slots and FLAGS flag words in LDS.
+template <int U, int SLOTS, int FLAGS>
+struct Sinks {
+  static constexpr uint32_t kBytes = SLOTS * U * 1024u + FLAGS * 4u;
+  u32x4 *slots;
+  uint32_t *flags;
+  uint32_t lane;
+  __device__ __forceinline__ Sinks(u32x4 *lds, uint32_t lane_) : slots(lds), lane(lane_) {
+    flags = reinterpret_cast<uint32_t *>(lds + SLOTS * U * 64);
+    if (threadIdx.x < (uint32_t)FLAGS) flags[threadIdx.x] = 0;   // never more than the work-group has lanes
+  }
+  // All waves' flag words are zero from here on.
+  static __device__ __forceinline__ void ready() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  }
+  __device__ __forceinline__ void put(int slot, const Msg<U> &m) const {
+#pragma unroll
+    for (int u = 0; u < U; ++u) slots[(slot * U + u) * 64 + lane] = m.d[u];
+  }
+  __device__ __forceinline__ Msg<U> get(int slot) const {
+    Msg<U> m;
+#pragma unroll
+    for (int u = 0; u < U; ++u) m.d[u] = slots[(slot * U + u) * 64 + lane];
+    return m;
+  }
+  // What was put before is in the slots once the flag can be seen.
+  static __device__ __forceinline__ void publish() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local"); }
+  __device__ __forceinline__ void raise(int flag, uint32_t value) const {
+    if (lane == 0) __hip_atomic_store(flags + flag, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __device__ __forceinline__ uint32_t look(int flag) const {
+    return __hip_atomic_load(flags + flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  // Raises / awaits, with one access by the first N lanes, the N flag words from `first`
+  // on except number `self`.
+  template <int N>
+  __device__ __forceinline__ void raise_others(int first, int self, int stride = 1) const {
+    if (lane < (uint32_t)N && (int)lane != self)
+      __hip_atomic_store(flags + first + (int)lane * stride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  template <int N>
+  __device__ __forceinline__ void await_others(Poll &poll, int first, int self, int stride = 1) const {
+    poll.until([&] { return lane >= (uint32_t)N || (int)lane == self || look(first + (int)lane * stride) != 0; });
+  }
+};
+
+#define VR_GROUP_PROLOGUE                                                                    \
+  extern __shared__ u32x4 lds[];                                                              \
+  const uint32_t lane = threadIdx.x & 63u;                                                    \
+  const int r = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));                      \
+  Poll poll{a.spin_limit, a.status, false};                                                   \
+  const size_t chunk = a.chunk_bytes, off = (size_t)blockIdx.x * (1024u * U)
+
+// ---- ParallelTransmit (parallel_transmit.hpp:63-131) -----------------------------------
+// Row y of the grid sweeps chunk y; the wave of rank y owns the column's reduction.
+// Peer p's slot carries its message to the owner and then the owner's sum back.
+template <int N, int U>
+using ParallelSinks = Sinks<U, N, 2 * N>;
+
+template <int N, int DT, int U, int LD, int ST>
+__global__ __launch_bounds__(64 * N) void k_group_parallel(Args a) {
+  VR_GROUP_PROLOGUE;
+  const ParallelSinks<N, U> sk(lds, lane);
+  const int y = (int)blockIdx.y;
+  Msg<U> v = load<U, LD>(piece<U>(a.in.p[r], y * chunk, off, chunk), lane);
+  sk.ready();
+  if (r != y) {
+    sk.put(r, v);
+    sk.publish();
+    sk.raise(r, 1);
+    poll.until([&] { return sk.look(N + r) != 0; });
+    v = sk.get(r);
+  } else {
+    sk.template await_others<N>(poll, 0, r);
+    Msg<U> m[N - 1];
+#pragma unroll
+    for (int i = 0; i < N - 1; ++i) m[i] = sk.get((r + i + 1) % N);
+#pragma unroll
+    for (int i = 0; i < N - 1; ++i) add<DT, U>(v, m[i]);     // peers in order rank+1, rank+2, ...
+#pragma unroll
+    for (int i = 0; i < N - 1; ++i) sk.put((r + i + 1) % N, v);
+    sk.publish();
+    sk.template raise_others<N>(N, r);
+  }
+  store<U, ST>(piece<U>(a.out.p[r], y * chunk, off, chunk), lane, v);
+}
+
+// ---- SequentialTransmit, SimpleTransmit (sequential_transmit.hpp:83-207, simple_transmit.hpp:16-179) ----
+// One wave does everything its rank owes a column, peer after peer.  The slot of the
+// pair (owner, peer) carries the peer's message to the owner and then the owner's sum back.
+template <int N, int U>
+using SequentialSinks = Sinks<U, N * N, 2 * N * N>;
+
+template <int N, int DT, int U, int LD, int ST>
+__global__ __launch_bounds__(64 * N) void k_group_sequential(Args a) {
+  VR_GROUP_PROLOGUE;
+  const SequentialSinks<N, U> sk(lds, lane);
+  Msg<U> x[N];                                             // x[i]: chunk of rank r + i
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(piece<U>(a.in.p[r], (r + i) % N * chunk, off, chunk), lane);
+  sk.ready();
+#pragma unroll
+  for (int i = 1; i < N; ++i) sk.put((r + i) % N * N + r, x[i]);
+  sk.publish();
+  sk.template raise_others<N>(r, r, N);                    // flag owner * N + r
+  Msg<U> v = x[0];
+  sk.template await_others<N>(poll, r * N, r);
+#pragma unroll
+  for (int i = 1; i < N; ++i) x[i] = sk.get(r * N + (r + i) % N);
+#pragma unroll
+  for (int i = 1; i < N; ++i) add<DT, U>(v, x[i]);         // peers in order rank+1, rank+2, ...
+#pragma unroll
+  for (int i = 1; i < N; ++i) sk.put(r * N + (r + i) % N, v);
+  sk.publish();
+  sk.template raise_others<N>(N * N + r * N, r);           // flag owner r, peer
+  store<U, ST>(piece<U>(a.out.p[r], r * chunk, off, chunk), lane, v);
+  sk.template await_others<N>(poll, N * N + r, r, N);
+#pragma unroll
+  for (int i = 1; i < N; ++i) x[i] = sk.get((r + i) % N * N + r);
+#pragma unroll
+  for (int i = 1; i < N; ++i) store<U, ST>(piece<U>(a.out.p[r], (r + i) % N * chunk, off, chunk), lane, x[i]);
+}
+
+// ---- RingTransmit (sequential_transmit.hpp:429-516) --------------------------------------
+// A rank's sink is a ring of kRingDepth slots fed by its predecessor.  Flag r counts
+// the messages delivered to rank r, flag N + r those it has taken out, which is what
+// its predecessor looks at before it reuses a slot.
+constexpr int kRingDepth = 2;
+template <int N, int U>
+using RingSinks = Sinks<U, N * kRingDepth, 2 * N>;
+
+template <int N, int U>
+struct Ring {
+  const RingSinks<N, U> &sk;
+  Poll &poll;
+  int r, next;
+  __device__ __forceinline__ void send(int k, const Msg<U> &m) const {
+    if (k >= kRingDepth) poll.until([&] { return sk.look(N + next) >= (uint32_t)(k - kRingDepth + 1); });
+    sk.put(next * kRingDepth + k % kRingDepth, m);
+    sk.publish();
+    sk.raise(next, (uint32_t)(k + 1));
+  }
+  __device__ __forceinline__ Msg<U> recv(int k) const {
+    poll.until([&] { return sk.look(r) >= (uint32_t)(k + 1); });
+    const Msg<U> m = sk.get(r * kRingDepth + k % kRingDepth);
+    sk.publish();
+    sk.raise(N + r, (uint32_t)(k + 1));
+    return m;
+  }
+};
+
+template <int N, int DT, int U, int LD, int ST>
+__global__ __launch_bounds__(64 * N) void k_group_ring(Args a) {
+  VR_GROUP_PROLOGUE;
+  const RingSinks<N, U> sk(lds, lane);
+  Msg<U> x[N];                                             // x[i]: chunk of rank r - i
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(piece<U>(a.in.p[r], (r + N - i) % N * chunk, off, chunk), lane);
+  const Ring<N, U> ring{sk, poll, r, (r + 1) % N};
+  sk.ready();
+  ring.send(0, x[0]);
+#pragma unroll
+  for (int i = 1; i < N; ++i) {                            // reduce and forward; the last add starts the gather ring
+    add<DT, U>(x[i], ring.recv(i - 1));
+    ring.send(i, x[i]);
+  }
+  store<U, ST>(piece<U>(a.out.p[r], (r + 1) % N * chunk, off, chunk), lane, x[N - 1]);
+#pragma unroll
+  for (int i = 1; i < N; ++i) {                            // write back, forward except on the last hop
+    const Msg<U> v = ring.recv(N - 2 + i);
+    if (i < N - 1) ring.send(N - 1 + i, v);
+    store<U, ST>(piece<U>(a.out.p[r], (r + 1 + N - i) % N * chunk, off, chunk), lane, v);
+  }
+}
+
+template <int N, int DT, int U, int LD, int ST>
+__global__ __launch_bounds__(64 * N) void k_group_allgather(Args a) {
+  VR_GROUP_PROLOGUE;
+  const RingSinks<N, U> sk(lds, lane);
+  Msg<U> v = load<U, LD>(piece<U>(a.in.p[r], 0, off, chunk), lane);
+  const Ring<N, U> ring{sk, poll, r, (r + 1) % N};
+  const char *own = static_cast<const char *>(a.out.p[r]) + r * chunk;
+  sk.ready();
+  ring.send(0, v);
+  // the own slot needs no store when it is the input (sequential_transmit.hpp:496-497)
+  if (own != a.in.p[r]) store<U, ST>(piece<U>(a.out.p[r], r * chunk, off, chunk), lane, v);
+#pragma unroll
+  for (int i = 1; i < N; ++i) {
+    v = ring.recv(i - 1);
+    if (i < N - 1) ring.send(i, v);
+    store<U, ST>(piece<U>(a.out.p[r], (r + N - i) % N * chunk, off, chunk), lane, v);
+  }
+}
+
+// ---- BisectPTransmit (bisect_transmit.hpp:286-424) -----------------------------------------
+// Row y of the grid sweeps chunk y of both halves.  Slot r (far): the pair's message to
+// rank r, then r's sum back to the pair.  Slot N + r (close): r's pair sum to the owner,
+// then the owner's sum back.
+template <int N, int U>
+using BisectSinks = Sinks<U, 2 * N, 4 * N>;
+
+template <int N, int DT, int U, int LD, int ST>
+__global__ __launch_bounds__(64 * N) void k_group_bisect(Args a) {
+  constexpr int B = N / 2;
+  VR_GROUP_PROLOGUE;
+  const BisectSinks<N, U> sk(lds, lane);
+  const int y = (int)blockIdx.y, h = r & 1, l = r >> 1, pair = r ^ 1;
+  const size_t close = (size_t)(h * B + y) * chunk, far = (size_t)((1 - h) * B + y) * chunk;
+  const Msg<U> f = load<U, LD>(piece<U>(a.in.p[r], far, off, chunk), lane);
+  Msg<U> v = load<U, LD>(piece<U>(a.in.p[r], close, off, chunk), lane);
+  sk.ready();
+  sk.put(pair, f);                                         // scatterFar
+  sk.publish();
+  sk.raise(pair, 1);
+  poll.until([&] { return sk.look(r) != 0; });
+  add<DT, U>(v, sk.get(r));                                // pair sum
+  if (y != l) {
+    sk.put(N + r, v);                                      // scatterClose to the owner, rank 2y + h
+    sk.publish();
+    sk.raise(N + r, 1);
+    poll.until([&] { return sk.look(2 * N + r) != 0; });
+    v = sk.get(N + r);
+  } else {
+    sk.template await_others<B>(poll, N + h, l, 2);
+    Msg<U> m[B - 1];
+#pragma unroll
+    for (int i = 0; i < B - 1; ++i) m[i] = sk.get(N + (r + 2 * i + 2) % N);
+#pragma unroll
+    for (int i = 0; i < B - 1; ++i) add<DT, U>(v, m[i]);   // pair sums in order l+1, l+2, ...
+#pragma unroll
+    for (int i = 0; i < B - 1; ++i) sk.put(N + (r + 2 * i + 2) % N, v);
+    sk.publish();
+    sk.template raise_others<B>(2 * N + h, l, 2);
+  }
+  sk.put(r, v);                                            // forward to the pair
+  sk.publish();
+  sk.raise(3 * N + pair, 1);
+  store<U, ST>(piece<U>(a.out.p[r], close, off, chunk), lane, v);
+  poll.until([&] { return sk.look(3 * N + r) != 0; });     // pollFarGatherOutput
+  store<U, ST>(piece<U>(a.out.p[r], far, off, chunk), lane, sk.get(pair));
+}
+
+#undef VR_GROUP_PROLOGUE
+
+struct Pick {
+  const void *fn;
+  uint32_t rows, lds;   // rows of the grid, bytes of LDS the sinks take
+};
+
+template <int N, int DT, int LD, int ST, int U>
+Pick pick_flow(WireFlow flow) {
+  if constexpr (N <= 8) {
+    switch (flow) {
+      case WIRE_PARALLEL: return {reinterpret_cast<const void *>(&k_group_parallel<N, DT, U, LD, ST>), N, ParallelSinks<N, U>::kBytes};
+      case WIRE_SEQUENTIAL:
+      case WIRE_SIMPLE: return {reinterpret_cast<const void *>(&k_group_sequential<N, DT, U, LD, ST>), 1, SequentialSinks<N, U>::kBytes};
+      case WIRE_RING: return {reinterpret_cast<const void *>(&k_group_ring<N, DT, U, LD, ST>), 1, RingSinks<N, U>::kBytes};
+      case WIRE_ALLGATHER:   // no adds: one instantiation serves both element types
+        if constexpr (U == 1)
+          return {reinterpret_cast<const void *>(&k_group_allgather<N, DT_F16, U, LD, ST>), 1, RingSinks<N, U>::kBytes};
+        break;
+      default: break;
+    }
+  }
+  if constexpr (N >= 4) {
+    if (flow == WIRE_BISECT) return {reinterpret_cast<const void *>(&k_group_bisect<N, DT, U, LD, ST>), N / 2, BisectSinks<N, U>::kBytes};
+  }
+  return {nullptr, 0, 0};
+}
+
+template <int DT, int LD, int ST>
+Pick pick_ranks(WireFlow flow, int nranks, int unroll) {
+  switch (nranks) {
+    case 2: return pick_flow<2, DT, LD, ST, 1>(flow);
+    case 4: return pick_flow<4, DT, LD, ST, 1>(flow);
+    case 8: return unroll == 2 ? pick_flow<8, DT, LD, ST, 2>(flow) : pick_flow<8, DT, LD, ST, 1>(flow);
+    case 16: return unroll == 2 ? pick_flow<16, DT, LD, ST, 2>(flow) : pick_flow<16, DT, LD, ST, 1>(flow);
+    default: return {nullptr, 0, 0};
+  }
+}
+
+template <int LD, int ST>
+Pick pick_type(WireFlow flow, int nranks, DType dtype, int unroll) {
+  return dtype == DT_BF16 ? pick_ranks<DT_BF16, LD, ST>(flow, nranks, unroll)
+                          : pick_ranks<DT_F16, LD, ST>(flow, nranks, unroll);
+}
+
+}  // namespace
+
+hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow, int nranks, DType dtype,
+                             const PtrTable &in, const PtrTable &out, size_t chunk_bytes, const GroupPlan &plan,
+                             uint32_t spin_limit, uint32_t *status) {
+  if (chunk_bytes == 0) return hipSuccess;
+  const Pick k = plan.policy == GROUP_STREAM     ? pick_type<kStreamLoad, kStreamStore>(flow, nranks, dtype, plan.unroll)
+                 : plan.policy == GROUP_RESIDENT ? pick_type<0, 0>(flow, nranks, dtype, plan.unroll)
+                                                 : pick_type<0, kStreamStore>(flow, nranks, dtype, plan.unroll);
+  if (!k.fn) return hipErrorInvalidValue;
+  const size_t wire = 1024u * (size_t)(nranks >= 8 ? plan.unroll : 1);   // payload of one wave
+  const size_t wires = (chunk_bytes + wire - 1) / wire;
+  if (wires > 0x7fffffffull) return hipErrorInvalidValue;
+  Args a;
+  a.in = in;
+  a.out = out;
+  a.chunk_bytes = chunk_bytes;
+  a.spin_limit = spin_limit;
+  a.status = status;
+  uint32_t lds = k.lds;
+  const uint32_t cap = lds_cap_bytes(dev, plan.wgs_per_cu);
+  if (cap > lds) lds = cap;
+  if (hipError_t e = allow_dynamic_lds(k.fn, dev, lds); e != hipSuccess) return e;
+  void *kargs[] = {&a};
+  const dim3 grid((uint32_t)wires, k.rows), block(64u * (uint32_t)nranks);
+  if (tl_kernel_events.start || tl_kernel_events.stop)
+    return hipExtLaunchKernel(k.fn, grid, block, kargs, lds, s, tl_kernel_events.start, tl_kernel_events.stop, 0);
+  return hipLaunchKernel(k.fn, grid, block, kargs, lds, s);
+}
+
+}  // namespace vr

@@ -89,6 +89,73 @@ static int wire_clear(const WireSinks &k, int nranks, hipStream_t s) {
   return VR_OK;
 }
 
+// May this launch take the work-group form (vr_wire_group.hip)?  It holds all ranks, and
+// nothing asks for a particular message format, launch or grid.
+static bool takes_group_form(const vr_ctx *c, uint32_t user_wires) {
+  const TuningOverrides &t = c->tune;
+  return user_wires == 0 && t.wire_fenced == -1 && t.wire_cooperative == -1 && t.wire_blocks_per_cu == -1 &&
+         t.wire_ahead == -1 && t.wire_msg16 == -1 && t.wire_stream_io == -1;
+}
+
+static uint32_t spin_limit_of(const vr_ctx *c) {
+  const uint64_t limit = c->spin_limit ? c->spin_limit : kDefaultSpinLimit;
+  return limit > 0xffffffffull ? 0xffffffffu : (uint32_t)limit;
+}
+
+// Launch shape of the work-group form.  `reads` = bytes of all ranks' inputs.
+static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_place) {
+  const size_t MiB = (size_t)1 << 20;
+  GroupPlan p = {GROUP_MIXED, 1, 0};
+  // Cache policies, us per pass on one / three / ten sets of buffers in turn:
+  //  * in place up to 64 MiB everything stays cacheable (8 x 4 MiB 9.1 / 12.9 / 16.0, streamed
+  //    13.9 / 15.9 / 15.9; 4 x 16 MiB 22.2 / 21.9 / 26.8 against 25.1 / 24.8 / 24.5), beyond it
+  //    streaming wins as soon as the buffers do not all fit the memory-side cache
+  //    (8 x 16 MiB 39.5 / 50.5 / 53.2 against 49.9 / 48.9 / 49.4);
+  //  * out of place, and all-gather, up to half the memory-side cache of inputs: results
+  //    are streamed past inputs that may stay (8 x 16 MiB 41.3 / 49.3 / 50.5, everything
+  //    streamed 50.2 / 50.2 / 49.4), beyond it everything streams (8 x 128 MiB 355, 351 us).
+  if (in_place) p.policy = reads <= 64 * MiB ? GROUP_RESIDENT : GROUP_STREAM;
+  else if (reads > 128 * MiB) p.policy = GROUP_STREAM;
+  // Two vectors per lane at 8 and 16 ranks, where that is the faster (fewer waves for the
+  // same bytes where the caches feed them quicker than waves start; at 2 and 4 ranks one vector
+  // is 10 to 40 % faster at every size):
+  switch (flow) {
+    case WIRE_PARALLEL:
+      // 8 x 4 MiB 16.6 -> 12.9 us, 8 x 8 MiB 27.4 -> 23.0; 8 x 16 MiB is better off with one
+      // (50.5, two: 55.5).  From 512 MiB on with three work-groups per CU, 48 KiB of loads
+      // in flight: 8 x 64 MiB 173.9 -> 168.7 us, 8 x 256 MiB 720 -> 689; 8 x 48 MiB 132.2, two: 133.1.
+      if (nranks == 8 && reads <= 64 * MiB) p.unroll = 2;
+      if (nranks == 8 && reads >= 512 * MiB) p.unroll = 2, p.wgs_per_cu = 3;
+      break;
+    case WIRE_BISECT:
+      // 8 x 4 MiB 15.2 -> 11.8 us, 8 x 2 and 8 x 8 MiB even; 16 x 4 MiB 29.8 -> 22.0 us,
+      // 16 x 8 MiB 53.8, two: 57.4
+      p.unroll = nranks == 8 ? (reads >= 16 * MiB && reads < 64 * MiB ? 2 : 1) : nranks == 16 && reads <= 96 * MiB ? 2 : 1;
+      break;
+    case WIRE_RING:
+    case WIRE_SEQUENTIAL:
+    case WIRE_SIMPLE:
+      // ring 8 x 16 MiB 65.1 -> 48.9 us, sequential 65.6 -> 46.8; 8 x 4 MiB even, 8 x 2 MiB
+      // 8.4, two: 9.9; 8 x 32 MiB 97.7, two: 108.8
+      if (nranks == 8 && reads >= 32 * MiB && reads <= 192 * MiB) p.unroll = 2;
+      break;
+    default: break;   // all-gather 8 x 4 MiB: 49.0, two: 59.1 us
+  }
+  return p;
+}
+
+static int group_launch(vr_ctx *c, hipStream_t s, const AlgoInfo *a, const PtrTable &in, const PtrTable &out,
+                        size_t chunk_bytes) {
+  const int N = c->nranks;
+  const WireFlow flow = a->wire_flow();
+  bool in_place = !a->allgather;
+  for (int r = 0; r < N; ++r) in_place = in_place && in.p[r] == out.p[r];
+  const size_t reads = (size_t)N * chunk_bytes * (a->allgather ? 1 : N);
+  const hipError_t e = launch_wire_group(s, c->dev, flow, N, c->dtype, in, out, chunk_bytes,
+                                         group_plan(flow, N, reads, in_place), spin_limit_of(c), c->status);
+  return e == hipSuccess ? VR_OK : fail_hip(e, "launch_wire_group");
+}
+
 struct WireLaunch {
   const WireSinks *sinks;
   WireHistory *hist;      // null: the caller owns the sinks and the sequence numbers (rank-group launches)
@@ -231,6 +298,13 @@ static int wire_launch(vr_ctx *c, hipStream_t s, const AlgoInfo *a, const PtrTab
                                   "are per-launch kernel arguments (capture the direct transport)");
     (void)hipGetLastError();
   }
+  // Sinks the library owns (a launch against a caller's sinks leaves its messages there).
+  // No flag value outlives the launch; one is counted as used, as for the shortest launch.
+  if ((wlch.hist || wlch.always_clear) && takes_group_form(c, user_wires)) {
+    *flags_used = chunk_bytes ? 1u : 0u;
+    if (seq + *flags_used == 0) *seq_io = 1;   // 0 is never handed out
+    return group_launch(c, s, a, in, out, chunk_bytes);
+  }
   WirePlan plan;
   if (int rc = plan_wire(c, a, chunk_bytes, vec_halves, user_wires, k, &plan)) return rc;
   *flags_used = plan.flags_used;
@@ -285,8 +359,7 @@ static int wire_launch(vr_ctx *c, hipStream_t s, const AlgoInfo *a, const PtrTab
   args.chunk_bytes = chunk_bytes;
   args.waves_per_rank = wpr;
   args.seq = seq;
-  const uint64_t limit = c->spin_limit ? c->spin_limit : kDefaultSpinLimit;
-  args.spin_limit = limit > 0xffffffffull ? 0xffffffffu : (uint32_t)limit;
+  args.spin_limit = spin_limit_of(c);
   args.status = wlch.status;
   args.ahead = c->tune.wire_ahead > 0 ? (uint32_t)c->tune.wire_ahead : kWireAhead;
   args.io_narrow = wlch.io_narrow ? 1u : 0u;

@@ -91,16 +91,22 @@ typedef enum vr_algo {
  *          in place, add in the protocol's order, and write every rank's output.
  *          One pass over HBM; no scratch, no flags.  Default for every algo
  *          except VR_ALGO_PARALLEL.
- *  WIRE  : the reference's stage structure — scatter into the owner's sink,
- *          reduce, gather into every peer's sink — through the context's scratch,
- *          one persistent kernel whose workgroups are partitioned between the
- *          virtual ranks.  Receivers learn of a message from a flag: the reference's
- *          flag inside every message (Rt64, Rt64_PCIE, and on request Rt64_128 /
- *          Rt64_128_PCIE byte for byte), or one flag word per message beside full
- *          payload lines, every access at agent scope (what the Rt64_128 families of
- *          the all-to-all flows take when left alone; see "wire_fenced").  This is
- *          the form that carries over to several GPUs.  Default for
- *          VR_ALGO_PARALLEL. */
+ *  WIRE  : the reference's stage structure — every rank's waves load their own input
+ *          only, scatter into the owner's sink, reduce, gather into every peer's sink
+ *          and store their own output only; receivers learn of a message from a flag.
+ *          Default for VR_ALGO_PARALLEL.  Two forms:
+ *          - a call that holds all ranks and leaves every "wire_*" setting and the grid
+ *            to the library: the N waves of a wire column (one per rank) are one
+ *            work-group and the sinks lie in its compute unit's LDS, flag words at
+ *            work-group scope;
+ *          - everything else (launches that hold some of the ranks, a user grid, any
+ *            "wire_*" setting): sinks in scratch memory, one persistent kernel whose
+ *            work-groups are partitioned between the ranks.  Flags are the reference's,
+ *            inside every message (Rt64, Rt64_PCIE, and on request Rt64_128 /
+ *            Rt64_128_PCIE byte for byte), or one flag word per message beside full
+ *            payload lines, every access at agent scope (what the Rt64_128 families of
+ *            the all-to-all flows take when left alone; see "wire_fenced").  This is
+ *            the form that carries over to several GPUs. */
 typedef enum vr_transport {
   VR_TRANSPORT_DEFAULT = 0,
   VR_TRANSPORT_DIRECT = 1,
@@ -281,7 +287,8 @@ int vr_ipc_barrier(int rank, int world, const char *instance, int generation);
  * VR_ERR_INVALID.  Every context on a GPU shares that GPU's region and each call
  * first clears the message slots it is about to use (a fill kernel on `stream`),
  * so calls that overlap in time on one GPU race: keep them on one stream or
- * otherwise ordered.  A time-out is recorded in the calling context's own status
+ * otherwise ordered.  (A call whose context leaves every "wire_*" setting alone keeps
+ * its messages in LDS: it neither touches the region nor clears anything.)  A time-out is recorded in the calling context's own status
  * word and reported by vr_ctx_check like those of vr_allreduce. */
 int vr_allreduce_static(vr_ctx *ctx, void *stream, int algo, void *const bufs[], void *const outs[],
                         size_t nelems);
@@ -328,7 +335,8 @@ int vr_ctx_set_spin_limit(vr_ctx *ctx, uint64_t polls);
  * binary32 and rounded back after every add: the same bits, a longer ALU section),
  * "segment_kib" (KiB of a chunk one launch
  * covers; chunks longer than this, at most 1 GiB, take several launches);
- * for the wire transport "wire_fenced" (how the Rt64_128 families, i.e. simple,
+ * for the wire transport, where setting any of them also moves launches that hold all
+ * ranks from LDS to scratch memory, "wire_fenced" (how the Rt64_128 families, i.e. simple,
  * bisect, parallel, simple_pcie_p, simple_ring, simple_pcie, simple_transmit,
  * tell a receiver that a message is there: 0 = the reference's 128 / 256-byte
  * messages with a flag in every 64 bytes; 1 = full payload lines and a separate

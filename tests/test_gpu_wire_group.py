@@ -1,0 +1,77 @@
+"""Wire-transport launches that hold all ranks (messages through LDS) at the sizes where
+the work-group form can go wrong, bit for bit against the oracle.  A wave's wire is 1 KiB
+of a chunk, 2 KiB where a lane carries two vectors (parallel at 8 ranks up to 64 MiB and
+from 512 MiB of inputs, bisect at 16, ring and sequential at 8 from 32 MiB); a chunk of
+8-byte messages may end inside a lane's 16 bytes."""
+import numpy as np
+import pytest
+
+import gpu_ipc_example_amd as vr
+from gpu_ipc_example_amd.binding import DeviceBuffer
+from tests.oracle_lib import BF16, DIST_NORMAL, F16
+from tests.test_gpu_wire import run_allgather_wire
+
+pytestmark = pytest.mark.gpu
+WIRE = vr.TRANSPORT_WIRE
+
+
+def run(oracle, ctx, algo, n, dtype, inplace, offset, seed):
+    N = ctx.nranks
+    ctx.set_dtype(1 if dtype == BF16 else 0)
+    ins = [oracle.generate_dt(dtype, n, seed + r, DIST_NORMAL, 0.0, 1.0) for r in range(N)]
+    want = oracle.order_dt(dtype, 2 if algo == "bisect" else 1, ins)
+    what = (algo, N, n, dtype, inplace, offset)
+    src = [DeviceBuffer(n * 2 + 64) for _ in range(N)]
+    dst = src if inplace else [DeviceBuffer(n * 2 + 64) for _ in range(N)]
+    for b in src + dst:
+        b.fill(0xAB)
+    for b, a in zip(src, ins):
+        b.upload(a, offset)
+    ctx.allreduce(algo, [b.ptr + offset for b in src], n,
+                  outs=None if inplace else [b.ptr + offset for b in dst], transport=WIRE)
+    ctx.check()
+    for r, b in enumerate(dst):
+        got = b.download(np.uint16, n + 32)
+        assert oracle.count_mismatch_dt(dtype, got[offset // 2:offset // 2 + n], want) == 0, (what, r)
+        # nothing is written around the buffer
+        assert (got[:offset // 2] == 0xABAB).all() and (got[offset // 2 + n:] == 0xABAB).all(), (what, r)
+    for b in src + (dst if dst is not src else []):
+        b.free()
+
+
+@pytest.mark.parametrize("nranks,algo", [(2, "simple"), (4, "parallel"), (8, "parallel"), (8, "simple_transmit"),
+                                         (4, "bisect"), (8, "bisect"), (16, "bisect"), (2, "simple_ring"),
+                                         (8, "simple_ring"), (8, "simple_pcie")])
+def test_edges_of_a_wire(oracle, nranks, algo):
+    msg = 16 if algo in ("simple_ring", "simple_pcie") else 8
+    ctx = vr.VirtualRanks(nranks)
+    for k, chunk in enumerate((msg, 1024 - msg, 1024, 1024 + msg, 2048 - msg, 2048, 2048 + msg, 5 * 2048 + 3 * msg)):
+        for dtype in (F16, BF16):
+            for inplace in (True, False):
+                for offset in (0, 8) if msg == 8 else (0,):
+                    run(oracle, ctx, algo, nranks * chunk // 2, dtype, inplace, offset, 40_000 + 100 * k)
+    ctx.close()
+
+
+@pytest.mark.parametrize("algo,mib", [("simple_ring", 34), ("simple_pcie", 34), ("bisect", 20), ("parallel", 66),
+                                      ("parallel", 514)])
+def test_ragged_sizes_of_the_larger_launches(oracle, algo, mib):
+    """Eight ranks, just inside the sizes that change the vectors per lane, the residency and
+    (in place) the cache policy."""
+    ctx = vr.VirtualRanks(8)
+    msg = 16 if algo in ("simple_ring", "simple_pcie") else 8
+    chunk = (mib << 20) // 64 + 3 * msg
+    run(oracle, ctx, algo, 8 * chunk // 2, F16, True, 0, 50_000)
+    ctx.close()
+
+
+@pytest.mark.parametrize("nranks", [2, 8])
+def test_allgather_edges(oracle, nranks):
+    ctx = vr.VirtualRanks(nranks)
+    for n in (8, 504, 512, 520, 8 * 643):
+        ins = [oracle.generate_dt(F16, n, 60_000 + r, DIST_NORMAL, 0.0, 1.0) for r in range(nranks)]
+        want = oracle.allgather(ins)
+        for alias in (False, True):
+            for r, got in enumerate(run_allgather_wire(ctx, "allgather_simple", ins, alias)):
+                assert (got == want).all(), (n, r, alias)
+    ctx.close()
