@@ -601,7 +601,7 @@ static int run_allreduce(vr_ctx *ctx, hipStream_t s, const Prepared &p, int tran
     return VR_OK;
   }
   hipError_t e = launch_direct_allreduce(s, ctx->dev, t, ctx->nranks, p.a->order, ctx->dtype, p.in,
-                                         p.out, p.chunk_elems, p.vec_halves);
+                                         p.out, p.chunk_elems);
   if (e != hipSuccess) return fail_hip(e, "launch_direct_allreduce");
   return VR_OK;
 }
@@ -722,7 +722,7 @@ static int run_allgather(vr_ctx *ctx, hipStream_t s, const PreparedGather &p, in
     return VR_OK;
   }
   if (transport != VR_TRANSPORT_DEFAULT && transport != VR_TRANSPORT_DIRECT) return fail(VR_ERR_INVALID, "bad transport");
-  hipError_t e = launch_direct_allgather(s, ctx->dev, t, ctx->nranks, p.in, p.out, nelems, p.vec_halves);
+  hipError_t e = launch_direct_allgather(s, ctx->dev, t, ctx->nranks, p.in, p.out, nelems);
   if (e != hipSuccess) return fail_hip(e, "launch_direct_allgather");
   *next_seq = seq_no + p.geom.steps;
   if (*next_seq == 0) *next_seq = 1;
@@ -1009,7 +1009,7 @@ extern "C" int vr_stream_probe_multi(vr_ctx *ctx, void *stream, void *const dsts
   const size_t all = (size_t)N * bytes_each;
   const Tuning t = tuning_for(ctx, &kAlgos[VR_ALGO_BISECT], all, all, false);
   hipError_t e = launch_direct_allreduce((hipStream_t)stream, ctx->dev, t, N, ORDER_COPY, DT_F16, in, out,
-                                         bytes_each / 2 / (size_t)N, 8);
+                                         bytes_each / 2 / (size_t)N);
   return e == hipSuccess ? VR_OK : fail_hip(e, "launch_direct_allreduce (copy yardstick)");
 }
 

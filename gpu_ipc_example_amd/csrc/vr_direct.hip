@@ -40,7 +40,6 @@ namespace vr {
 thread_local KernelEvents tl_kernel_events;
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
@@ -58,20 +57,47 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, uint3
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
 }
 
-template <typename V, int AUX>
-__device__ __forceinline__ V ld(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  if constexpr (sizeof(V) == 16)
-    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, AUX));
-  else
-    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, AUX));
+template <int AUX>
+__device__ __forceinline__ h8 ld(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, AUX));
 }
 
-template <typename V, int AUX>
-__device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off, V v) {
-  if constexpr (sizeof(V) == 16)
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off, 0, AUX);
-  else
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, AUX);
+template <int AUX>
+__device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off, h8 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off, 0, AUX);
+}
+
+// Half a vector.
+template <int AUX>
+__device__ __forceinline__ h8 ld_low(__amdgpu_buffer_rsrc_t r) {
+  const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, AUX);
+  return __builtin_bit_cast(h8, u32x4{w.x, w.y, 0u, 0u});
+}
+template <int AUX>
+__device__ __forceinline__ void st_low(__amdgpu_buffer_rsrc_t r, h8 v) {
+  const u32x4 w = __builtin_bit_cast(u32x4, v);
+  __builtin_amdgcn_raw_buffer_store_b64(u32x2{w.x, w.y}, r, 0, 0, AUX);
+}
+
+// Where the tiles of a chunk lie.  Chunks may start at any multiple of 8 bytes, but tiles
+// are laid on 128-byte lines of the outputs and vectors on 16 bytes: a tile that starts
+// inside a line makes two work-groups, on two XCDs, write parts of it.  (With 8 bytes per
+// lane and tiles counted from the chunk's start: bisect, 16 x 12 MB bfloat16 of odd length
+// 112.5 us, now 69.8; simple, 4 x 20 MB in place 26.0, now 23.8.)
+//   head: bytes (0 or 8) of the chunk ahead of its first whole vector.  `head_mask` is 0 where
+//         the buffers disagree modulo 16: then a lane's 16 bytes are 8-byte aligned in some
+//         of them, which the hardware takes.
+//   skew: bytes of the first tile's line below the first vector; lanes there form offsets
+//         below zero, which are beyond the buffer's length like those of the last tile.
+struct TileStart {
+  uint32_t head, skew;
+};
+// `lines` (lines_of): place of the first output in its line, and head_mask in the second
+// byte: an argument of its own, so that nothing waits for the pointer table.
+__device__ __forceinline__ TileStart tile_start(uint32_t lines, size_t base) {
+  const uint32_t at = (lines & 0xffu) + (uint32_t)base;
+  const uint32_t head = at & (lines >> 8);
+  return {head, (at + head) & 112u};
 }
 
 // The chunk a protocol owner reduces.
@@ -152,18 +178,18 @@ __device__ __forceinline__ int owner_of_group(int x) {
 
 // Sum of the N operands in the protocol's association.  The received message is
 // always the left operand of the add (rt64_128.hpp:951-956).
-template <int N, int ORDER, int DT, typename V>
-__device__ __forceinline__ V reduce_operands(const V (&x)[N]) {
+template <int N, int ORDER, int DT>
+__device__ __forceinline__ h8 reduce_operands(const h8 (&x)[N]) {
   if constexpr (ORDER == ORDER_ROTATED) {
-    V acc = x[0];
+    h8 acc = x[0];
 #pragma unroll
     for (int k = 1; k < N; ++k) acc = vadd<DT>(x[k], acc);
     return acc;
   } else {
-    V acc = vadd<DT>(x[1], x[0]);
+    h8 acc = vadd<DT>(x[1], x[0]);
 #pragma unroll
     for (int k = 2; k < N; k += 2) {
-      const V pair = vadd<DT>(x[k + 1], x[k]);
+      const h8 pair = vadd<DT>(x[k + 1], x[k]);
       acc = vadd<DT>(pair, acc);
     }
     return acc;
@@ -172,12 +198,12 @@ __device__ __forceinline__ V reduce_operands(const V (&x)[N]) {
 
 // One launch covers bytes [seg_off, seg_off + seg_bytes) of every chunk;
 // chunk_pitch is the full chunk length (the distance between chunk starts).
-template <int N, int ORDER, int DT, typename V, int UNROLL, int LD_AUX, int ST_AUX>
+template <int N, int ORDER, int DT, int UNROLL, int LD_AUX, int ST_AUX>
 __global__ __launch_bounds__(1024) void k_direct_allreduce(PtrTable in, PtrTable out,
                                                            size_t chunk_pitch, size_t seg_off,
                                                            uint32_t seg_bytes,
                                                            uint32_t blocks_per_rank, uint32_t deal_log2,
-                                                           uint32_t row) {
+                                                           uint32_t row, uint32_t lines) {
   // 2^deal_log2 chunks ("deal") are worked on at a time: row y of the grid, deal *
   // blocks_per_rank work-groups, belongs to owners y * deal ... y * deal + deal - 1,
   // round robin (rows are dispatched one after the other).  deal = N: work-group b
@@ -186,7 +212,10 @@ __global__ __launch_bounds__(1024) void k_direct_allreduce(PtrTable in, PtrTable
   const uint32_t deal = 1u << deal_log2;
   const int owner = owner_of_group<N, ORDER>((int)(blockIdx.y * deal + (blockIdx.x & (deal - 1))));
   const uint32_t jblock = blockIdx.x >> deal_log2;
-  const size_t base = (size_t)chunk_of_owner<N, ORDER>(owner) * chunk_pitch + seg_off;
+  size_t base = (size_t)chunk_of_owner<N, ORDER>(owner) * chunk_pitch + seg_off;
+  const TileStart ts = tile_start(lines, base);
+  base += ts.head;
+  seg_bytes -= ts.head;
 
   const char *op[N];
   select_operands<N, ORDER>(in, owner, op);
@@ -196,49 +225,62 @@ __global__ __launch_bounds__(1024) void k_direct_allreduce(PtrTable in, PtrTable
     src[k] = make_rsrc(op[k] + base, seg_bytes);
     dst[k] = make_rsrc(static_cast<char *>(out.p[k]) + base, seg_bytes);
   }
-  const uint32_t lane = threadIdx.x * (uint32_t)sizeof(V);
-  // `row` = bytes one unroll step spans, blockDim.x * sizeof(V): an argument, so that it
+  const uint32_t lane = threadIdx.x * 16u - ts.skew;
+  // `row` = bytes one unroll step spans, blockDim.x * 16: an argument, so that it
   // arrives with the others instead of through a separate load of the launch's dimensions
   const uint32_t tile = row * UNROLL;
   const uint32_t stride = tile * blocks_per_rank;
   // Every work-group has a first tile (the host launches at most one work-group per tile),
   // so the loop tests at its end and nothing separates the kernel's argument loads.
   uint32_t t = jblock * tile;
+  const uint32_t end = seg_bytes + ts.skew;
   do {
-    V x[UNROLL][N];
+    h8 x[UNROLL][N];
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
-      for (int k = 0; k < N; ++k) x[u][k] = ld<V, LD_AUX>(src[k], t + u * row + lane);
+      for (int k = 0; k < N; ++k) x[u][k] = ld<LD_AUX>(src[k], t + u * row + lane);
     // Every load of the trip is issued before the first add waits for one: left to
     // itself the scheduler may hold a load back behind the adds of earlier operands,
     // which puts a whole memory latency into the trip (measured: +4 us on 83).  (Not
     // where a trip's loads alone fill 64 registers or more: pinned there, they spill.)
-    if constexpr (UNROLL * N * sizeof(V) <= 256) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (UNROLL * N * 16 <= 256) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       if constexpr (ORDER == ORDER_COPY) {
         // the all-reduce's N read streams and N write streams with the adds removed
 #pragma unroll
-        for (int k = 0; k < N; ++k) st<V, ST_AUX>(dst[k], t + u * row + lane, x[u][k]);
+        for (int k = 0; k < N; ++k) st<ST_AUX>(dst[k], t + u * row + lane, x[u][k]);
       } else {
-        const V acc = reduce_operands<N, ORDER, DT, V>(x[u]);
+        const h8 acc = reduce_operands<N, ORDER, DT>(x[u]);
 #pragma unroll
-        for (int k = 0; k < N; ++k) st<V, ST_AUX>(dst[k], t + u * row + lane, acc);
+        for (int k = 0; k < N; ++k) st<ST_AUX>(dst[k], t + u * row + lane, acc);
       }
     }
     t += stride;
-  } while (t < seg_bytes);
+  } while (t < end);
+  if constexpr (ORDER != ORDER_COPY) {
+    // The 8 bytes ahead of the first whole vector: one lane of the chunk's first work-group,
+    // after its tiles (a branch beside the stores of the loop cost cache-resident launches 4 %).
+    if (ts.head != 0 && jblock == 0 && threadIdx.x == 0) {
+      h8 x[N];
+#pragma unroll
+      for (int k = 0; k < N; ++k) x[k] = ld_low<LD_AUX>(make_rsrc(op[k] + base - 8, 8));
+      const h8 acc = reduce_operands<N, ORDER, DT>(x);
+#pragma unroll
+      for (int k = 0; k < N; ++k) st_low<ST_AUX>(make_rsrc(static_cast<char *>(out.p[k]) + base - 8, 8), acc);
+    }
+  }
 }
 
 // All-gather: the groups of rank p read p's slice once and store it into slot p
 // of every rank's output (allgather.hpp:79-100 collapsed to one hop).
-template <int N, typename V, int UNROLL, int LD_AUX, int ST_AUX>
+template <int N, int UNROLL, int LD_AUX, int ST_AUX>
 __global__ __launch_bounds__(1024) void k_direct_allgather(PtrTable in, PtrTable out,
                                                            size_t slice_pitch, size_t seg_off,
                                                            uint32_t seg_bytes,
                                                            uint32_t blocks_per_rank, uint32_t deal_log2,
-                                                           uint32_t row) {
+                                                           uint32_t row, uint32_t lines) {
   // 2^deal_log2 source slices are worked on at a time (see k_direct_allreduce): deal = N
   // gives work-group b to source b % N throughout, deal = 1 lets all work-groups sweep
   // one source's slice after the other.
@@ -272,20 +314,22 @@ __global__ __launch_bounds__(1024) void k_direct_allgather(PtrTable in, PtrTable
     // per CU ran up to 20 % slower).
     dst[r] = make_rsrc(d, d == src_ptr ? 0u : seg_bytes);
   }
-  const uint32_t lane = threadIdx.x * (uint32_t)sizeof(V);
+  // every address is a multiple of the 16-byte messages, so no vector straddles a start
+  const TileStart ts = tile_start(lines, (size_t)p * slice_pitch + seg_off);
+  const uint32_t lane = threadIdx.x * 16u - ts.skew;
   const uint32_t tile = row * UNROLL;
   const uint32_t stride = tile * blocks_per_rank;
   uint32_t t = jblock * tile;   // every work-group has a first tile, as in k_direct_allreduce
   do {
-    V x[UNROLL];
+    h8 x[UNROLL];
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) x[u] = ld<V, LD_AUX>(src, t + u * row + lane);
+    for (int u = 0; u < UNROLL; ++u) x[u] = ld<LD_AUX>(src, t + u * row + lane);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
-      for (int r = 0; r < N; ++r) st<V, ST_AUX>(dst[r], t + u * row + lane, x[u]);
+      for (int r = 0; r < N; ++r) st<ST_AUX>(dst[r], t + u * row + lane, x[u]);
     t += stride;
-  } while (t < seg_bytes);
+  } while (t < seg_bytes + ts.skew);
 }
 
 // Streaming yardsticks over one segment: MODE 0 copies, 1 only reads (the sum is
@@ -301,17 +345,17 @@ __global__ __launch_bounds__(1024) void k_probe(char *dst_ptr, const char *src_p
     h8 x[UNROLL];
     if constexpr (MODE != 2) {
 #pragma unroll
-      for (int u = 0; u < UNROLL; ++u) x[u] = ld<h8, LD_AUX>(src, t + u * row + lane);
+      for (int u = 0; u < UNROLL; ++u) x[u] = ld<LD_AUX>(src, t + u * row + lane);
     }
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      if constexpr (MODE == 0) st<h8, ST_AUX>(dst, t + u * row + lane, x[u]);
+      if constexpr (MODE == 0) st<ST_AUX>(dst, t + u * row + lane, x[u]);
       if constexpr (MODE == 1) acc = acc + x[u];
-      if constexpr (MODE == 2) st<h8, ST_AUX>(dst, t + u * row + lane, acc);
+      if constexpr (MODE == 2) st<ST_AUX>(dst, t + u * row + lane, acc);
     }
   }
   if constexpr (MODE == 1) {
-    if (acc[0] == (_Float16)12345.0f && acc[7] == (_Float16)-321.0f) st<h8, kAuxCached>(dst, 0, acc);
+    if (acc[0] == (_Float16)12345.0f && acc[7] == (_Float16)-321.0f) st<kAuxCached>(dst, 0, acc);
   }
 }
 
@@ -400,30 +444,48 @@ static hipError_t with_policy(const Tuning &t, F &&f) {
   return hipErrorInvalidValue;
 }
 
-template <int N, int ORDER, int DT, typename V, int UNROLL>
+// Bytes the tiles of a chunk may have to start early to lie on the outputs' lines (tile_start).
+static size_t skew_of(const PtrTable &out, size_t pitch, size_t seg_off) {
+  return (((uintptr_t)out.p[0] | pitch | seg_off) & 127u) ? 120 : 0;
+}
+
+uint32_t lines_of(const PtrTable &out, uint32_t head_mask) {
+  return ((uint32_t)(uintptr_t)out.p[0] & 127u) | head_mask << 8;
+}
+
+// 8 where a chunk that starts in the middle of 16 bytes does so in every buffer, else 0.
+uint32_t head_mask_of(int nranks, const PtrTable &in, const PtrTable &out) {
+  uintptr_t differ = 0;
+  for (int r = 0; r < nranks; ++r)
+    differ |= ((uintptr_t)in.p[r] ^ (uintptr_t)out.p[0]) | ((uintptr_t)out.p[r] ^ (uintptr_t)out.p[0]);
+  return (differ & 15u) ? 0u : 8u;
+}
+
+template <int N, int ORDER, int DT, int UNROLL>
 static hipError_t launch_ar_segments(hipStream_t s, const DeviceInfo &dev, const Tuning &t,
                                      const PtrTable &in, const PtrTable &out, size_t chunk_bytes) {
-  const uint32_t row = (uint32_t)(t.block * sizeof(V));   // bytes one unroll step of a work-group spans
+  const uint32_t row = (uint32_t)t.block * 16u;   // bytes one unroll step of a work-group spans
   const size_t tile = (size_t)row * UNROLL;
   const size_t seg_max = segment_of(t);
   const uint32_t lds = lds_cap_bytes(dev, t.wgs_per_cu);
   // chunks dealt at a time: a divisor of N, N itself unless the launch says otherwise
   const uint32_t deal = (t.deal > 0 && t.deal <= N && N % t.deal == 0) ? (uint32_t)t.deal : (uint32_t)N;
+  const uint32_t lines = lines_of(out, ORDER == ORDER_COPY ? 0u : head_mask_of(N, in, out));
   const uint32_t deal_log2 = (uint32_t)__builtin_ctz(deal);   // N is a power of two, so are its divisors
   for (size_t off = 0; off < chunk_bytes; off += seg_max) {
     const size_t seg = chunk_bytes - off < seg_max ? chunk_bytes - off : seg_max;
-    const uint32_t bpr = blocks_per_rank_for(dev, t, N, seg, tile);
+    const uint32_t bpr = blocks_per_rank_for(dev, t, N, seg + skew_of(out, chunk_bytes, off), tile);
     const dim3 grid(bpr * deal, N / deal), block(t.block);
     // kernel-attached profiling events: start on the first segment, stop on the last
     hipEvent_t ev0 = off == 0 ? tl_kernel_events.start : nullptr;
     hipEvent_t ev1 = off + seg >= chunk_bytes ? tl_kernel_events.stop : nullptr;
     hipError_t e = with_policy(t, [&](auto ld_aux, auto st_aux) {
-      auto kernel = k_direct_allreduce<N, ORDER, DT, V, UNROLL, decltype(ld_aux)::value, decltype(st_aux)::value>;
+      auto kernel = k_direct_allreduce<N, ORDER, DT, UNROLL, decltype(ld_aux)::value, decltype(st_aux)::value>;
       if (hipError_t a = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), dev, lds); a != hipSuccess) return a;
       if (ev0 || ev1)
-        hipExtLaunchKernelGGL(kernel, grid, block, lds, s, ev0, ev1, 0, in, out, chunk_bytes, off, (uint32_t)seg, bpr, deal_log2, row);
+        hipExtLaunchKernelGGL(kernel, grid, block, lds, s, ev0, ev1, 0, in, out, chunk_bytes, off, (uint32_t)seg, bpr, deal_log2, row, lines);
       else
-        hipLaunchKernelGGL(kernel, grid, block, lds, s, in, out, chunk_bytes, off, (uint32_t)seg, bpr, deal_log2, row);
+        hipLaunchKernelGGL(kernel, grid, block, lds, s, in, out, chunk_bytes, off, (uint32_t)seg, bpr, deal_log2, row, lines);
       return hipGetLastError();
     });
     if (e != hipSuccess) return e;
@@ -431,7 +493,7 @@ static hipError_t launch_ar_segments(hipStream_t s, const DeviceInfo &dev, const
   return hipSuccess;
 }
 
-template <int N, int ORDER, int DT, typename V>
+template <int N, int ORDER, int DT>
 static hipError_t launch_ar_unroll(hipStream_t s, const DeviceInfo &dev, const Tuning &t,
                                    const PtrTable &in, const PtrTable &out, size_t chunk_bytes) {
   // 16 ranks already keep 16 loads per lane in flight; the bfloat16 add needs
@@ -440,44 +502,34 @@ static hipError_t launch_ar_unroll(hipStream_t s, const DeviceInfo &dev, const T
   if constexpr (N <= 8) {
     // (the no-add yardstick at eight ranks would hold 128 registers of loaded data: two vectors at most)
     if constexpr (DT == DT_F16 && !(ORDER == ORDER_COPY && N == 8))
-      if (unroll == 4) return launch_ar_segments<N, ORDER, DT, V, 4>(s, dev, t, in, out, chunk_bytes);
-    if (unroll >= 2) return launch_ar_segments<N, ORDER, DT, V, 2>(s, dev, t, in, out, chunk_bytes);
+      if (unroll == 4) return launch_ar_segments<N, ORDER, DT, 4>(s, dev, t, in, out, chunk_bytes);
+    if (unroll >= 2) return launch_ar_segments<N, ORDER, DT, 2>(s, dev, t, in, out, chunk_bytes);
   }
-  return launch_ar_segments<N, ORDER, DT, V, 1>(s, dev, t, in, out, chunk_bytes);
+  return launch_ar_segments<N, ORDER, DT, 1>(s, dev, t, in, out, chunk_bytes);
 }
+
 template <int N, int ORDER>
-static hipError_t launch_ar_vec(hipStream_t s, const DeviceInfo &dev, const Tuning &t, DType dtype,
-                                const PtrTable &in, const PtrTable &out, size_t chunk_elems,
-                                int vec_halves) {
-  const size_t bytes = chunk_elems * 2;
-  if (dtype == DT_BF16) {
-    if (vec_halves == 8) return launch_ar_unroll<N, ORDER, DT_BF16, h8>(s, dev, t, in, out, bytes);
-    return launch_ar_unroll<N, ORDER, DT_BF16, h4>(s, dev, t, in, out, bytes);
-  }
-  if (vec_halves == 8) {
-    if (t.f16_wide) return launch_ar_unroll<N, ORDER, DT_F16_WIDE, h8>(s, dev, t, in, out, bytes);
-    return launch_ar_unroll<N, ORDER, DT_F16, h8>(s, dev, t, in, out, bytes);
-  }
-  return launch_ar_unroll<N, ORDER, DT_F16, h4>(s, dev, t, in, out, bytes);
+static hipError_t launch_ar_type(hipStream_t s, const DeviceInfo &dev, const Tuning &t, DType dtype,
+                                 const PtrTable &in, const PtrTable &out, size_t bytes) {
+  if (dtype == DT_BF16) return launch_ar_unroll<N, ORDER, DT_BF16>(s, dev, t, in, out, bytes);
+  if (t.f16_wide) return launch_ar_unroll<N, ORDER, DT_F16_WIDE>(s, dev, t, in, out, bytes);
+  return launch_ar_unroll<N, ORDER, DT_F16>(s, dev, t, in, out, bytes);
 }
 
 hipError_t launch_direct_allreduce(hipStream_t s, const DeviceInfo &dev, const Tuning &t, int nranks,
                                    Order order, DType dtype, const PtrTable &in, const PtrTable &out,
-                                   size_t chunk_elems, int vec_halves) {
+                                   size_t chunk_elems) {
   if (chunk_elems == 0) return hipSuccess;
   if (t.block < 64 || t.block > 1024 || t.block % 64) return hipErrorInvalidValue;
 #define VR_CASE(NN)                                                                              \
   case NN:                                                                                       \
-    if (order == ORDER_COPY) {                                                                   \
-      if (vec_halves != 8) return hipErrorInvalidValue;                                          \
-      return launch_ar_unroll<NN, ORDER_COPY, DT_F16, h8>(s, dev, t, in, out, chunk_elems * 2);  \
-    }                                                                                            \
+    if (order == ORDER_COPY) return launch_ar_unroll<NN, ORDER_COPY, DT_F16>(s, dev, t, in, out, chunk_elems * 2); \
     if (order == ORDER_BISECT) {                                                                 \
       if constexpr (NN >= 4)                                                                     \
-        return launch_ar_vec<NN, ORDER_BISECT>(s, dev, t, dtype, in, out, chunk_elems, vec_halves);     \
+        return launch_ar_type<NN, ORDER_BISECT>(s, dev, t, dtype, in, out, chunk_elems * 2);     \
       return hipErrorInvalidValue;                                                               \
     }                                                                                            \
-    return launch_ar_vec<NN, ORDER_ROTATED>(s, dev, t, dtype, in, out, chunk_elems, vec_halves);
+    return launch_ar_type<NN, ORDER_ROTATED>(s, dev, t, dtype, in, out, chunk_elems * 2);
   switch (nranks) {
     VR_CASE(2)
     VR_CASE(4)
@@ -489,10 +541,10 @@ hipError_t launch_direct_allreduce(hipStream_t s, const DeviceInfo &dev, const T
 #undef VR_CASE
 }
 
-template <int N, typename V, int UNROLL>
+template <int N, int UNROLL>
 static hipError_t launch_ag_segments(hipStream_t s, const DeviceInfo &dev, const Tuning &t,
                                      const PtrTable &in, const PtrTable &out, size_t slice_bytes) {
-  const uint32_t row = (uint32_t)(t.block * sizeof(V));   // bytes one unroll step of a work-group spans
+  const uint32_t row = (uint32_t)t.block * 16u;   // bytes one unroll step of a work-group spans
   const size_t tile = (size_t)row * UNROLL;
   const size_t seg_max = segment_of(t);
   const uint32_t lds = lds_cap_bytes(dev, t.wgs_per_cu);
@@ -502,17 +554,17 @@ static hipError_t launch_ag_segments(hipStream_t s, const DeviceInfo &dev, const
   if (t.run > 1 && deal == 1 && t.oneshot) deal_log2 |= (uint32_t)__builtin_ctz((unsigned)t.run) << 8;
   for (size_t off = 0; off < slice_bytes; off += seg_max) {
     const size_t seg = slice_bytes - off < seg_max ? slice_bytes - off : seg_max;
-    const uint32_t bpr = blocks_per_rank_for(dev, t, N, seg, tile);
+    const uint32_t bpr = blocks_per_rank_for(dev, t, N, seg + skew_of(out, slice_bytes, off), tile);
     const dim3 grid(bpr * deal, N / deal), block(t.block);
     hipEvent_t ev0 = off == 0 ? tl_kernel_events.start : nullptr;
     hipEvent_t ev1 = off + seg >= slice_bytes ? tl_kernel_events.stop : nullptr;
     hipError_t e = with_policy(t, [&](auto ld_aux, auto st_aux) {
-      auto kernel = k_direct_allgather<N, V, UNROLL, decltype(ld_aux)::value, decltype(st_aux)::value>;
+      auto kernel = k_direct_allgather<N, UNROLL, decltype(ld_aux)::value, decltype(st_aux)::value>;
       if (hipError_t a = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), dev, lds); a != hipSuccess) return a;
       if (ev0 || ev1)
-        hipExtLaunchKernelGGL(kernel, grid, block, lds, s, ev0, ev1, 0, in, out, slice_bytes, off, (uint32_t)seg, bpr, deal_log2, row);
+        hipExtLaunchKernelGGL(kernel, grid, block, lds, s, ev0, ev1, 0, in, out, slice_bytes, off, (uint32_t)seg, bpr, deal_log2, row, lines_of(out, 0));
       else
-        hipLaunchKernelGGL(kernel, grid, block, lds, s, in, out, slice_bytes, off, (uint32_t)seg, bpr, deal_log2, row);
+        hipLaunchKernelGGL(kernel, grid, block, lds, s, in, out, slice_bytes, off, (uint32_t)seg, bpr, deal_log2, row, lines_of(out, 0));
       return hipGetLastError();
     });
     if (e != hipSuccess) return e;
@@ -520,22 +572,19 @@ static hipError_t launch_ag_segments(hipStream_t s, const DeviceInfo &dev, const
   return hipSuccess;
 }
 
-template <int N, typename V>
+template <int N>
 static hipError_t launch_ag(hipStream_t s, const DeviceInfo &dev, const Tuning &t, const PtrTable &in,
                             const PtrTable &out, size_t slice_bytes) {
-  if (t.unroll >= 2) return launch_ag_segments<N, V, 2>(s, dev, t, in, out, slice_bytes);
-  return launch_ag_segments<N, V, 1>(s, dev, t, in, out, slice_bytes);
+  if (t.unroll >= 2) return launch_ag_segments<N, 2>(s, dev, t, in, out, slice_bytes);
+  return launch_ag_segments<N, 1>(s, dev, t, in, out, slice_bytes);
 }
 
 hipError_t launch_direct_allgather(hipStream_t s, const DeviceInfo &dev, const Tuning &t, int nranks,
-                                   const PtrTable &in, const PtrTable &out, size_t nelems,
-                                   int vec_halves) {
+                                   const PtrTable &in, const PtrTable &out, size_t nelems) {
   if (nelems == 0) return hipSuccess;
   if (t.block < 64 || t.block > 1024 || t.block % 64) return hipErrorInvalidValue;
-#define VR_CASE(NN)                                                              \
-  case NN:                                                                       \
-    if (vec_halves == 8) return launch_ag<NN, h8>(s, dev, t, in, out, nelems * 2); \
-    return launch_ag<NN, h4>(s, dev, t, in, out, nelems * 2);
+#define VR_CASE(NN) \
+  case NN: return launch_ag<NN>(s, dev, t, in, out, nelems * 2);
   switch (nranks) {
     VR_CASE(2)
     VR_CASE(4)

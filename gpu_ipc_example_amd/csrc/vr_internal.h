@@ -69,20 +69,22 @@ struct KernelEvents {
 extern thread_local KernelEvents tl_kernel_events;
 
 // Direct transport -----------------------------------------------------------
-// in/out hold nranks pointers; chunk_elems = nelems / nranks; vec_halves is 8
-// (16-byte accesses) or 4 (8-byte accesses, for chunks or pointers that are only
-// 8-byte aligned).
+// in/out hold nranks pointers; chunk_elems = nelems / nranks.  Pointers and chunks are
+// multiples of 8 bytes (all-gather: 16).
 hipError_t launch_direct_allreduce(hipStream_t s, const DeviceInfo &dev, const Tuning &t, int nranks,
                                    Order order, DType dtype, const PtrTable &in, const PtrTable &out,
-                                   size_t chunk_elems, int vec_halves);
+                                   size_t chunk_elems);
 hipError_t launch_direct_allgather(hipStream_t s, const DeviceInfo &dev, const Tuning &t, int nranks,
-                                   const PtrTable &in, const PtrTable &out, size_t nelems,
-                                   int vec_halves);
+                                   const PtrTable &in, const PtrTable &out, size_t nelems);
 // mode: 0 copy, 1 read only, 2 write only
 hipError_t launch_copy(hipStream_t s, const DeviceInfo &dev, const Tuning &t, void *dst,
                        const void *src, size_t bytes, int mode = 0);
 
 
+// 8 where a chunk that starts in the middle of 16 bytes does so in every buffer, else 0.
+uint32_t head_mask_of(int nranks, const PtrTable &in, const PtrTable &out);
+// Place of the first output in its 128-byte line, and head_mask in the second byte.
+uint32_t lines_of(const PtrTable &out, uint32_t head_mask);
 // Residency cap of a launch: bytes of dynamic LDS (never touched) with which at most `wgs`
 // work-groups share a compute unit; 0 = no cap.  And the allowance a kernel needs before
 // it may ask for more than 48 KiB.

@@ -38,14 +38,19 @@ namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 // Cache policies of the accesses to inputs and outputs (see vr_direct.hip).
 constexpr int kStreamLoad = 2;        // nt
 constexpr int kStreamStore = 2 | 16;  // nt sc1
 
+// One launch covers bytes [seg_off, seg_off + seg_bytes) of every chunk.
 struct Args {
   PtrTable in, out;
-  size_t chunk_bytes;     // bytes per rank-chunk (all-gather: of one slice)
+  size_t pitch;           // bytes per rank-chunk (all-gather: of one slice)
+  size_t seg_off;
+  uint32_t seg_bytes;
+  uint32_t lines;         // see lines_of
   uint32_t spin_limit;
   uint32_t *status;       // non-zero once any poll gave up
 };
@@ -78,27 +83,60 @@ struct Msg {
   u32x4 d[U];
 };
 
-// A wave's piece of a rank's buffer: the bytes that remain of the chunk at the
-// wire's offset, behind a buffer resource (accesses beyond it return zero / are
-// dropped, dword by dword, so a chunk may end inside a lane's 16 bytes).
-template <int U>
-static __device__ __forceinline__ __amdgpu_buffer_rsrc_t piece(const void *base, size_t at, size_t off, size_t chunk) {
-  const size_t left = chunk - off;
-  const uint32_t n = left < 1024u * U ? (uint32_t)left : 1024u * U;
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(static_cast<const char *>(base) + at + off), 0, (int)n,
+// Where a chunk lies in every rank's buffer.  As in the direct kernels (tile_start,
+// vr_direct.hip) wires are laid on 128-byte lines of the outputs and vectors on 16 bytes:
+// the first wire may begin up to 112 bytes before the chunk (lanes there form offsets below
+// zero, beyond the buffer's length) and its first vector may straddle the chunk's start:
+// it is loaded whole (the 8 bytes below lie in the same 16 bytes of the same buffer) and its
+// upper half is stored.  A chunk may end inside a vector: the bounds check works dword by
+// dword.  LINED = every chunk starts on a line: none of that (the extra scalar instructions
+// of eight waves per 8 KiB cost 7 % at 8 x 32 MiB).
+template <bool LINED>
+struct Span {
+  size_t at;        // first byte, from the start of a buffer
+  uint32_t bytes;   // length of the buffer resource
+  uint32_t off;     // the lane's offset in it
+  bool straddles;   // the vector at offset 0 begins 8 bytes below the chunk
+};
+template <bool LINED, int U>
+static __device__ __forceinline__ Span<LINED> span_of(const Args &a, uint32_t chunk, uint32_t lane) {
+  const size_t base = chunk * a.pitch + a.seg_off;
+  const uint32_t off = blockIdx.x * (1024u * U) + lane * 16u;
+  if constexpr (LINED) return {base, a.seg_bytes, off, false};
+  const uint32_t addr = (a.lines & 0xffu) + (uint32_t)base, head = addr & (a.lines >> 8);
+  return {base - head, a.seg_bytes + head, off - ((addr - head) & 112u), blockIdx.x == 0 && head != 0};
+}
+template <bool LINED>
+static __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *base, const Span<LINED> &s) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(static_cast<const char *>(base) + s.at), 0, (int)s.bytes,
                                            0x00020000);
 }
-template <int U, int LD>
-static __device__ __forceinline__ Msg<U> load(__amdgpu_buffer_rsrc_t rs, uint32_t lane) {
+// Offset of the lane's vector u, added up in a register: as an immediate of the instruction
+// it would be added after the wrap of a first wire's offset below zero had been compared.
+template <bool LINED>
+static __device__ __forceinline__ uint32_t vec_off(const Span<LINED> &s, int u) {
+  uint32_t off = s.off + (uint32_t)u * 1024u;
+  if (!LINED && u) asm("" : "+v"(off));
+  return off;
+}
+template <int U, int LD, bool LINED>
+static __device__ __forceinline__ Msg<U> load(const void *base, const Span<LINED> &s) {
+  const __amdgpu_buffer_rsrc_t rs = rsrc(base, s);
   Msg<U> m;
 #pragma unroll
-  for (int u = 0; u < U; ++u) m.d[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, (u * 64u + lane) * 16u, 0, LD);
+  for (int u = 0; u < U; ++u) m.d[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, vec_off(s, u), 0, LD);
   return m;
 }
-template <int U, int ST>
-static __device__ __forceinline__ void store(__amdgpu_buffer_rsrc_t rs, uint32_t lane, const Msg<U> &m) {
+template <int U, int ST, bool LINED>
+static __device__ __forceinline__ void store(void *base, const Span<LINED> &s, const Msg<U> &m) {
+  const __amdgpu_buffer_rsrc_t rs = rsrc(base, s);
 #pragma unroll
-  for (int u = 0; u < U; ++u) __builtin_amdgcn_raw_buffer_store_b128(m.d[u], rs, (u * 64u + lane) * 16u, 0, ST);
+  for (int u = 0; u < U; ++u) {
+    if (!LINED && u == 0 && s.straddles && s.off == 0)
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2{m.d[0].z, m.d[0].w}, rs, 8u, 0, ST);
+    else
+      __builtin_amdgcn_raw_buffer_store_b128(m.d[u], rs, vec_off(s, u), 0, ST);
+  }
 }
 // v = m + v, the received message on the left (rt64_128.hpp:947-957)
 template <int DT, int U>
@@ -160,8 +198,12 @@ struct Sinks {
   extern __shared__ u32x4 lds[];                                                              \
   const uint32_t lane = threadIdx.x & 63u;                                                    \
   const int r = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));                      \
-  Poll poll{a.spin_limit, a.status, false};                                                   \
-  const size_t chunk = a.chunk_bytes, off = (size_t)blockIdx.x * (1024u * U)
+  const char *const src = static_cast<const char *>(a.in.p[r]);                               \
+  char *const dst = static_cast<char *>(a.out.p[r]);                                          \
+  /* every argument arrives behind one wait */                                                \
+  asm volatile("" ::"s"(src), "s"(dst), "s"(a.pitch), "s"(a.seg_off), "s"(a.seg_bytes), "s"(a.lines), \
+               "s"(a.spin_limit));                                                            \
+  Poll poll{a.spin_limit, a.status, false}
 
 // ---- ParallelTransmit (parallel_transmit.hpp:63-131) -----------------------------------
 // Row y of the grid sweeps chunk y; the wave of rank y owns the column's reduction.
@@ -169,12 +211,13 @@ struct Sinks {
 template <int N, int U>
 using ParallelSinks = Sinks<U, N, 2 * N>;
 
-template <int N, int DT, int U, int LD, int ST>
+template <int N, int DT, int U, bool LINED, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_parallel(Args a) {
   VR_GROUP_PROLOGUE;
   const ParallelSinks<N, U> sk(lds, lane);
   const int y = (int)blockIdx.y;
-  Msg<U> v = load<U, LD>(piece<U>(a.in.p[r], y * chunk, off, chunk), lane);
+  const auto at = span_of<LINED, U>(a, y, lane);
+  Msg<U> v = load<U, LD>(src, at);
   sk.ready();
   if (r != y) {
     sk.put(r, v);
@@ -194,7 +237,7 @@ __global__ __launch_bounds__(64 * N) void k_group_parallel(Args a) {
     sk.publish();
     sk.template raise_others<N>(N, r);
   }
-  store<U, ST>(piece<U>(a.out.p[r], y * chunk, off, chunk), lane, v);
+  store<U, ST>(dst, at, v);
 }
 
 // ---- SequentialTransmit, SimpleTransmit (sequential_transmit.hpp:83-207, simple_transmit.hpp:16-179) ----
@@ -203,13 +246,13 @@ __global__ __launch_bounds__(64 * N) void k_group_parallel(Args a) {
 template <int N, int U>
 using SequentialSinks = Sinks<U, N * N, 2 * N * N>;
 
-template <int N, int DT, int U, int LD, int ST>
+template <int N, int DT, int U, bool LINED, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_sequential(Args a) {
   VR_GROUP_PROLOGUE;
   const SequentialSinks<N, U> sk(lds, lane);
   Msg<U> x[N];                                             // x[i]: chunk of rank r + i
 #pragma unroll
-  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(piece<U>(a.in.p[r], (r + i) % N * chunk, off, chunk), lane);
+  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<LINED, U>(a, (r + i) % N, lane));
   sk.ready();
 #pragma unroll
   for (int i = 1; i < N; ++i) sk.put((r + i) % N * N + r, x[i]);
@@ -225,12 +268,12 @@ __global__ __launch_bounds__(64 * N) void k_group_sequential(Args a) {
   for (int i = 1; i < N; ++i) sk.put(r * N + (r + i) % N, v);
   sk.publish();
   sk.template raise_others<N>(N * N + r * N, r);           // flag owner r, peer
-  store<U, ST>(piece<U>(a.out.p[r], r * chunk, off, chunk), lane, v);
+  store<U, ST>(dst, span_of<LINED, U>(a, r, lane), v);
   sk.template await_others<N>(poll, N * N + r, r, N);
 #pragma unroll
   for (int i = 1; i < N; ++i) x[i] = sk.get((r + i) % N * N + r);
 #pragma unroll
-  for (int i = 1; i < N; ++i) store<U, ST>(piece<U>(a.out.p[r], (r + i) % N * chunk, off, chunk), lane, x[i]);
+  for (int i = 1; i < N; ++i) store<U, ST>(dst, span_of<LINED, U>(a, (r + i) % N, lane), x[i]);
 }
 
 // ---- RingTransmit (sequential_transmit.hpp:429-516) --------------------------------------
@@ -261,13 +304,13 @@ struct Ring {
   }
 };
 
-template <int N, int DT, int U, int LD, int ST>
+template <int N, int DT, int U, bool LINED, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_ring(Args a) {
   VR_GROUP_PROLOGUE;
   const RingSinks<N, U> sk(lds, lane);
   Msg<U> x[N];                                             // x[i]: chunk of rank r - i
 #pragma unroll
-  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(piece<U>(a.in.p[r], (r + N - i) % N * chunk, off, chunk), lane);
+  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<LINED, U>(a, (r + N - i) % N, lane));
   const Ring<N, U> ring{sk, poll, r, (r + 1) % N};
   sk.ready();
   ring.send(0, x[0]);
@@ -276,31 +319,33 @@ __global__ __launch_bounds__(64 * N) void k_group_ring(Args a) {
     add<DT, U>(x[i], ring.recv(i - 1));
     ring.send(i, x[i]);
   }
-  store<U, ST>(piece<U>(a.out.p[r], (r + 1) % N * chunk, off, chunk), lane, x[N - 1]);
+  store<U, ST>(dst, span_of<LINED, U>(a, (r + 1) % N, lane), x[N - 1]);
 #pragma unroll
   for (int i = 1; i < N; ++i) {                            // write back, forward except on the last hop
     const Msg<U> v = ring.recv(N - 2 + i);
     if (i < N - 1) ring.send(N - 1 + i, v);
-    store<U, ST>(piece<U>(a.out.p[r], (r + 1 + N - i) % N * chunk, off, chunk), lane, v);
+    store<U, ST>(dst, span_of<LINED, U>(a, (r + 1 + N - i) % N, lane), v);
   }
 }
 
-template <int N, int DT, int U, int LD, int ST>
+template <int N, int DT, int U, bool LINED, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_allgather(Args a) {
   VR_GROUP_PROLOGUE;
   const RingSinks<N, U> sk(lds, lane);
-  Msg<U> v = load<U, LD>(piece<U>(a.in.p[r], 0, off, chunk), lane);
+  const auto own = span_of<LINED, U>(a, r, lane);
+  // the input is one slice long: the same bytes of it as of the own slot
+  const char *slot0 = src - (size_t)r * a.pitch;
+  Msg<U> v = load<U, LD>(slot0, own);
   const Ring<N, U> ring{sk, poll, r, (r + 1) % N};
-  const char *own = static_cast<const char *>(a.out.p[r]) + r * chunk;
   sk.ready();
   ring.send(0, v);
   // the own slot needs no store when it is the input (sequential_transmit.hpp:496-497)
-  if (own != a.in.p[r]) store<U, ST>(piece<U>(a.out.p[r], r * chunk, off, chunk), lane, v);
+  if (slot0 != dst) store<U, ST>(dst, own, v);
 #pragma unroll
   for (int i = 1; i < N; ++i) {
     v = ring.recv(i - 1);
     if (i < N - 1) ring.send(i, v);
-    store<U, ST>(piece<U>(a.out.p[r], (r + N - i) % N * chunk, off, chunk), lane, v);
+    store<U, ST>(dst, span_of<LINED, U>(a, (r + N - i) % N, lane), v);
   }
 }
 
@@ -311,15 +356,16 @@ __global__ __launch_bounds__(64 * N) void k_group_allgather(Args a) {
 template <int N, int U>
 using BisectSinks = Sinks<U, 2 * N, 4 * N>;
 
-template <int N, int DT, int U, int LD, int ST>
+template <int N, int DT, int U, bool LINED, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_bisect(Args a) {
   constexpr int B = N / 2;
   VR_GROUP_PROLOGUE;
   const BisectSinks<N, U> sk(lds, lane);
   const int y = (int)blockIdx.y, h = r & 1, l = r >> 1, pair = r ^ 1;
-  const size_t close = (size_t)(h * B + y) * chunk, far = (size_t)((1 - h) * B + y) * chunk;
-  const Msg<U> f = load<U, LD>(piece<U>(a.in.p[r], far, off, chunk), lane);
-  Msg<U> v = load<U, LD>(piece<U>(a.in.p[r], close, off, chunk), lane);
+  const auto close = span_of<LINED, U>(a, h * B + y, lane),
+             far = span_of<LINED, U>(a, (1 - h) * B + y, lane);
+  const Msg<U> f = load<U, LD>(src, far);
+  Msg<U> v = load<U, LD>(src, close);
   sk.ready();
   sk.put(pair, f);                                         // scatterFar
   sk.publish();
@@ -347,9 +393,9 @@ __global__ __launch_bounds__(64 * N) void k_group_bisect(Args a) {
   sk.put(r, v);                                            // forward to the pair
   sk.publish();
   sk.raise(3 * N + pair, 1);
-  store<U, ST>(piece<U>(a.out.p[r], close, off, chunk), lane, v);
+  store<U, ST>(dst, close, v);
   poll.until([&] { return sk.look(3 * N + r) != 0; });     // pollFarGatherOutput
-  store<U, ST>(piece<U>(a.out.p[r], far, off, chunk), lane, sk.get(pair));
+  store<U, ST>(dst, far, sk.get(pair));
 }
 
 #undef VR_GROUP_PROLOGUE
@@ -359,42 +405,45 @@ struct Pick {
   uint32_t rows, lds;   // rows of the grid, bytes of LDS the sinks take
 };
 
-template <int N, int DT, int LD, int ST, int U>
+template <int N, int DT, int LD, int ST, int U, bool LINED>
 Pick pick_flow(WireFlow flow) {
   if constexpr (N <= 8) {
     switch (flow) {
-      case WIRE_PARALLEL: return {reinterpret_cast<const void *>(&k_group_parallel<N, DT, U, LD, ST>), N, ParallelSinks<N, U>::kBytes};
+      case WIRE_PARALLEL: return {reinterpret_cast<const void *>(&k_group_parallel<N, DT, U, LINED, LD, ST>), N, ParallelSinks<N, U>::kBytes};
       case WIRE_SEQUENTIAL:
-      case WIRE_SIMPLE: return {reinterpret_cast<const void *>(&k_group_sequential<N, DT, U, LD, ST>), 1, SequentialSinks<N, U>::kBytes};
-      case WIRE_RING: return {reinterpret_cast<const void *>(&k_group_ring<N, DT, U, LD, ST>), 1, RingSinks<N, U>::kBytes};
+      case WIRE_SIMPLE: return {reinterpret_cast<const void *>(&k_group_sequential<N, DT, U, LINED, LD, ST>), 1, SequentialSinks<N, U>::kBytes};
+      case WIRE_RING: return {reinterpret_cast<const void *>(&k_group_ring<N, DT, U, LINED, LD, ST>), 1, RingSinks<N, U>::kBytes};
       case WIRE_ALLGATHER:   // no adds: one instantiation serves both element types
         if constexpr (U == 1)
-          return {reinterpret_cast<const void *>(&k_group_allgather<N, DT_F16, U, LD, ST>), 1, RingSinks<N, U>::kBytes};
+          return {reinterpret_cast<const void *>(&k_group_allgather<N, DT_F16, U, LINED, LD, ST>), 1, RingSinks<N, U>::kBytes};
         break;
       default: break;
     }
   }
   if constexpr (N >= 4) {
-    if (flow == WIRE_BISECT) return {reinterpret_cast<const void *>(&k_group_bisect<N, DT, U, LD, ST>), N / 2, BisectSinks<N, U>::kBytes};
+    if (flow == WIRE_BISECT) return {reinterpret_cast<const void *>(&k_group_bisect<N, DT, U, LINED, LD, ST>), N / 2, BisectSinks<N, U>::kBytes};
   }
   return {nullptr, 0, 0};
 }
 
-template <int DT, int LD, int ST>
+template <int DT, int LD, int ST, bool LINED>
 Pick pick_ranks(WireFlow flow, int nranks, int unroll) {
   switch (nranks) {
-    case 2: return pick_flow<2, DT, LD, ST, 1>(flow);
-    case 4: return pick_flow<4, DT, LD, ST, 1>(flow);
-    case 8: return unroll == 2 ? pick_flow<8, DT, LD, ST, 2>(flow) : pick_flow<8, DT, LD, ST, 1>(flow);
-    case 16: return unroll == 2 ? pick_flow<16, DT, LD, ST, 2>(flow) : pick_flow<16, DT, LD, ST, 1>(flow);
+    case 2: return pick_flow<2, DT, LD, ST, 1, LINED>(flow);
+    case 4: return pick_flow<4, DT, LD, ST, 1, LINED>(flow);
+    case 8: return unroll == 2 ? pick_flow<8, DT, LD, ST, 2, LINED>(flow) : pick_flow<8, DT, LD, ST, 1, LINED>(flow);
+    case 16: return unroll == 2 ? pick_flow<16, DT, LD, ST, 2, LINED>(flow) : pick_flow<16, DT, LD, ST, 1, LINED>(flow);
     default: return {nullptr, 0, 0};
   }
 }
 
 template <int LD, int ST>
-Pick pick_type(WireFlow flow, int nranks, DType dtype, int unroll) {
-  return dtype == DT_BF16 ? pick_ranks<DT_BF16, LD, ST>(flow, nranks, unroll)
-                          : pick_ranks<DT_F16, LD, ST>(flow, nranks, unroll);
+Pick pick_type(WireFlow flow, int nranks, DType dtype, int unroll, bool lined) {
+  if (lined)
+    return dtype == DT_BF16 ? pick_ranks<DT_BF16, LD, ST, true>(flow, nranks, unroll)
+                            : pick_ranks<DT_F16, LD, ST, true>(flow, nranks, unroll);
+  return dtype == DT_BF16 ? pick_ranks<DT_BF16, LD, ST, false>(flow, nranks, unroll)
+                          : pick_ranks<DT_F16, LD, ST, false>(flow, nranks, unroll);
 }
 
 }  // namespace
@@ -402,29 +451,38 @@ Pick pick_type(WireFlow flow, int nranks, DType dtype, int unroll) {
 hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow, int nranks, DType dtype,
                              const PtrTable &in, const PtrTable &out, size_t chunk_bytes, const GroupPlan &plan,
                              uint32_t spin_limit, uint32_t *status) {
-  if (chunk_bytes == 0) return hipSuccess;
-  const Pick k = plan.policy == GROUP_STREAM     ? pick_type<kStreamLoad, kStreamStore>(flow, nranks, dtype, plan.unroll)
-                 : plan.policy == GROUP_RESIDENT ? pick_type<0, 0>(flow, nranks, dtype, plan.unroll)
-                                                 : pick_type<0, kStreamStore>(flow, nranks, dtype, plan.unroll);
+  const bool lined = (((uintptr_t)out.p[0] | chunk_bytes) & 127u) == 0;
+  const Pick k =
+      plan.policy == GROUP_STREAM     ? pick_type<kStreamLoad, kStreamStore>(flow, nranks, dtype, plan.unroll, lined)
+      : plan.policy == GROUP_RESIDENT ? pick_type<0, 0>(flow, nranks, dtype, plan.unroll, lined)
+                                      : pick_type<0, kStreamStore>(flow, nranks, dtype, plan.unroll, lined);
   if (!k.fn) return hipErrorInvalidValue;
   const size_t wire = 1024u * (size_t)(nranks >= 8 ? plan.unroll : 1);   // payload of one wave
-  const size_t wires = (chunk_bytes + wire - 1) / wire;
-  if (wires > 0x7fffffffull) return hipErrorInvalidValue;
-  Args a;
-  a.in = in;
-  a.out = out;
-  a.chunk_bytes = chunk_bytes;
-  a.spin_limit = spin_limit;
-  a.status = status;
   uint32_t lds = k.lds;
   const uint32_t cap = lds_cap_bytes(dev, plan.wgs_per_cu);
   if (cap > lds) lds = cap;
   if (hipError_t e = allow_dynamic_lds(k.fn, dev, lds); e != hipSuccess) return e;
+  Args a;
+  a.in = in;
+  a.out = out;
+  a.pitch = chunk_bytes;
+  a.lines = lines_of(out, flow == WIRE_ALLGATHER ? 0u : head_mask_of(nranks, in, out));   // (whole 16-byte messages)
+  a.spin_limit = spin_limit;
+  a.status = status;
   void *kargs[] = {&a};
-  const dim3 grid((uint32_t)wires, k.rows), block(64u * (uint32_t)nranks);
-  if (tl_kernel_events.start || tl_kernel_events.stop)
-    return hipExtLaunchKernel(k.fn, grid, block, kargs, lds, s, tl_kernel_events.start, tl_kernel_events.stop, 0);
-  return hipLaunchKernel(k.fn, grid, block, kargs, lds, s);
+  const size_t seg_max = (size_t)1 << 30;   // 32-bit offsets
+  for (size_t off = 0; off < chunk_bytes; off += seg_max) {
+    const size_t seg = chunk_bytes - off < seg_max ? chunk_bytes - off : seg_max;
+    a.seg_off = off;
+    a.seg_bytes = (uint32_t)seg;
+    const dim3 grid((uint32_t)((seg + (lined ? 0 : 120) + wire - 1) / wire), k.rows), block(64u * (uint32_t)nranks);
+    hipEvent_t ev0 = off == 0 ? tl_kernel_events.start : nullptr;
+    hipEvent_t ev1 = off + seg >= chunk_bytes ? tl_kernel_events.stop : nullptr;
+    const hipError_t e = ev0 || ev1 ? hipExtLaunchKernel(k.fn, grid, block, kargs, lds, s, ev0, ev1, 0)
+                                    : hipLaunchKernel(k.fn, grid, block, kargs, lds, s);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace vr
