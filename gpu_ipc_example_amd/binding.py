@@ -1,6 +1,8 @@
-"""ctypes binding of libvrank_allreduce.so (the C ABI in include/vrank_allreduce.h).
+"""Binding of libvrank_allreduce.so (the C ABI in include/vrank_allreduce.h): ctypes, and for
+the collective calls, where the time a call takes is the host's, the CPython module _call
+(csrc/vr_pycall.c).
 
-No fallback exists: if the shared library is missing or a call fails, an
+No fallback exists: if a shared library is missing or a call fails, an
 exception is raised.  Device buffers are plain integers (device addresses), so
 callers may hand in ``torch.Tensor.data_ptr()`` values or use the library's own
 vr_malloc plumbing through :class:`DeviceBuffer`.
@@ -57,10 +59,11 @@ def build_library(force=False):
 
 
 _lib = None
+_call = None       # the collective calls (csrc/vr_pycall.c)
 
 
 def lib():
-    global _lib
+    global _lib, _call
     if _lib is not None:
         return _lib
     if not os.path.exists(_SO):
@@ -141,7 +144,8 @@ def lib():
         f = getattr(L, name)          # AttributeError here = header and library disagree
         f.restype, f.argtypes = res, args
     L._signatures = sig
-    _lib = L
+    from . import _call as call
+    _lib, _call = L, call
     return L
 
 
@@ -258,12 +262,14 @@ class VirtualRanks:
         h = C.c_void_p()
         _check(lib().vr_ctx_create(device, nranks, C.byref(h)))
         self._h, self.nranks, self.device = h, nranks, device
+        self._address = h.value          # of the context, 0 once closed
+        self._wire_reserved = False
         self.seq_no = C.c_uint32(1)
 
     def close(self):
         if self._h:
             lib().vr_ctx_destroy(self._h)
-            self._h = None
+            self._h, self._address = None, 0
 
     def __del__(self):
         try:
@@ -276,7 +282,9 @@ class VirtualRanks:
 
     def reserve_wire(self):
         """Allocate and zero the wire transport's scratch (idempotent)."""
-        _check(lib().vr_ctx_reserve_wire(self._h))
+        if not self._wire_reserved:
+            _check(lib().vr_ctx_reserve_wire(self._h))
+            self._wire_reserved = True
 
     def _reserve_for(self, algo, transport):
         # The C ABI never allocates inside a collective call; this wrapper reserves
@@ -349,8 +357,9 @@ class VirtualRanks:
 
     def allreduce_static(self, algo, bufs, nelems, outs=None, stream=None):
         """Wire-transport all-reduce through the library's fixed scratch region (no allocation)."""
-        _check(lib().vr_allreduce_static(self._h, stream, algo_id(algo), _table(bufs),
-                                         _table(outs) if outs is not None else None, nelems))
+        rc = _call.allreduce_static(self._address, algo, bufs, outs, nelems, stream)
+        if rc:
+            _check(rc)
 
     def set_tuning(self, **kw):
         for k, v in kw.items():
@@ -366,10 +375,11 @@ class VirtualRanks:
 
     def allreduce(self, algo, bufs, nelems, outs=None, transport=TRANSPORT_DEFAULT, stream=None):
         assert len(bufs) == self.nranks
-        self._reserve_for(algo, transport)
-        _check(lib().vr_allreduce(self._h, stream, algo_id(algo), transport, _table(bufs),
-                                  _table(outs) if outs is not None else None, nelems,
-                                  C.byref(self.seq_no)))
+        if transport != TRANSPORT_DIRECT and not self._wire_reserved:
+            self._reserve_for(algo, transport)
+        rc = _call.allreduce(self._address, self.seq_no, algo, transport, bufs, outs, nelems, stream)
+        if rc:
+            _check(rc)
 
     def allreduce_grid(self, algo, bufs, nelems, groups, subgroups, simd=16, outs=None,
                        transport=TRANSPORT_DEFAULT, stream=None, seq_no=0xE00F100F):
@@ -379,9 +389,11 @@ class VirtualRanks:
                                        groups, subgroups, simd))
 
     def allgather(self, algo, inputs, outputs, nelems, transport=TRANSPORT_DEFAULT, stream=None):
-        self._reserve_for(algo, transport)
-        _check(lib().vr_allgather(self._h, stream, algo_id(algo), transport, _table(inputs),
-                                  _table(outputs), nelems, C.byref(self.seq_no)))
+        if transport == TRANSPORT_WIRE:
+            self.reserve_wire()
+        rc = _call.allgather(self._address, self.seq_no, algo, transport, inputs, outputs, nelems, stream)
+        if rc:
+            _check(rc)
 
     def allgather_grid(self, algo, inputs, outputs, nelems, groups, subgroups, simd=16,
                        transport=TRANSPORT_DEFAULT, stream=None, seq_no=0xE00F100F):

@@ -1,0 +1,137 @@
+/* The three collective calls for Python: pointer lists into stack tables, one C ABI call.
+ *
+ * A collective call at launch-bound sizes costs what the host spends on it.  Through
+ * ctypes that was 5.5 us a call, over half of it spent on turning lists into c_void_p
+ * arrays and arguments into C types; the call itself is one kernel launch (2.3 us).
+ * Everything else of the C ABI stays with ctypes (binding.py), which also holds the
+ * argument checks, the context and the error texts: these functions return the status. */
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <stdint.h>
+
+#include "vrank_allreduce.h"
+
+/* Device addresses of a sequence; unused entries stay null.  -1 with an exception set. */
+static int fill_table(PyObject *seq, void *table[VR_MAX_RANKS]) {
+  for (int i = 0; i < VR_MAX_RANKS; ++i) table[i] = NULL;
+  PyObject *fast = PySequence_Fast(seq, "device addresses must be a sequence");
+  if (!fast) return -1;
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(fast);
+  if (n > VR_MAX_RANKS) {
+    Py_DECREF(fast);
+    PyErr_Format(PyExc_ValueError, "at most %d device addresses, got %zd", VR_MAX_RANKS, n);
+    return -1;
+  }
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject *item = PySequence_Fast_GET_ITEM(fast, i), *number = NULL;
+    if (!PyLong_Check(item)) {
+      number = PyNumber_Long(item);
+      if (!number) {
+        Py_DECREF(fast);
+        return -1;
+      }
+      item = number;
+    }
+    table[i] = (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(item);
+    Py_XDECREF(number);
+  }
+  Py_DECREF(fast);
+  return PyErr_Occurred() ? -1 : 0;
+}
+
+/* A hipStream_t: None (the null stream), an address, or a ctypes c_void_p.  -1 with an exception set. */
+static int stream_of(PyObject *o, void **stream) {
+  *stream = NULL;
+  if (o == Py_None) return 0;
+  PyObject *value = NULL;
+  if (!PyLong_Check(o)) {
+    value = PyObject_GetAttrString(o, "value");
+    if (!value) return -1;
+    o = value;
+  }
+  if (o != Py_None) *stream = (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(o);
+  Py_XDECREF(value);
+  return PyErr_Occurred() ? -1 : 0;
+}
+
+/* The status of looking the name up; -1 with an exception set. */
+static int algo_of(PyObject *name, int *algo) {
+  const char *text = PyUnicode_AsUTF8(name);
+  return text ? vr_algo_from_string(text, algo) : -1;
+}
+
+/* (context, sequence number, algo name, transport, inputs, outputs or None, nelems, stream) -> status.
+ * The context is an address, the sequence number a writable buffer of 4 bytes (a ctypes c_uint32). */
+static PyObject *collective(PyObject *const *args, Py_ssize_t nargs, int gather) {
+  if (nargs != 8) {
+    PyErr_SetString(PyExc_TypeError, "8 arguments expected");
+    return NULL;
+  }
+  void *ins[VR_MAX_RANKS], *outs[VR_MAX_RANKS], *stream;
+  int algo = -1, rc = algo_of(args[2], &algo);
+  if (rc) return rc < 0 ? NULL : PyLong_FromLong(rc);
+  vr_ctx *ctx = (vr_ctx *)(uintptr_t)PyLong_AsUnsignedLongLongMask(args[0]);
+  const long transport = PyLong_AsLong(args[3]);
+  const size_t nelems = (size_t)PyLong_AsUnsignedLongLongMask(args[6]);
+  if (PyErr_Occurred() || stream_of(args[7], &stream)) return NULL;
+  const int in_place = args[5] == Py_None;
+  if (fill_table(args[4], ins) || (!in_place && fill_table(args[5], outs))) return NULL;
+  Py_buffer seq;
+  if (PyObject_GetBuffer(args[1], &seq, PyBUF_WRITABLE)) return NULL;
+  if (seq.len != (Py_ssize_t)sizeof(uint32_t)) {
+    PyBuffer_Release(&seq);
+    PyErr_SetString(PyExc_ValueError, "the sequence number has 4 bytes");
+    return NULL;
+  }
+  Py_BEGIN_ALLOW_THREADS
+  if (gather)
+    rc = vr_allgather(ctx, stream, algo, (int)transport, (const void *const *)ins, in_place ? NULL : outs, nelems,
+                      (uint32_t *)seq.buf);
+  else
+    rc = vr_allreduce(ctx, stream, algo, (int)transport, ins, in_place ? NULL : outs, nelems, (uint32_t *)seq.buf);
+  Py_END_ALLOW_THREADS
+  PyBuffer_Release(&seq);
+  return PyLong_FromLong(rc);
+}
+
+static PyObject *allreduce(PyObject *self, PyObject *const *args, Py_ssize_t nargs) {
+  (void)self;
+  return collective(args, nargs, 0);
+}
+
+static PyObject *allgather(PyObject *self, PyObject *const *args, Py_ssize_t nargs) {
+  (void)self;
+  return collective(args, nargs, 1);
+}
+
+/* (context, algo name, inputs, outputs or None, nelems, stream) -> status */
+static PyObject *allreduce_static(PyObject *self, PyObject *const *args, Py_ssize_t nargs) {
+  (void)self;
+  if (nargs != 6) {
+    PyErr_SetString(PyExc_TypeError, "6 arguments expected");
+    return NULL;
+  }
+  void *ins[VR_MAX_RANKS], *outs[VR_MAX_RANKS], *stream;
+  int algo = -1, rc = algo_of(args[1], &algo);
+  if (rc) return rc < 0 ? NULL : PyLong_FromLong(rc);
+  vr_ctx *ctx = (vr_ctx *)(uintptr_t)PyLong_AsUnsignedLongLongMask(args[0]);
+  const size_t nelems = (size_t)PyLong_AsUnsignedLongLongMask(args[4]);
+  if (PyErr_Occurred() || stream_of(args[5], &stream)) return NULL;
+  const int in_place = args[3] == Py_None;
+  if (fill_table(args[2], ins) || (!in_place && fill_table(args[3], outs))) return NULL;
+  Py_BEGIN_ALLOW_THREADS
+  rc = vr_allreduce_static(ctx, stream, algo, ins, in_place ? NULL : outs, nelems);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong(rc);
+}
+
+static PyMethodDef methods[] = {
+    {"allreduce", (PyCFunction)(void (*)(void))allreduce, METH_FASTCALL, "vr_allreduce"},
+    {"allgather", (PyCFunction)(void (*)(void))allgather, METH_FASTCALL, "vr_allgather"},
+    {"allreduce_static", (PyCFunction)(void (*)(void))allreduce_static, METH_FASTCALL, "vr_allreduce_static"},
+    {NULL, NULL, 0, NULL}};
+
+static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "_call", "Collective calls of the C ABI.", -1, methods,
+                                    NULL, NULL, NULL, NULL};
+
+PyMODINIT_FUNC PyInit__call(void) { return PyModule_Create(&module); }
