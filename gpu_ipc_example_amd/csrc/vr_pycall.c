@@ -16,12 +16,8 @@ static int fill_table(PyObject *seq, void *table[VR_MAX_RANKS]) {
   for (int i = 0; i < VR_MAX_RANKS; ++i) table[i] = NULL;
   PyObject *fast = PySequence_Fast(seq, "device addresses must be a sequence");
   if (!fast) return -1;
-  const Py_ssize_t n = PySequence_Fast_GET_SIZE(fast);
-  if (n > VR_MAX_RANKS) {
-    Py_DECREF(fast);
-    PyErr_Format(PyExc_ValueError, "at most %d device addresses, got %zd", VR_MAX_RANKS, n);
-    return -1;
-  }
+  Py_ssize_t n = PySequence_Fast_GET_SIZE(fast);
+  if (n > VR_MAX_RANKS) n = VR_MAX_RANKS;   /* no context looks further */
   for (Py_ssize_t i = 0; i < n; ++i) {
     PyObject *item = PySequence_Fast_GET_ITEM(fast, i), *number = NULL;
     if (!PyLong_Check(item)) {
@@ -39,17 +35,28 @@ static int fill_table(PyObject *seq, void *table[VR_MAX_RANKS]) {
   return PyErr_Occurred() ? -1 : 0;
 }
 
-/* A hipStream_t: None (the null stream), an address, or a ctypes c_void_p.  -1 with an exception set. */
+/* A hipStream_t as ctypes takes a c_void_p argument: None (the null stream), an address, a
+ * ctypes c_void_p, or an object that has one as its _as_parameter_ (torch's streams do).
+ * -1 with an exception set. */
 static int stream_of(PyObject *o, void **stream) {
   *stream = NULL;
   if (o == Py_None) return 0;
-  PyObject *value = NULL;
+  PyObject *inner = NULL, *value = NULL;
   if (!PyLong_Check(o)) {
+    inner = PyObject_GetAttrString(o, "_as_parameter_");
+    if (inner)
+      o = inner;
+    else if (!PyErr_ExceptionMatches(PyExc_AttributeError))
+      return -1;
+    else
+      PyErr_Clear();
+  }
+  if (o != Py_None && !PyLong_Check(o)) {
     value = PyObject_GetAttrString(o, "value");
-    if (!value) return -1;
     o = value;
   }
-  if (o != Py_None) *stream = (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(o);
+  if (o && o != Py_None) *stream = (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(o);
+  Py_XDECREF(inner);
   Py_XDECREF(value);
   return PyErr_Occurred() ? -1 : 0;
 }

@@ -1,0 +1,38 @@
+"""What the collective calls from Python take for a stream and for a table of device addresses:
+all that ctypes converts to a c_void_p.  Null contexts, so that nothing reaches a device."""
+import ctypes as C
+
+import pytest
+
+import gpu_ipc_example_amd as vr
+from gpu_ipc_example_amd import binding
+
+
+def call(stream, ptrs=(8, 16)):
+    vr.lib()
+    return binding._call.allreduce(0, C.c_uint32(1), "simple", vr.TRANSPORT_DIRECT, ptrs, None, 16, stream)
+
+
+class Holder:
+    def __init__(self, p):
+        self._as_parameter_ = p
+
+
+def test_streams_that_ctypes_takes():
+    want = call(None)
+    assert want != 0        # no context
+    for stream in (0, 64, C.c_void_p(), C.c_void_p(64), Holder(C.c_void_p(64)), Holder(C.c_void_p()), Holder(64),
+                   Holder(None)):
+        assert call(stream) == want
+    for stream in ("x", 1.5, object(), [], Holder("x")):
+        with pytest.raises((TypeError, AttributeError)):
+            call(stream)
+
+
+def test_tables():
+    want = call(None)
+    for ptrs in ((8, 16), [8, 16], (8, 16.0), [8] * 17, []):
+        assert call(None, ptrs) == want
+    for ptrs in ([None, 8], 5, [[]]):
+        with pytest.raises(TypeError):
+            call(None, ptrs)
