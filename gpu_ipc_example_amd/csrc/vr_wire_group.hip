@@ -17,7 +17,7 @@
 // 8 TB/s however much of it the memory-side cache serves; here only inputs and
 // outputs cross it.  ParallelTransmit, 8 ranks in place: 256 MiB per rank
 // 2196 -> 688 us (6.2 TB/s), 1 MiB per rank 14.4 -> 5.6 us (the host's pace);
-// RingTransmit, 4 x 8 MB: 39.3 -> 11.4 us; ring all-gather, 8 x 1 MB: 51 -> 13 us.
+// RingTransmit, 4 x 8 MB: 39.3 -> 11.1 us; ring all-gather, 8 x 1 MB: 51 -> 12.2 us.
 //
 // One wire per work-group and no loop: the hardware starts work-groups in index
 // order, so a launch sweeps the chunks front to back with all compute units close
@@ -277,29 +277,42 @@ __global__ __launch_bounds__(64 * N) void k_group_sequential(Args a) {
 }
 
 // ---- RingTransmit (sequential_transmit.hpp:429-516) --------------------------------------
-// A rank's sink is a ring of kRingDepth slots fed by its predecessor.  Flag r counts
-// the messages delivered to rank r, flag N + r those it has taken out, which is what
-// its predecessor looks at before it reuses a slot.
-constexpr int kRingDepth = 2;
+// A rank's sink is a ring of slots fed by its predecessor; flag r counts the messages
+// delivered to rank r.  With N slots nothing more is needed: message k + N comes into the
+// slot of message k, and it is sent after message k + N - 1 was received, which was sent
+// after ..., N - 1 ranks back, message k + 1 of the slot's own rank, and that one is made of
+// (or sent after) message k, read from the slot.  Where N slots of U KiB a rank would take
+// the room of too many work-groups, two slots, and flag N + r counts the messages rank r has
+// taken out, which its predecessor looks at before it reuses one.  A hop is a chain of LDS
+// round trips, and the count and the look at it were two of five: with two slots
+// throughout, 8 x 256 KiB 7.3 us, now 5.9, 8 x 2 MiB 11.6, now 9.8, 4 x 2 MiB 5.2, now 4.6 (14
+// and 6 hops); all-gather 8 x 1 MiB 13.1, now 11.9, 8 x 2 MiB 25.1, now 22.9 (there the 64 KiB of
+// slots also hold a compute unit at two work-groups, which suits its 8 write streams).
 template <int N, int U>
-using RingSinks = Sinks<U, N * kRingDepth, 2 * N>;
+struct RingSinks : Sinks<U, N * (N * U <= 8 ? N : 2), 2 * N> {
+  static constexpr int kDepth = N * U <= 8 ? N : 2;
+  using Sinks<U, N * kDepth, 2 * N>::Sinks;
+};
 
 template <int N, int U>
 struct Ring {
+  static constexpr int kDepth = RingSinks<N, U>::kDepth;
   const RingSinks<N, U> &sk;
   Poll &poll;
   int r, next;
   __device__ __forceinline__ void send(int k, const Msg<U> &m) const {
-    if (k >= kRingDepth) poll.until([&] { return sk.look(N + next) >= (uint32_t)(k - kRingDepth + 1); });
-    sk.put(next * kRingDepth + k % kRingDepth, m);
+    if (kDepth < N && k >= kDepth) poll.until([&] { return sk.look(N + next) >= (uint32_t)(k - kDepth + 1); });
+    sk.put(next * kDepth + k % kDepth, m);
     sk.publish();
     sk.raise(next, (uint32_t)(k + 1));
   }
   __device__ __forceinline__ Msg<U> recv(int k) const {
     poll.until([&] { return sk.look(r) >= (uint32_t)(k + 1); });
-    const Msg<U> m = sk.get(r * kRingDepth + k % kRingDepth);
-    sk.publish();
-    sk.raise(N + r, (uint32_t)(k + 1));
+    const Msg<U> m = sk.get(r * kDepth + k % kDepth);
+    if constexpr (kDepth < N) {
+      sk.publish();
+      sk.raise(N + r, (uint32_t)(k + 1));
+    }
     return m;
   }
 };
