@@ -107,15 +107,20 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
   const size_t MiB = (size_t)1 << 20;
   GroupPlan p = {GROUP_MIXED, 1, 0};
   // Cache policies, us per pass on one / three / ten sets of buffers in turn:
-  //  * in place up to 64 MiB everything stays cacheable (8 x 4 MiB 9.1 / 12.9 / 16.0, streamed
-  //    13.9 / 15.9 / 15.9; 4 x 16 MiB 22.2 / 21.9 / 26.8 against 25.1 / 24.8 / 24.5), beyond it
-  //    streaming wins as soon as the buffers do not all fit the memory-side cache
-  //    (8 x 16 MiB 39.5 / 50.5 / 53.2 against 49.9 / 48.9 / 49.4);
-  //  * out of place, and all-gather, up to half the memory-side cache of inputs: results
-  //    are streamed past inputs that may stay (8 x 16 MiB 41.3 / 49.3 / 50.5, everything
-  //    streamed 50.2 / 50.2 / 49.4), beyond it everything streams (8 x 128 MiB 355, 351 us).
-  if (in_place) p.policy = reads <= 64 * MiB ? GROUP_RESIDENT : GROUP_STREAM;
-  else if (reads > 128 * MiB) p.policy = GROUP_STREAM;
+  //  * in place up to 72 MiB, of which three sets fit the memory-side cache, everything stays
+  //    cacheable (8 x 4 MiB 9.1 / 12.9 / 16.0, streamed 13.9 / 15.9 / 15.9; 9 MiB per rank on 8, one
+  //    and three sets: parallel 23.4 / 23.8, streamed 27.6 / 27.9, ring 8 x 8 MiB + 16 B
+  //    20.7 / 20.5, streamed 27.2 / 27.3), beyond it streaming wins as soon as the buffers do
+  //    not all fit (8 x 10 MiB: simple 26.3 / 33.5, streamed 30.4 / 30.5; 8 x 16 MiB
+  //    39.5 / 50.5 / 53.2, streamed 49.9 / 48.9 / 49.4);
+  //  * out of place up to half the memory-side cache of inputs: results are streamed past
+  //    inputs that may stay (8 x 16 MiB 41.3 / 49.3 / 50.5, everything streamed
+  //    50.2 / 50.2 / 49.4), beyond it everything streams (8 x 128 MiB 355, 351 us);
+  //  * all-gather: results are streamed past the inputs at every size, they are N times as
+  //    long (2 x 64 MiB 58.2 / 65.9, everything streamed 68.0 / 66.9; 8 x 16 MiB 193 / 222, streamed
+  //    238 / 230).
+  if (in_place) p.policy = reads <= 72 * MiB ? GROUP_RESIDENT : GROUP_STREAM;
+  else if (reads > 128 * MiB && flow != WIRE_ALLGATHER) p.policy = GROUP_STREAM;
   // Two vectors per lane at 8 and 16 ranks, where that is the faster (fewer waves for the
   // same bytes where the caches feed them quicker than waves start; at 2 and 4 ranks one vector
   // is 10 to 40 % faster at every size):
@@ -130,7 +135,11 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
     case WIRE_BISECT:
       // 8 x 4 MiB 15.2 -> 11.8 us, 8 x 2 and 8 x 8 MiB even; 16 x 4 MiB 29.8 -> 22.0 us,
       // 16 x 8 MiB 53.8, two: 57.4
+      // Four ranks, streaming, from 192 MiB on: five work-groups per CU (40 KiB of loads in
+      // flight, uncapped 64).  4 x 64 MiB 91.7 -> 84.1 us, 4 x 128 MiB 165.5 -> 163.2.  (Eight
+      // ranks with three: from 5 % faster to 11 % slower.)
       p.unroll = nranks == 8 ? (reads >= 16 * MiB && reads < 64 * MiB ? 2 : 1) : nranks == 16 && reads <= 96 * MiB ? 2 : 1;
+      if (nranks == 4 && reads >= 192 * MiB) p.wgs_per_cu = 5;
       break;
     case WIRE_RING:
     case WIRE_SEQUENTIAL:
@@ -138,8 +147,15 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
       // ring 8 x 16 MiB 65.1 -> 48.9 us, sequential 65.6 -> 46.8; 8 x 4 MiB even, 8 x 2 MiB
       // 8.4, two: 9.9; 8 x 32 MiB 97.7, two: 108.8
       if (nranks == 8 && reads >= 32 * MiB && reads <= 192 * MiB) p.unroll = 2;
+      // Ring, four ranks, streaming: 48 KiB of loads per CU in flight instead of 128.
+      // 4 x 64 MiB 106 -> 94 us, 4 x 128 MiB 190.5 -> 169.5; 4 x 32 MiB 50.7, capped 50.9
+      if (flow == WIRE_RING && nranks == 4 && reads >= 192 * MiB) p.wgs_per_cu = 3;
       break;
-    default: break;   // all-gather 8 x 4 MiB: 49.0, two: 59.1 us
+    case WIRE_ALLGATHER:   // one vector: 8 x 4 MiB 49.0, two: 59.1 us
+      // Four ranks with four work-groups per CU: 4 x 4 MiB 14.5 -> 13.6 us, 4 x 16 MiB 52.9 -> 48.6,
+      // 4 x 32 MiB 121.6 -> 109.2; 4 x 2 MiB 6.7, capped 6.5
+      if (nranks == 4 && reads >= 8 * MiB) p.wgs_per_cu = 4;
+      break;
   }
   return p;
 }

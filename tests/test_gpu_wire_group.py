@@ -75,3 +75,26 @@ def test_allgather_edges(oracle, nranks):
             for r, got in enumerate(run_allgather_wire(ctx, "allgather_simple", ins, alias)):
                 assert (got == want).all(), (n, r, alias)
     ctx.close()
+
+
+@pytest.mark.parametrize("nranks,algo,mib,inplace", [(4, "simple_ring", 194, True), (4, "bisect", 194, False),
+                                                     (8, "simple", 71, True)])
+def test_capped_and_resident_launches(oracle, nranks, algo, mib, inplace):
+    """Just inside the sizes (bytes of all ranks' inputs) that cap the work-groups per compute unit,
+    and the largest that stay cacheable in place, with a chunk that ends inside a wire."""
+    ctx = vr.VirtualRanks(nranks)
+    msg = 16 if algo == "simple_ring" else 8
+    chunk = (mib << 20) // nranks ** 2 // 16 * 16 + 3 * msg
+    run(oracle, ctx, algo, nranks * chunk // 2, F16, inplace, 0, 70_000)
+    ctx.close()
+
+
+def test_allgather_beyond_half_the_cache(oracle):
+    """Four ranks with 4 x 33 MiB of inputs and a ragged slice: capped, results streamed past cached inputs."""
+    ctx = vr.VirtualRanks(4)
+    n = (33 << 19) + 24
+    ins = [oracle.generate_dt(F16, n, 71_000 + r, DIST_NORMAL, 0.0, 1.0) for r in range(4)]
+    want = oracle.allgather(ins)
+    for r, got in enumerate(run_allgather_wire(ctx, "allgather_simple", ins, False)):
+        assert (got == want).all(), r
+    ctx.close()
