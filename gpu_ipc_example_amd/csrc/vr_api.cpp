@@ -414,10 +414,13 @@ static Tuning default_tuning(int nranks, const AlgoInfo *a, size_t read_bytes, s
         t.run = run;
       }
     }
-  } else if (a->latency_tuned && (in_place ? read_bytes : read_bytes + write_bytes) < kMall) {
-    // "small" family at the sizes it is meant for: every lane makes one trip;
-    // results stay cacheable for the kernel that consumes them next.  (Beyond the
-    // cache it streams like the other protocols.)
+  } else if (a->latency_tuned && read_bytes <= ((size_t)(in_place ? 12 : 8) << 20)) {
+    // "small" family at the sizes it is meant for: every lane makes one trip; results stay
+    // cacheable for the kernel that consumes them next.  Up to 8 MiB of inputs (in place 12: 8 ranks,
+    // 9 MiB 4.5 us, the other launch 4.7), where both are bound by their start; beyond, the other protocols' launch is the faster
+    // (out of place, 8 ranks, one / three sets of buffers: 16 MiB 5.9 / 7.3 -> 4.4 / 6.4 us,
+    // 32 MiB 11.6 / 11.7 -> 8.1 / 11.0, 64 MiB 21.1 / 28.7 -> 20.4 / 20.2, 96 MiB 30.2 / 43.3 ->
+    // 29.6 / 34.9; in place 32 MiB 8.8 / 12.2 -> 8.0 / 11.3, 96 MiB even).
     t.waves_per_cu = 8;
     t.oneshot = 1;
     t.nt_load = 0;

@@ -31,7 +31,7 @@ struct AlgoInfo {
   int wire_capacity;   // payload bytes per wire at sub-group size 16
   bool allgather;
   Order order;
-  bool latency_tuned;  // "small" family: one-shot grid, cached accesses
+  bool latency_tuned;  // "small" family: one-shot grid, cached accesses (up to 8 or 12 MiB of inputs)
   WireFlow wire_flow() const {
     if (allgather) return WIRE_ALLGATHER;
     switch (transmit) {

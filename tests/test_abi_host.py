@@ -129,6 +129,18 @@ def test_no_device_is_a_clean_error():
     assert e.value.code == "NO_DEVICE"
 
 
+def test_latency_family_launches_like_the_others_beyond_its_sizes():
+    MiB = 1 << 20
+    for nranks in (2, 4, 8):
+        for in_place in (False, True):
+            n = (12 if in_place else 8) * MiB // 2 // nranks // (4 * nranks) * (4 * nranks)
+            p = vr.direct_launch_plan("small", nranks, n, in_place)
+            assert (p["one_trip"], p["block"], p["nt_store"]) == (1, 256, 0)
+            for more in (n + 4 * nranks, 4 * n):
+                assert vr.direct_launch_plan("small", nranks, more, in_place) == vr.direct_launch_plan(
+                    "simple", nranks, more, in_place)
+
+
 def test_launch_plans_of_the_direct_transport():
     """The launches the library picks by itself, as its documentation states them (pure host
     arithmetic behind vr_direct_launch_plan)."""
@@ -165,7 +177,7 @@ def test_launch_plans_of_the_direct_transport():
     assert plan("simple", 8, 2 * MiB, False)["nt_store"] == 2 and plan("simple", 8, 1 * MiB, False)["nt_store"] == 1
     p = plan("bisect", 8, 8 * MiB, False)
     assert (p["one_trip"], p["nt_load"], p["nt_store"]) == (0, 0, 2)
-    # the latency family: one trip per lane, everything cacheable, up to the size of the cache
+    # the latency family: one trip per lane, everything cacheable
     p = plan("small", 8, MiB // 2, True)
     assert (p["one_trip"], p["block"], p["wgs_per_cu"], p["nt_load"], p["nt_store"]) == (1, 256, 0, 0, 0)
     assert plan("small", 8, 16 * MiB, True)["nt_load"] == 1
