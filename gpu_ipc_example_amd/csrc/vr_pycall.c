@@ -11,27 +11,30 @@
 
 #include "vrank_allreduce.h"
 
-/* Device addresses of a sequence; unused entries stay null.  -1 with an exception set. */
+/* Device addresses of a sequence; unused entries stay null.  -1 with an exception set.
+ * Turning anything but an int into an address runs the caller's code, which may change the
+ * caller's sequence: those are read from a tuple that is nobody else's. */
 static int fill_table(PyObject *seq, void *table[VR_MAX_RANKS]) {
   for (int i = 0; i < VR_MAX_RANKS; ++i) table[i] = NULL;
-  PyObject *fast = PySequence_Fast(seq, "device addresses must be a sequence");
-  if (!fast) return -1;
-  Py_ssize_t n = PySequence_Fast_GET_SIZE(fast);
-  if (n > VR_MAX_RANKS) n = VR_MAX_RANKS;   /* no context looks further */
-  for (Py_ssize_t i = 0; i < n; ++i) {
-    PyObject *item = PySequence_Fast_GET_ITEM(fast, i), *number = NULL;
-    if (!PyLong_Check(item)) {
-      number = PyNumber_Long(item);
-      if (!number) {
-        Py_DECREF(fast);
-        return -1;
-      }
-      item = number;
-    }
-    table[i] = (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(item);
-    Py_XDECREF(number);
+  if (PyList_CheckExact(seq) || PyTuple_CheckExact(seq)) {
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+    PyObject *const *items = PySequence_Fast_ITEMS(seq);
+    Py_ssize_t i = 0;
+    for (; i < n && PyLong_CheckExact(items[i]); ++i)
+      if (i < VR_MAX_RANKS)   /* no context looks further */
+        table[i] = (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(items[i]);
+    if (i == n) return 0;
   }
-  Py_DECREF(fast);
+  PyObject *own = PySequence_Tuple(seq);
+  if (!own) return -1;
+  const Py_ssize_t n = PyTuple_GET_SIZE(own);
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject *number = PyNumber_Long(PyTuple_GET_ITEM(own, i));
+    if (!number) break;
+    if (i < VR_MAX_RANKS) table[i] = (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(number);
+    Py_DECREF(number);
+  }
+  Py_DECREF(own);
   return PyErr_Occurred() ? -1 : 0;
 }
 

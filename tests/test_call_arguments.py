@@ -36,3 +36,30 @@ def test_tables():
     for ptrs in ([None, 8], 5, [[]]):
         with pytest.raises(TypeError):
             call(None, ptrs)
+
+
+class Shrinks:
+    """An address whose conversion empties the list it came from."""
+
+    def __init__(self, table):
+        self.table = table
+
+    def __int__(self):
+        self.table.clear()
+        return 8
+
+
+def test_tables_that_change_while_they_are_read():
+    """In a process of its own: a table read beyond its end would end that process."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = ("from tests.test_call_arguments import Shrinks, call\n"
+            "for n in (1, 2, 16):\n"
+            "    table = []\n"
+            "    table.extend([Shrinks(table)] + [8] * (n - 1))\n"
+            "    assert call(None, table) == call(None)\n"
+            "print('read whole')\n")
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "read whole" in r.stdout, (r.returncode, r.stderr)
