@@ -38,30 +38,52 @@ static int fill_table(PyObject *seq, void *table[VR_MAX_RANKS]) {
   return PyErr_Occurred() ? -1 : 0;
 }
 
-/* A hipStream_t as ctypes takes a c_void_p argument: None (the null stream), an address, a
- * ctypes c_void_p, or an object that has one as its _as_parameter_ (torch's streams do).
- * -1 with an exception set. */
+/* Of the module ctypes: what converts an argument that is not a plain int. */
+static PyObject *ct_cast, *ct_void_p, *ct_size_t, *ct_int, *ct_error;
+
+/* A hipStream_t as ctypes takes a c_void_p argument.  None (the null stream), an int and a
+ * c_void_p are read here; ctypes converts the rest (objects with an _as_parameter_, pointers,
+ * ...) or refuses it.  -1 with an exception set. */
 static int stream_of(PyObject *o, void **stream) {
   *stream = NULL;
   if (o == Py_None) return 0;
-  PyObject *inner = NULL, *value = NULL;
-  if (!PyLong_Check(o)) {
-    inner = PyObject_GetAttrString(o, "_as_parameter_");
-    if (inner)
-      o = inner;
-    else if (!PyErr_ExceptionMatches(PyExc_AttributeError))
-      return -1;
-    else
-      PyErr_Clear();
-  }
-  if (o != Py_None && !PyLong_Check(o)) {
-    value = PyObject_GetAttrString(o, "value");
-    o = value;
+  PyObject *pointer = NULL, *value = NULL;
+  if (!PyLong_CheckExact(o)) {
+    if (Py_TYPE(o) != (PyTypeObject *)ct_void_p) {
+      pointer = PyObject_CallFunctionObjArgs(ct_cast, o, ct_void_p, NULL);
+      if (!pointer) return -1;
+      o = pointer;
+    }
+    o = value = PyObject_GetAttrString(o, "value");
   }
   if (o && o != Py_None) *stream = (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(o);
-  Py_XDECREF(inner);
   Py_XDECREF(value);
+  Py_XDECREF(pointer);
   return PyErr_Occurred() ? -1 : 0;
+}
+
+/* A number as ctypes takes an argument of the integer type `type`: an int (or what has an
+ * __index__), a `type`, or an object that has one of these as its _as_parameter_.  -1 with an
+ * exception set. */
+static int number_of(PyObject *o, PyObject *type, unsigned long long *number) {
+  if (PyLong_Check(o) || PyIndex_Check(o)) {
+    *number = PyLong_AsUnsignedLongLongMask(o);
+    return PyErr_Occurred() ? -1 : 0;
+  }
+  const int holds = PyObject_IsInstance(o, type);
+  PyObject *inner = holds < 0 ? NULL : PyObject_GetAttrString(o, holds ? "value" : "_as_parameter_");
+  if (!inner) {
+    if (holds == 0 && PyErr_ExceptionMatches(PyExc_AttributeError))
+      PyErr_Format(ct_error, "a number cannot be made of a %s", Py_TYPE(o)->tp_name);
+    return -1;
+  }
+  int rc = Py_EnterRecursiveCall(" while converting an argument") ? -1 : 0;
+  if (!rc) {
+    rc = number_of(inner, type, number);
+    Py_LeaveRecursiveCall();
+  }
+  Py_DECREF(inner);
+  return rc;
 }
 
 /* The status of looking the name up; -1 with an exception set. */
@@ -81,9 +103,10 @@ static PyObject *collective(PyObject *const *args, Py_ssize_t nargs, int gather)
   int algo = -1, rc = algo_of(args[2], &algo);
   if (rc) return rc < 0 ? NULL : PyLong_FromLong(rc);
   vr_ctx *ctx = (vr_ctx *)(uintptr_t)PyLong_AsUnsignedLongLongMask(args[0]);
-  const long transport = PyLong_AsLong(args[3]);
-  const size_t nelems = (size_t)PyLong_AsUnsignedLongLongMask(args[6]);
-  if (PyErr_Occurred() || stream_of(args[7], &stream)) return NULL;
+  unsigned long long transport, nelems;
+  if (PyErr_Occurred() || number_of(args[3], ct_int, &transport) || number_of(args[6], ct_size_t, &nelems) ||
+      stream_of(args[7], &stream))
+    return NULL;
   const int in_place = args[5] == Py_None;
   if (fill_table(args[4], ins) || (!in_place && fill_table(args[5], outs))) return NULL;
   Py_buffer seq;
@@ -95,10 +118,11 @@ static PyObject *collective(PyObject *const *args, Py_ssize_t nargs, int gather)
   }
   Py_BEGIN_ALLOW_THREADS
   if (gather)
-    rc = vr_allgather(ctx, stream, algo, (int)transport, (const void *const *)ins, in_place ? NULL : outs, nelems,
+    rc = vr_allgather(ctx, stream, algo, (int)transport, (const void *const *)ins, in_place ? NULL : outs, (size_t)nelems,
                       (uint32_t *)seq.buf);
   else
-    rc = vr_allreduce(ctx, stream, algo, (int)transport, ins, in_place ? NULL : outs, nelems, (uint32_t *)seq.buf);
+    rc = vr_allreduce(ctx, stream, algo, (int)transport, ins, in_place ? NULL : outs, (size_t)nelems,
+                      (uint32_t *)seq.buf);
   Py_END_ALLOW_THREADS
   PyBuffer_Release(&seq);
   return PyLong_FromLong(rc);
@@ -125,12 +149,12 @@ static PyObject *allreduce_static(PyObject *self, PyObject *const *args, Py_ssiz
   int algo = -1, rc = algo_of(args[1], &algo);
   if (rc) return rc < 0 ? NULL : PyLong_FromLong(rc);
   vr_ctx *ctx = (vr_ctx *)(uintptr_t)PyLong_AsUnsignedLongLongMask(args[0]);
-  const size_t nelems = (size_t)PyLong_AsUnsignedLongLongMask(args[4]);
-  if (PyErr_Occurred() || stream_of(args[5], &stream)) return NULL;
+  unsigned long long nelems;
+  if (PyErr_Occurred() || number_of(args[4], ct_size_t, &nelems) || stream_of(args[5], &stream)) return NULL;
   const int in_place = args[3] == Py_None;
   if (fill_table(args[2], ins) || (!in_place && fill_table(args[3], outs))) return NULL;
   Py_BEGIN_ALLOW_THREADS
-  rc = vr_allreduce_static(ctx, stream, algo, ins, in_place ? NULL : outs, nelems);
+  rc = vr_allreduce_static(ctx, stream, algo, ins, in_place ? NULL : outs, (size_t)nelems);
   Py_END_ALLOW_THREADS
   return PyLong_FromLong(rc);
 }
@@ -144,4 +168,14 @@ static PyMethodDef methods[] = {
 static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "_call", "Collective calls of the C ABI.", -1, methods,
                                     NULL, NULL, NULL, NULL};
 
-PyMODINIT_FUNC PyInit__call(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__call(void) {
+  PyObject *ct = PyImport_ImportModule("ctypes");
+  if (!ct) return NULL;
+  ct_cast = PyObject_GetAttrString(ct, "cast");
+  ct_void_p = PyObject_GetAttrString(ct, "c_void_p");
+  ct_size_t = PyObject_GetAttrString(ct, "c_size_t");
+  ct_int = PyObject_GetAttrString(ct, "c_int");
+  ct_error = PyObject_GetAttrString(ct, "ArgumentError");
+  Py_DECREF(ct);
+  return ct_cast && ct_void_p && ct_size_t && ct_int && ct_error ? PyModule_Create(&module) : NULL;
+}

@@ -1,16 +1,23 @@
-"""What the collective calls from Python take for a stream and for a table of device addresses:
-all that ctypes converts to a c_void_p.  Null contexts, so that nothing reaches a device."""
+"""What the collective calls from Python take for a stream, a count and a table of device
+addresses: all that ctypes converts in a call of the C ABI, and nothing that it refuses.  Null
+contexts, so that nothing reaches a device."""
 import ctypes as C
 
+import numpy as np
 import pytest
 
 import gpu_ipc_example_amd as vr
 from gpu_ipc_example_amd import binding
 
 
-def call(stream, ptrs=(8, 16)):
+def call(stream, ptrs=(8, 16), nelems=16, transport=vr.TRANSPORT_DIRECT):
     vr.lib()
-    return binding._call.allreduce(0, C.c_uint32(1), "simple", vr.TRANSPORT_DIRECT, ptrs, None, 16, stream)
+    return binding._call.allreduce(0, C.c_uint32(1), "simple", transport, ptrs, None, nelems, stream)
+
+
+def call_ctypes(stream, nelems=16, transport=vr.TRANSPORT_DIRECT):
+    return vr.lib().vr_allreduce(None, stream, vr.algo_id("simple"), transport, (C.c_void_p * 2)(8, 16), None, nelems,
+                                 C.byref(C.c_uint32(1)))
 
 
 class Holder:
@@ -18,15 +25,34 @@ class Holder:
         self._as_parameter_ = p
 
 
+def same_as_ctypes(**where):
+    """Taken or refused as ctypes does."""
+    try:
+        want = call_ctypes(**where)
+    except C.ArgumentError as e:
+        with pytest.raises(type(e)):
+            call(**where)
+        return False
+    assert call(**where) == want != 0        # no context
+    return True
+
+
 def test_streams_that_ctypes_takes():
-    want = call(None)
-    assert want != 0        # no context
-    for stream in (0, 64, C.c_void_p(), C.c_void_p(64), Holder(C.c_void_p(64)), Holder(C.c_void_p()), Holder(64),
-                   Holder(None)):
-        assert call(stream) == want
-    for stream in ("x", 1.5, object(), [], Holder("x")):
-        with pytest.raises((TypeError, AttributeError)):
-            call(stream)
+    for stream in (None, 0, 64, True, -1, 1 << 70, C.c_void_p(), C.c_void_p(64), Holder(C.c_void_p(64)),
+                   Holder(C.c_void_p()), Holder(64), Holder(None), Holder(Holder(8)), C.pointer(C.c_int(3)),
+                   C.byref(C.c_int(3)), (C.c_char * 8)(), C.c_char_p(b"x"), b"x", "x", Holder("x")):
+        assert same_as_ctypes(stream=stream), stream
+    for stream in (1.5, object(), [], C.c_int(4), C.c_size_t(4), Holder(1.5), Holder(C.c_int(4))):
+        assert not same_as_ctypes(stream=stream), stream
+
+
+@pytest.mark.parametrize("where", ["nelems", "transport"])
+def test_numbers_that_ctypes_takes(where):
+    exact = C.c_size_t if where == "nelems" else C.c_int
+    for number in (1, True, np.int64(1), np.uint8(1), exact(1), Holder(1), Holder(exact(1)), Holder(Holder(1)), -1, 1 << 70):
+        assert same_as_ctypes(stream=None, **{where: number}), number
+    for number in (16.0, None, "16", b"16", object(), C.c_short(16), Holder(16.0)):
+        assert not same_as_ctypes(stream=None, **{where: number}), number
 
 
 def test_tables():
