@@ -263,13 +263,13 @@ class VirtualRanks:
         _check(lib().vr_ctx_create(device, nranks, C.byref(h)))
         self._h, self.nranks, self.device = h, nranks, device
         self._address = h.value          # of the context, 0 once closed
-        self._wire_reserved = False
+        self._wire_reserved = False      # spares collective calls the reservation's own call
         self.seq_no = C.c_uint32(1)
 
     def close(self):
         if self._h:
             lib().vr_ctx_destroy(self._h)
-            self._h, self._address = None, 0
+            self._h, self._address, self._wire_reserved = None, 0, False
 
     def __del__(self):
         try:
@@ -282,14 +282,14 @@ class VirtualRanks:
 
     def reserve_wire(self):
         """Allocate and zero the wire transport's scratch (idempotent)."""
-        if not self._wire_reserved:
-            _check(lib().vr_ctx_reserve_wire(self._h))
-            self._wire_reserved = True
+        _check(lib().vr_ctx_reserve_wire(self._h))
+        self._wire_reserved = True
 
     def _reserve_for(self, algo, transport):
         # The C ABI never allocates inside a collective call; this wrapper reserves
         # the scratch on the first call that will take the wire transport.
-        if transport == TRANSPORT_WIRE or (transport == TRANSPORT_DEFAULT and algo == "parallel"):
+        if not self._wire_reserved and (transport == TRANSPORT_WIRE or
+                                        (transport == TRANSPORT_DEFAULT and algo == "parallel")):
             self.reserve_wire()
 
     def rank_scratch_bytes(self):
@@ -375,7 +375,7 @@ class VirtualRanks:
 
     def allreduce(self, algo, bufs, nelems, outs=None, transport=TRANSPORT_DEFAULT, stream=None):
         assert len(bufs) == self.nranks
-        if transport != TRANSPORT_DIRECT and not self._wire_reserved:
+        if not self._wire_reserved:
             self._reserve_for(algo, transport)
         rc = _call.allreduce(self._address, self.seq_no, algo, transport, bufs, outs, nelems, stream)
         if rc:
@@ -389,8 +389,8 @@ class VirtualRanks:
                                        groups, subgroups, simd))
 
     def allgather(self, algo, inputs, outputs, nelems, transport=TRANSPORT_DEFAULT, stream=None):
-        if transport == TRANSPORT_WIRE:
-            self.reserve_wire()
+        if not self._wire_reserved:
+            self._reserve_for(algo, transport)
         rc = _call.allgather(self._address, self.seq_no, algo, transport, inputs, outputs, nelems, stream)
         if rc:
             _check(rc)

@@ -129,6 +129,29 @@ def test_no_device_is_a_clean_error():
     assert e.value.code == "NO_DEVICE"
 
 
+def test_a_closed_context_is_refused_whatever_it_had_reserved(monkeypatch):
+    """Every call that needs the scratch, on a handle that is closed after a reservation (of a
+    context that is none: no GPU here)."""
+    L = vr.lib()
+    ctx = vr.VirtualRanks.__new__(vr.VirtualRanks)
+    ctx._h, ctx._address, ctx.nranks, ctx.device = C.c_void_p(8), 8, 2, 0
+    ctx._wire_reserved, ctx.seq_no = False, C.c_uint32(1)
+    with monkeypatch.context() as m:
+        m.setattr(binding, "lib", lambda: type("L", (), {
+            "vr_ctx_reserve_wire": staticmethod(lambda h: 0), "vr_ctx_destroy": staticmethod(lambda h: 0)}))
+        ctx.reserve_wire()
+        ctx.close()
+    calls = (ctx.reserve_wire,
+             lambda: ctx.allreduce("parallel", (8, 16), 16),
+             lambda: ctx.allreduce("simple", (8, 16), 16, transport=vr.TRANSPORT_WIRE),
+             lambda: ctx.allgather("allgather_simple", (8, 16), (32, 64), 8, transport=vr.TRANSPORT_WIRE),
+             lambda: ctx.allreduce_static("simple", (8, 16), 16))
+    for call in calls:
+        with pytest.raises(vr.VRError) as e:
+            call()
+        assert e.value.code == "INVALID" and L.vr_last_error_detail() == b"null ctx"
+
+
 def test_latency_family_launches_like_the_others_beyond_its_sizes():
     MiB = 1 << 20
     for nranks in (2, 4, 8):
