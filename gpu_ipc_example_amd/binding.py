@@ -2,14 +2,17 @@
 the collective calls, where the time a call takes is the host's, the CPython module _call
 (csrc/vr_pycall.c).
 
-No fallback exists: if a shared library is missing or a call fails, an
-exception is raised.  Device buffers are plain integers (device addresses), so
+No fallback exists: if the shared library is missing or a call fails, an
+exception is raised.  (Where _call was not built for this interpreter the same calls of the
+library are made through ctypes.)  Device buffers are plain integers (device addresses), so
 callers may hand in ``torch.Tensor.data_ptr()`` values or use the library's own
 vr_malloc plumbing through :class:`DeviceBuffer`.
 """
 import ctypes as C
+import importlib
 import os
 import subprocess
+import sys
 
 import numpy as np
 
@@ -19,6 +22,7 @@ _SO = os.path.join(_HERE, "libvrank_allreduce.so")
 ALGOS = ("small", "simple", "bisect", "parallel", "small_pcie_p", "simple_pcie_p", "small_ring",
          "simple_ring", "small_pcie", "simple_pcie", "allgather_small", "allgather_simple",
          "simple_transmit")
+MAX_RANKS = 16       # VR_MAX_RANKS
 TRANSPORT_DEFAULT, TRANSPORT_DIRECT, TRANSPORT_WIRE = 0, 1, 2
 
 # vr_status -> Python exception class; the texts come from vr_strerror.
@@ -52,14 +56,14 @@ def library_path():
 
 def build_library(force=False):
     """Compile the gfx950 library in-tree with hipcc (works without a GPU)."""
-    args = ["make", "-s", "-C", os.path.join(_HERE, "csrc"), "-j8"]
+    args = ["make", "-s", "-C", os.path.join(_HERE, "csrc"), "-j8", "PYTHON=" + sys.executable]
     if force:
         subprocess.run(args + ["clean"], check=True)
     subprocess.run(args, check=True)
 
 
 _lib = None
-_call = None       # the collective calls (csrc/vr_pycall.c)
+_call = None       # the collective calls: csrc/vr_pycall.c, or _CtypesCalls where it was not built
 
 
 def lib():
@@ -144,9 +148,31 @@ def lib():
         f = getattr(L, name)          # AttributeError here = header and library disagree
         f.restype, f.argtypes = res, args
     L._signatures = sig
-    from . import _call as call
+    try:
+        call = importlib.import_module("._call", __package__)
+    except ModuleNotFoundError:       # not built for this interpreter; one that does not load raises
+        call = _CtypesCalls
     _lib, _call = L, call
     return L
+
+
+class _CtypesCalls:
+    """What _call does, through ctypes."""
+
+    @staticmethod
+    def allreduce(address, seq_no, algo, transport, bufs, outs, nelems, stream):
+        return lib().vr_allreduce(address, stream, algo_id(algo), transport, _table(bufs),
+                                  _table(outs) if outs is not None else None, nelems, C.byref(seq_no))
+
+    @staticmethod
+    def allgather(address, seq_no, algo, transport, inputs, outputs, nelems, stream):
+        return lib().vr_allgather(address, stream, algo_id(algo), transport, _table(inputs),
+                                  _table(outputs) if outputs is not None else None, nelems, C.byref(seq_no))
+
+    @staticmethod
+    def allreduce_static(address, algo, bufs, outs, nelems, stream):
+        return lib().vr_allreduce_static(address, stream, algo_id(algo), _table(bufs),
+                                         _table(outs) if outs is not None else None, nelems)
 
 
 def _check(status):
@@ -168,7 +194,8 @@ def parse_nelems(text):
 
 
 def _table(ptrs):
-    return (C.c_void_p * len(ptrs))(*[C.c_void_p(int(p)) for p in ptrs])
+    # (as long as any context's table, so that one that is too short ends in null pointers)
+    return (C.c_void_p * max(len(ptrs), MAX_RANKS))(*[C.c_void_p(int(p)) for p in ptrs])
 
 
 def check_allreduce(algo, nranks, ptrs, nelems):

@@ -89,3 +89,35 @@ def test_tables_that_change_while_they_are_read():
             "print('read whole')\n")
     r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and "read whole" in r.stdout, (r.returncode, r.stderr)
+
+
+def test_the_module_is_built_for_one_interpreter_where_its_headers_are():
+    """Its name carries the interpreter's tag; without Python's headers the library and the CLI
+    are built all the same."""
+    import os
+    import subprocess
+    import sys
+    import sysconfig
+    headers = os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h"))
+    if headers:
+        assert binding._call.__file__.endswith("_call" + sysconfig.get_config_var("EXT_SUFFIX"))
+    csrc = os.path.join(os.path.dirname(binding.__file__), "csrc")
+    for include, built in ((sysconfig.get_paths()["include"], headers), ("/nonexistent", False)):
+        r = subprocess.run(["make", "-n", "-B", "-C", csrc, "PYTHON=" + sys.executable, "PYINC=" + include], capture_output=True,
+                           text=True, timeout=120)
+        assert r.returncode == 0 and "libvrank_allreduce.so" in r.stdout and "vr_main" in r.stdout
+        assert ("vr_pycall.c" in r.stdout) == built
+
+
+def test_the_calls_through_ctypes():
+    """What stands in for the module where it was not built: the same results of the same calls."""
+    vr.lib()
+    for outs in (None, (24, 32)):
+        for algo, n in (("simple", 16), ("allgather_simple", 16), ("simple", 1 << 41)):
+            a, b = C.c_uint32(3), C.c_uint32(3)
+            args = (algo, vr.TRANSPORT_DIRECT, [8, 16], outs, n, None)
+            assert binding._call.allreduce(0, a, *args) == binding._CtypesCalls.allreduce(0, b, *args) != 0
+            assert binding._call.allgather(0, a, *args) == binding._CtypesCalls.allgather(0, b, *args) != 0
+            assert a.value == b.value == 3
+            args = (algo, [8, 16], outs, n, None)
+            assert binding._call.allreduce_static(0, *args) == binding._CtypesCalls.allreduce_static(0, *args) != 0
