@@ -355,7 +355,7 @@ static int wire_launch(vr_ctx *c, hipStream_t s, const AlgoInfo *a, const PtrTab
     if (e != hipSuccess) return fail_hip(e, "launch_wire_clear_sinks");
   } else if (wlch.hist) {
     WireHistory &h = *wlch.hist;
-    const bool moved_back = h.used && (int32_t)(seq - h.next_min_seq) < 0;
+    const bool moved_back = h.used && wl::flags_may_repeat(seq, h.next_min_seq);
     if (wraps || moved_back || (h.used && (h.last_flow != (int)flow || h.last_fmt != (int)fmt))) {
       if (int rc = wire_clear(k, N, s)) return rc;
       h.used = false;

@@ -101,5 +101,14 @@ VR_HD Layout layout_for(int nranks, uint32_t wpr_max, bool with_simple) {
   return Layout{slots, flag_off, sink_bytes, 2 * sink_bytes};
 }
 
+// ---- flag values ----------------------------------------------------------------------------
+// May the flag values of a launch that starts at `seq` lie in the sinks already?  `next_min`
+// is one more than the largest value written since they were cleared (no launch writes across
+// the wrap through 0).  Receivers look for equal values, so only values above all written ones
+// are safe, and above means as unsigned numbers: a counter that wrapped between two launches
+// that use the sinks (in calls that use none: direct transport, messages through LDS) is far
+// below, though the difference modulo 2^32 is small and positive.
+VR_HD bool flags_may_repeat(uint32_t seq, uint32_t next_min) { return seq < next_min; }
+
 }  // namespace wl
 }  // namespace vr

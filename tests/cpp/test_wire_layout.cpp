@@ -2,10 +2,12 @@
 // slot) combination the kernels of each flow form, with the slot functions the
 // kernels themselves use (vr_wire_layout.h), and proves that every message slot
 // and every flag word lies inside a sink sized by the host code's layout_for().
+// Then the rule by which the host clears the sinks' flag values.
 // No GPU, no library: plain g++.
 #include <stdio.h>
 
 #include <initializer_list>
+#include <set>
 
 #include "vr_wire_layout.h"
 
@@ -75,7 +77,33 @@ static void walk(int flow, int N, uint32_t wpr, const Layout &l) {
   EXPECT(p.max_slot + 1 == p.need);
 }
 
+// Launches that write flags [seq, seq + used) into sinks that are cleared when
+// flags_may_repeat says so, at sequence numbers that other calls move on in between (and
+// callers choose): no launch meets a value that is there already.
+static void walk_flags(uint32_t random) {
+  const uint32_t around[] = {1, 2, 40, 0x7fffffe0u, 0x80000000u, 0x80000021u, 0xffffff00u, 0xffffffd0u, 0xfffffff0u};
+  std::set<uint32_t> written;
+  uint32_t next_min = 0;
+  bool used = false;
+  for (int launch = 0; launch < 200; ++launch) {
+    random = random * 1664525u + 1013904223u;
+    const uint32_t seq = around[(random >> 8) % (sizeof around / sizeof *around)] + ((random >> 16) & 7u);
+    const uint32_t n = 1 + ((random >> 24) & 7u);     // (never across the wrap: the host clears there)
+    if (used && flags_may_repeat(seq, next_min)) {
+      written.clear();
+      used = false;
+    }
+    for (uint32_t f = seq; f < seq + n; ++f) EXPECT(written.insert(f).second);
+    used = true;
+    next_min = seq + n;
+  }
+}
+
 int main() {
+  for (uint32_t s = 1; s <= 64; ++s) walk_flags(s * 2654435761u);
+  EXPECT(!flags_may_repeat(7, 7) && !flags_may_repeat(0xffffffffu, 7) && flags_may_repeat(6, 7));
+  // small values, values near the end, then small ones again after a wrap
+  EXPECT(!flags_may_repeat(0xfffffff0u, 4) && flags_may_repeat(3, 0xfffffff4u));
   const int ranks[] = {2, 4, 8, 16};
   int cases = 0;
   for (int N : ranks)

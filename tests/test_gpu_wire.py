@@ -153,6 +153,37 @@ def test_sequence_number_wrap_never_uses_flag_zero(ctxs, oracle):
     src.free()
 
 
+@pytest.mark.parametrize("transport", [vr.TRANSPORT_DIRECT, WIRE])
+def test_counter_that_wraps_in_a_call_that_uses_no_scratch(oracle, transport):
+    """Flags of small values from early launches through scratch stay in its slots; launches near
+    the end of the counter, then a call that wraps it without looking at the scratch: the next
+    launch through scratch, at the small number that call returned, meets none of them."""
+    import ctypes as C
+    ctx = vr.VirtualRanks(8)
+    n = 8 * 4096
+
+    def through_scratch(seq, seed):
+        ins = H.make_inputs(oracle, 8, n, seed)
+        src = H.RankBuffers(8, n)
+        src.upload(ins)
+        ctx.allreduce_grid("simple", src.ptrs, n, 16, 8, 16, transport=WIRE, seq_no=seq)
+        ctx.check()
+        H.assert_all_ranks_equal(oracle, src.download(), oracle.rotated(ins), "seq %#x" % seq)
+        src.free()
+
+    for seq in range(1, 9):
+        through_scratch(seq, 8800 + 10 * seq)
+    through_scratch(0xFFFFFFF0, 8900)
+    ctx.seq_no = C.c_uint32(0xFFFFFFFF)
+    ins = H.make_inputs(oracle, 8, n, 8910)
+    got, _ = H.run_allreduce(ctx, "simple", ins, transport=transport)
+    H.assert_all_ranks_equal(oracle, got, oracle.rotated(ins))
+    assert 1 <= ctx.seq_no.value <= 8
+    for seq in range(ctx.seq_no.value, 9):
+        through_scratch(seq, 8920 + 10 * seq)
+    ctx.close()
+
+
 def test_poll_timeout_is_reported_and_recoverable(ctxs, oracle):
     """A spin limit of one poll makes some wave give up before its message has
     arrived; every wave still runs to completion, the context reports the
