@@ -83,56 +83,55 @@ struct Msg {
   u32x4 d[U];
 };
 
-// Where a chunk lies in every rank's buffer.  As in the direct kernels (tile_start,
-// vr_direct.hip) wires are laid on 128-byte lines of the outputs and vectors on 16 bytes:
-// the first wire may begin up to 112 bytes before the chunk (lanes there form offsets below
-// zero, beyond the buffer's length) and its first vector may straddle the chunk's start:
-// it is loaded whole (the 8 bytes below lie in the same 16 bytes of the same buffer) and its
-// upper half is stored.  A chunk may end inside a vector: the bounds check works dword by
-// dword.  LINED = every chunk starts on a line: none of that (the extra scalar instructions
-// of eight waves per 8 KiB cost 7 % at 8 x 32 MiB).
-template <bool LINED>
-struct Span {
-  size_t at;        // first byte, from the start of a buffer
-  uint32_t bytes;   // length of the buffer resource
-  uint32_t off;     // the lane's offset in it
-  bool straddles;   // the vector at offset 0 begins 8 bytes below the chunk
-};
-template <bool LINED, int U>
-static __device__ __forceinline__ Span<LINED> span_of(const Args &a, uint32_t chunk, uint32_t lane) {
-  const size_t base = chunk * a.pitch + a.seg_off;
-  const uint32_t off = blockIdx.x * (1024u * U) + lane * 16u;
-  if constexpr (LINED) return {base, a.seg_bytes, off, false};
-  const uint32_t addr = (a.lines & 0xffu) + (uint32_t)base, head = addr & (a.lines >> 8);
-  return {base - head, a.seg_bytes + head, off - ((addr - head) & 112u), blockIdx.x == 0 && head != 0};
+// Where a chunk lies in every rank's buffer (wl::wire_span), by what chunks are known to start
+// on.  ON_LINES: none of the arithmetic for other starts (the extra scalar instructions of eight
+// waves per 8 KiB cost 7 % at 8 x 32 MiB).  ON_VECTORS: messages of 16 bytes, no vector straddles
+// a start.
+enum Starts : int { ON_LINES, ON_VECTORS, ON_HALVES };
+template <Starts S>
+struct Span : wl::Span {};
+template <Starts S, int U>
+static __device__ __forceinline__ Span<S> span_of(const Args &a, uint32_t chunk, uint32_t lane) {
+  return {wl::wire_span(S == ON_LINES, chunk * a.pitch + a.seg_off, a.seg_bytes, a.lines,
+                        blockIdx.x * (1024u * U) + lane * 16u, blockIdx.x == 0)};
 }
-template <bool LINED>
-static __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *base, const Span<LINED> &s) {
+template <Starts S>
+static __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *base, const Span<S> &s) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(static_cast<const char *>(base) + s.at), 0, (int)s.bytes,
                                            0x00020000);
 }
 // Offset of the lane's vector u, added up in a register: as an immediate of the instruction
 // it would be added after the wrap of a first wire's offset below zero had been compared.
-template <bool LINED>
-static __device__ __forceinline__ uint32_t vec_off(const Span<LINED> &s, int u) {
+template <Starts S>
+static __device__ __forceinline__ uint32_t vec_off(const Span<S> &s, int u) {
   uint32_t off = s.off + (uint32_t)u * 1024u;
-  if (!LINED && u) asm("" : "+v"(off));
+  if (S != ON_LINES && u) asm("" : "+v"(off));
   return off;
 }
-template <int U, int LD, bool LINED>
-static __device__ __forceinline__ Msg<U> load(const void *base, const Span<LINED> &s) {
+template <int U, int LD, Starts S>
+static __device__ __forceinline__ Msg<U> load(const void *base, const Span<S> &s) {
   const __amdgpu_buffer_rsrc_t rs = rsrc(base, s);
   Msg<U> m;
 #pragma unroll
-  for (int u = 0; u < U; ++u) m.d[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, vec_off(s, u), 0, LD);
+  for (int u = 0; u < U; ++u)
+    m.d[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, S == ON_HALVES && u == 0 ? s.first_load() : vec_off(s, u), 0, LD);
   return m;
 }
-template <int U, int ST, bool LINED>
-static __device__ __forceinline__ void store(void *base, const Span<LINED> &s, const Msg<U> &m) {
+// To be called on a loaded message before it is used, and after other work that need not wait
+// for the load: puts the half of a straddling vector where it belongs.
+template <int U, Starts S>
+static __device__ __forceinline__ void settle(Msg<U> &m, const Span<S> &s) {
+  if (S == ON_HALVES && s.half()) {
+    m.d[0].z = m.d[0].x;
+    m.d[0].w = m.d[0].y;
+  }
+}
+template <int U, int ST, Starts S>
+static __device__ __forceinline__ void store(void *base, const Span<S> &s, const Msg<U> &m) {
   const __amdgpu_buffer_rsrc_t rs = rsrc(base, s);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    if (!LINED && u == 0 && s.straddles && s.off == 0)
+    if (S == ON_HALVES && u == 0 && s.half())
       __builtin_amdgcn_raw_buffer_store_b64(u32x2{m.d[0].z, m.d[0].w}, rs, 8u, 0, ST);
     else
       __builtin_amdgcn_raw_buffer_store_b128(m.d[u], rs, vec_off(s, u), 0, ST);
@@ -211,14 +210,15 @@ struct Sinks {
 template <int N, int U>
 using ParallelSinks = Sinks<U, N, 2 * N>;
 
-template <int N, int DT, int U, bool LINED, int LD, int ST>
+template <int N, int DT, int U, Starts S, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_parallel(Args a) {
   VR_GROUP_PROLOGUE;
   const ParallelSinks<N, U> sk(lds, lane);
   const int y = (int)blockIdx.y;
-  const auto at = span_of<LINED, U>(a, y, lane);
+  const auto at = span_of<S, U>(a, y, lane);
   Msg<U> v = load<U, LD>(src, at);
   sk.ready();
+  settle(v, at);
   if (r != y) {
     sk.put(r, v);
     sk.publish();
@@ -246,14 +246,16 @@ __global__ __launch_bounds__(64 * N) void k_group_parallel(Args a) {
 template <int N, int U>
 using SequentialSinks = Sinks<U, N * N, 2 * N * N>;
 
-template <int N, int DT, int U, bool LINED, int LD, int ST>
+template <int N, int DT, int U, Starts S, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_sequential(Args a) {
   VR_GROUP_PROLOGUE;
   const SequentialSinks<N, U> sk(lds, lane);
   Msg<U> x[N];                                             // x[i]: chunk of rank r + i
 #pragma unroll
-  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<LINED, U>(a, (r + i) % N, lane));
+  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<S, U>(a, (r + i) % N, lane));
   sk.ready();
+#pragma unroll
+  for (int i = 0; i < N; ++i) settle(x[i], span_of<S, U>(a, (r + i) % N, lane));
 #pragma unroll
   for (int i = 1; i < N; ++i) sk.put((r + i) % N * N + r, x[i]);
   sk.publish();
@@ -268,12 +270,12 @@ __global__ __launch_bounds__(64 * N) void k_group_sequential(Args a) {
   for (int i = 1; i < N; ++i) sk.put(r * N + (r + i) % N, v);
   sk.publish();
   sk.template raise_others<N>(N * N + r * N, r);           // flag owner r, peer
-  store<U, ST>(dst, span_of<LINED, U>(a, r, lane), v);
+  store<U, ST>(dst, span_of<S, U>(a, r, lane), v);
   sk.template await_others<N>(poll, N * N + r, r, N);
 #pragma unroll
   for (int i = 1; i < N; ++i) x[i] = sk.get((r + i) % N * N + r);
 #pragma unroll
-  for (int i = 1; i < N; ++i) store<U, ST>(dst, span_of<LINED, U>(a, (r + i) % N, lane), x[i]);
+  for (int i = 1; i < N; ++i) store<U, ST>(dst, span_of<S, U>(a, (r + i) % N, lane), x[i]);
 }
 
 // ---- RingTransmit (sequential_transmit.hpp:429-516) --------------------------------------
@@ -317,13 +319,13 @@ struct Ring {
   }
 };
 
-template <int N, int DT, int U, bool LINED, int LD, int ST>
+template <int N, int DT, int U, Starts S, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_ring(Args a) {
   VR_GROUP_PROLOGUE;
   const RingSinks<N, U> sk(lds, lane);
   Msg<U> x[N];                                             // x[i]: chunk of rank r - i
 #pragma unroll
-  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<LINED, U>(a, (r + N - i) % N, lane));
+  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<S, U>(a, (r + N - i) % N, lane));
   const Ring<N, U> ring{sk, poll, r, (r + 1) % N};
   sk.ready();
   ring.send(0, x[0]);
@@ -332,20 +334,20 @@ __global__ __launch_bounds__(64 * N) void k_group_ring(Args a) {
     add<DT, U>(x[i], ring.recv(i - 1));
     ring.send(i, x[i]);
   }
-  store<U, ST>(dst, span_of<LINED, U>(a, (r + 1) % N, lane), x[N - 1]);
+  store<U, ST>(dst, span_of<S, U>(a, (r + 1) % N, lane), x[N - 1]);
 #pragma unroll
   for (int i = 1; i < N; ++i) {                            // write back, forward except on the last hop
     const Msg<U> v = ring.recv(N - 2 + i);
     if (i < N - 1) ring.send(N - 1 + i, v);
-    store<U, ST>(dst, span_of<LINED, U>(a, (r + 1 + N - i) % N, lane), v);
+    store<U, ST>(dst, span_of<S, U>(a, (r + 1 + N - i) % N, lane), v);
   }
 }
 
-template <int N, int DT, int U, bool LINED, int LD, int ST>
+template <int N, int DT, int U, Starts S, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_allgather(Args a) {
   VR_GROUP_PROLOGUE;
   const RingSinks<N, U> sk(lds, lane);
-  const auto own = span_of<LINED, U>(a, r, lane);
+  const auto own = span_of<S, U>(a, r, lane);
   // the input is one slice long: the same bytes of it as of the own slot
   const char *slot0 = src - (size_t)r * a.pitch;
   Msg<U> v = load<U, LD>(slot0, own);
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(64 * N) void k_group_allgather(Args a) {
   for (int i = 1; i < N; ++i) {
     v = ring.recv(i - 1);
     if (i < N - 1) ring.send(i, v);
-    store<U, ST>(dst, span_of<LINED, U>(a, (r + N - i) % N, lane), v);
+    store<U, ST>(dst, span_of<S, U>(a, (r + N - i) % N, lane), v);
   }
 }
 
@@ -369,20 +371,22 @@ __global__ __launch_bounds__(64 * N) void k_group_allgather(Args a) {
 template <int N, int U>
 using BisectSinks = Sinks<U, 2 * N, 4 * N>;
 
-template <int N, int DT, int U, bool LINED, int LD, int ST>
+template <int N, int DT, int U, Starts S, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_bisect(Args a) {
   constexpr int B = N / 2;
   VR_GROUP_PROLOGUE;
   const BisectSinks<N, U> sk(lds, lane);
   const int y = (int)blockIdx.y, h = r & 1, l = r >> 1, pair = r ^ 1;
-  const auto close = span_of<LINED, U>(a, h * B + y, lane),
-             far = span_of<LINED, U>(a, (1 - h) * B + y, lane);
-  const Msg<U> f = load<U, LD>(src, far);
+  const auto close = span_of<S, U>(a, h * B + y, lane),
+             far = span_of<S, U>(a, (1 - h) * B + y, lane);
+  Msg<U> f = load<U, LD>(src, far);
   Msg<U> v = load<U, LD>(src, close);
   sk.ready();
+  settle(f, far);
   sk.put(pair, f);                                         // scatterFar
   sk.publish();
   sk.raise(pair, 1);
+  settle(v, close);
   poll.until([&] { return sk.look(r) != 0; });
   add<DT, U>(v, sk.get(r));                                // pair sum
   if (y != l) {
@@ -420,21 +424,22 @@ struct Pick {
 
 template <int N, int DT, int LD, int ST, int U, bool LINED>
 Pick pick_flow(WireFlow flow) {
+  constexpr Starts kWhole = LINED ? ON_LINES : ON_VECTORS, kAny = LINED ? ON_LINES : ON_HALVES;
   if constexpr (N <= 8) {
     switch (flow) {
-      case WIRE_PARALLEL: return {reinterpret_cast<const void *>(&k_group_parallel<N, DT, U, LINED, LD, ST>), N, ParallelSinks<N, U>::kBytes};
-      case WIRE_SEQUENTIAL:
-      case WIRE_SIMPLE: return {reinterpret_cast<const void *>(&k_group_sequential<N, DT, U, LINED, LD, ST>), 1, SequentialSinks<N, U>::kBytes};
-      case WIRE_RING: return {reinterpret_cast<const void *>(&k_group_ring<N, DT, U, LINED, LD, ST>), 1, RingSinks<N, U>::kBytes};
+      case WIRE_PARALLEL: return {reinterpret_cast<const void *>(&k_group_parallel<N, DT, U, kAny, LD, ST>), N, ParallelSinks<N, U>::kBytes};
+      case WIRE_SEQUENTIAL: return {reinterpret_cast<const void *>(&k_group_sequential<N, DT, U, kWhole, LD, ST>), 1, SequentialSinks<N, U>::kBytes};
+      case WIRE_SIMPLE: return {reinterpret_cast<const void *>(&k_group_sequential<N, DT, U, kAny, LD, ST>), 1, SequentialSinks<N, U>::kBytes};
+      case WIRE_RING: return {reinterpret_cast<const void *>(&k_group_ring<N, DT, U, kWhole, LD, ST>), 1, RingSinks<N, U>::kBytes};
       case WIRE_ALLGATHER:   // no adds: one instantiation serves both element types
         if constexpr (U == 1)
-          return {reinterpret_cast<const void *>(&k_group_allgather<N, DT_F16, U, LINED, LD, ST>), 1, RingSinks<N, U>::kBytes};
+          return {reinterpret_cast<const void *>(&k_group_allgather<N, DT_F16, U, kWhole, LD, ST>), 1, RingSinks<N, U>::kBytes};
         break;
       default: break;
     }
   }
   if constexpr (N >= 4) {
-    if (flow == WIRE_BISECT) return {reinterpret_cast<const void *>(&k_group_bisect<N, DT, U, LINED, LD, ST>), N / 2, BisectSinks<N, U>::kBytes};
+    if (flow == WIRE_BISECT) return {reinterpret_cast<const void *>(&k_group_bisect<N, DT, U, kAny, LD, ST>), N / 2, BisectSinks<N, U>::kBytes};
   }
   return {nullptr, 0, 0};
 }
@@ -479,7 +484,7 @@ hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow
   a.in = in;
   a.out = out;
   a.pitch = chunk_bytes;
-  a.lines = lines_of(out, flow == WIRE_ALLGATHER ? 0u : head_mask_of(nranks, in, out));   // (whole 16-byte messages)
+  a.lines = lines_of(out, flow == WIRE_PARALLEL || flow == WIRE_BISECT || flow == WIRE_SIMPLE ? head_mask_of(nranks, in, out) : 0u);
   a.spin_limit = spin_limit;
   a.status = status;
   void *kargs[] = {&a};

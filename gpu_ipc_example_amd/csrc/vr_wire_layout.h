@@ -101,6 +101,34 @@ VR_HD Layout layout_for(int nranks, uint32_t wpr_max, bool with_simple) {
   return Layout{slots, flag_off, sink_bytes, 2 * sink_bytes};
 }
 
+// ---- wires of the work-group form (vr_wire_group.hip) ------------------------------------------
+// Where a lane's vectors of a wire lie in a rank's buffer.  As in the direct kernels
+// (tile_start, vr_direct.hip) wires are laid on 128-byte lines of the outputs and vectors on 16
+// bytes: the first wire may begin up to 112 bytes before the chunk (lanes there form offsets
+// below zero, beyond the buffer's length) and its first vector may straddle the chunk's start.
+// A straddling vector's upper half is what the chunk begins with; the lower half belongs to the
+// chunk before, or lies ahead of the buffer.  A chunk may end inside a vector: the bounds check
+// works dword by dword.
+struct Span {
+  size_t at;        // first byte of the buffer resource, from the start of a rank's buffer
+  uint32_t bytes;   // length of the buffer resource
+  uint32_t off;     // the lane's offset in it
+  bool straddles;   // the vector at offset 0 begins 8 bytes below the chunk
+  // Is the lane's first vector the straddling one?
+  VR_HD bool half() const { return straddles && off == 0; }
+  // Its load takes the 16 bytes from the chunk's start on: the half that counts comes as the
+  // lower one, and no byte outside the buffer is read.
+  VR_HD uint32_t first_load() const { return half() ? 8u : off; }
+};
+// The chunk's bytes [base, base + seg_bytes) of each buffer; `lines` as lines_of forms it
+// (vr_direct.hip); `off` = the lane's place counted from the start of the first wire.  `lined` =
+// every chunk starts on a line.
+VR_HD Span wire_span(bool lined, size_t base, uint32_t seg_bytes, uint32_t lines, uint32_t off, bool first_wire) {
+  if (lined) return Span{base, seg_bytes, off, false};
+  const uint32_t addr = (lines & 0xffu) + (uint32_t)base, head = addr & (lines >> 8);
+  return Span{base - head, seg_bytes + head, off - ((addr - head) & 112u), first_wire && head != 0};
+}
+
 // ---- flag values ----------------------------------------------------------------------------
 // May the flag values of a launch that starts at `seq` lie in the sinks already?  `next_min`
 // is one more than the largest value written since they were cleared (no launch writes across

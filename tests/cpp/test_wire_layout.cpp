@@ -2,12 +2,13 @@
 // slot) combination the kernels of each flow form, with the slot functions the
 // kernels themselves use (vr_wire_layout.h), and proves that every message slot
 // and every flag word lies inside a sink sized by the host code's layout_for().
-// Then the rule by which the host clears the sinks' flag values.
+// Then the accesses of the work-group form to inputs and outputs, and the rule by which the host clears the sinks' flag values.
 // No GPU, no library: plain g++.
 #include <stdio.h>
 
 #include <initializer_list>
 #include <set>
+#include <vector>
 
 #include "vr_wire_layout.h"
 
@@ -77,6 +78,45 @@ static void walk(int flow, int N, uint32_t wpr, const Layout &l) {
   EXPECT(p.max_slot + 1 == p.need);
 }
 
+// The work-group form's loads and stores of one rank's buffer, dword by dword, as the buffer
+// resources of the kernels bound them: nothing outside the buffer is touched, every dword of it
+// is stored once, from the dword that was loaded for it.  `place` = the buffer's place in its
+// 128-byte line, `mask` = 8 where all buffers agree about their place in 16 bytes.
+static void walk_spans(int chunks, size_t pitch, size_t seg_max, uint32_t unroll, uint32_t place, uint32_t mask) {
+  const bool lined = ((place | pitch) & 127u) == 0;
+  const size_t total = (size_t)chunks * pitch;
+  const uint32_t lines = place | mask << 8;
+  std::vector<int> stored(total / 4, 0);
+  for (int c = 0; c < chunks; ++c)
+    for (size_t seg_off = 0; seg_off < pitch; seg_off += seg_max) {
+      const size_t seg = pitch - seg_off < seg_max ? pitch - seg_off : seg_max;
+      const uint32_t wires = (uint32_t)((seg + (lined ? 0 : 120) + 1024u * unroll - 1) / (1024u * unroll));
+      for (uint32_t block = 0; block < wires; ++block)
+        for (uint32_t lane = 0; lane < 64; ++lane) {
+          const Span s = wire_span(lined, c * pitch + seg_off, (uint32_t)seg, lines, block * (1024u * unroll) + lane * 16u, block == 0);
+          for (uint32_t u = 0; u < unroll; ++u) {
+            const uint32_t load = u ? s.off + u * 1024u : s.first_load(), store = s.off + u * 1024u;
+            long long source[4];          // the byte of the buffer each dword came from, -1: dropped
+            for (uint32_t d = 0; d < 4; ++d) {
+              source[d] = -1;
+              if ((uint64_t)load + 4 * d + 4 > s.bytes) continue;
+              source[d] = (long long)s.at + load + 4 * d;
+              EXPECT(source[d] >= 0 && source[d] + 4 <= (long long)total);
+            }
+            const bool half = u == 0 && s.half();
+            if (half) source[2] = source[0], source[3] = source[1];
+            for (uint32_t d = half ? 2 : 0; d < 4; ++d) {
+              if ((uint64_t)store + 4 * d + 4 > s.bytes) continue;
+              const long long to = (long long)s.at + store + 4 * d;
+              EXPECT(to >= 0 && to + 4 <= (long long)total && source[d] == to);
+              if (to >= 0 && to + 4 <= (long long)total) ++stored[to / 4];
+            }
+          }
+        }
+    }
+  for (int n : stored) EXPECT(n == 1);
+}
+
 // Launches that write flags [seq, seq + used) into sinks that are cleared when
 // flags_may_repeat says so, at sequence numbers that other calls move on in between (and
 // callers choose): no launch meets a value that is there already.
@@ -106,6 +146,14 @@ int main() {
   EXPECT(!flags_may_repeat(0xfffffff0u, 4) && flags_may_repeat(3, 0xfffffff4u));
   const int ranks[] = {2, 4, 8, 16};
   int cases = 0;
+  for (size_t pitch : {8u, 16u, 24u, 112u, 120u, 128u, 136u, 1016u, 1024u, 1032u, 2040u, 2048u, 2056u, 9u * 1024u + 24u})
+    for (size_t seg_max : {(size_t)1 << 30, (size_t)1024, (size_t)2048})
+      for (uint32_t unroll : {1u, 2u})
+        for (uint32_t place = 0; place < 128; place += 8)
+          for (uint32_t mask : {0u, 8u}) {
+            walk_spans(3, pitch, seg_max, unroll, place, mask);
+            ++cases;
+          }
   for (int N : ranks)
     for (uint32_t wpr_max = 4; wpr_max <= 2048; wpr_max *= 2)
       for (int with_simple = 0; with_simple < 2; ++with_simple) {
