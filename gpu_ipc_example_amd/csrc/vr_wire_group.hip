@@ -117,22 +117,13 @@ static __device__ __forceinline__ Msg<U> load(const void *base, const Span<S> &s
     m.d[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, S == ON_HALVES && u == 0 ? s.first_load() : vec_off(s, u), 0, LD);
   return m;
 }
-// To be called on a loaded message before it is used, and after other work that need not wait
-// for the load: puts the half of a straddling vector where it belongs.
-template <int U, Starts S>
-static __device__ __forceinline__ void settle(Msg<U> &m, const Span<S> &s) {
-  if (S == ON_HALVES && s.half()) {
-    m.d[0].z = m.d[0].x;
-    m.d[0].w = m.d[0].y;
-  }
-}
 template <int U, int ST, Starts S>
 static __device__ __forceinline__ void store(void *base, const Span<S> &s, const Msg<U> &m) {
   const __amdgpu_buffer_rsrc_t rs = rsrc(base, s);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if (S == ON_HALVES && u == 0 && s.half())
-      __builtin_amdgcn_raw_buffer_store_b64(u32x2{m.d[0].z, m.d[0].w}, rs, 8u, 0, ST);
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2{m.d[0].x, m.d[0].y}, rs, 8u, 0, ST);
     else
       __builtin_amdgcn_raw_buffer_store_b128(m.d[u], rs, vec_off(s, u), 0, ST);
   }
@@ -218,7 +209,6 @@ __global__ __launch_bounds__(64 * N) void k_group_parallel(Args a) {
   const auto at = span_of<S, U>(a, y, lane);
   Msg<U> v = load<U, LD>(src, at);
   sk.ready();
-  settle(v, at);
   if (r != y) {
     sk.put(r, v);
     sk.publish();
@@ -254,8 +244,6 @@ __global__ __launch_bounds__(64 * N) void k_group_sequential(Args a) {
 #pragma unroll
   for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<S, U>(a, (r + i) % N, lane));
   sk.ready();
-#pragma unroll
-  for (int i = 0; i < N; ++i) settle(x[i], span_of<S, U>(a, (r + i) % N, lane));
 #pragma unroll
   for (int i = 1; i < N; ++i) sk.put((r + i) % N * N + r, x[i]);
   sk.publish();
@@ -379,14 +367,12 @@ __global__ __launch_bounds__(64 * N) void k_group_bisect(Args a) {
   const int y = (int)blockIdx.y, h = r & 1, l = r >> 1, pair = r ^ 1;
   const auto close = span_of<S, U>(a, h * B + y, lane),
              far = span_of<S, U>(a, (1 - h) * B + y, lane);
-  Msg<U> f = load<U, LD>(src, far);
+  const Msg<U> f = load<U, LD>(src, far);
   Msg<U> v = load<U, LD>(src, close);
   sk.ready();
-  settle(f, far);
   sk.put(pair, f);                                         // scatterFar
   sk.publish();
   sk.raise(pair, 1);
-  settle(v, close);
   poll.until([&] { return sk.look(r) != 0; });
   add<DT, U>(v, sk.get(r));                                // pair sum
   if (y != l) {

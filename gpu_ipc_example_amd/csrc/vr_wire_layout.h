@@ -116,8 +116,9 @@ struct Span {
   bool straddles;   // the vector at offset 0 begins 8 bytes below the chunk
   // Is the lane's first vector the straddling one?
   VR_HD bool half() const { return straddles && off == 0; }
-  // Its load takes the 16 bytes from the chunk's start on: the half that counts comes as the
-  // lower one, and no byte outside the buffer is read.
+  // Its load takes the 16 bytes from the chunk's start on, so that no byte outside the buffer
+  // is read.  The half that counts comes, is added up (the lane does so in every rank) and is
+  // stored as the lower one.
   VR_HD uint32_t first_load() const { return half() ? 8u : off; }
 };
 // The chunk's bytes [base, base + seg_bytes) of each buffer; `lines` as lines_of forms it

@@ -104,10 +104,10 @@ static void walk_spans(int chunks, size_t pitch, size_t seg_max, uint32_t unroll
               EXPECT(source[d] >= 0 && source[d] + 4 <= (long long)total);
             }
             const bool half = u == 0 && s.half();
-            if (half) source[2] = source[0], source[3] = source[1];
-            for (uint32_t d = half ? 2 : 0; d < 4; ++d) {
-              if ((uint64_t)store + 4 * d + 4 > s.bytes) continue;
-              const long long to = (long long)s.at + store + 4 * d;
+            for (uint32_t d = 0; d < (half ? 2u : 4u); ++d) {
+              const uint32_t offset = (half ? 8u : store) + 4 * d;
+              if ((uint64_t)(half ? 8u : store) + 4 * d + 4 > s.bytes) continue;
+              const long long to = (long long)s.at + offset;
               EXPECT(to >= 0 && to + 4 <= (long long)total && source[d] == to);
               if (to >= 0 && to + 4 <= (long long)total) ++stored[to / 4];
             }
