@@ -445,14 +445,21 @@ static hipError_t with_policy(const Tuning &t, F &&f) {
 }
 
 // The runtime's launch call itself (the <<< >>> form goes through a push and a pop of the
-// configuration first: 2.47 us a launch, 2.27 without).
+// configuration first: 2.47 us a launch, 2.27 without).  A refused launch is this call's to
+// report: it must not stay the thread's last error for other code to find.
+hipError_t launch_kernel(const void *fn, dim3 grid, dim3 block, void **kargs, uint32_t lds, hipStream_t s,
+                         hipEvent_t ev0, hipEvent_t ev1) {
+  const hipError_t e = ev0 || ev1 ? hipExtLaunchKernel(fn, grid, block, kargs, lds, s, ev0, ev1, 0)
+                                  : hipLaunchKernel(fn, grid, block, kargs, lds, s);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
 template <typename... P>
 static hipError_t launch(void (*kernel)(P...), dim3 grid, dim3 block, uint32_t lds, hipStream_t s, hipEvent_t ev0,
                          hipEvent_t ev1, P... args) {
   void *kargs[] = {&args...};
-  const void *fn = reinterpret_cast<const void *>(kernel);
-  if (ev0 || ev1) return hipExtLaunchKernel(fn, grid, block, kargs, lds, s, ev0, ev1, 0);
-  return hipLaunchKernel(fn, grid, block, kargs, lds, s);
+  return launch_kernel(reinterpret_cast<const void *>(kernel), grid, block, kargs, lds, s, ev0, ev1);
 }
 
 // Bytes the tiles of a chunk may have to start early to lie on the outputs' lines (tile_start).

@@ -68,6 +68,11 @@ struct KernelEvents {
 };
 extern thread_local KernelEvents tl_kernel_events;
 
+// Launches a kernel with the events given (null: none); an error is returned and not left
+// behind as the thread's last.
+hipError_t launch_kernel(const void *fn, dim3 grid, dim3 block, void **kargs, uint32_t lds, hipStream_t s,
+                         hipEvent_t ev0, hipEvent_t ev1);
+
 // Direct transport -----------------------------------------------------------
 // in/out hold nranks pointers; chunk_elems = nelems / nranks.  Pointers and chunks are
 // multiples of 8 bytes (all-gather: 16).

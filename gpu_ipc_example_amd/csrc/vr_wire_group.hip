@@ -28,8 +28,6 @@
 // wave has given up) a wave records a time-out in the status word and runs to its
 // end without waiting again.
 
-#include <hip/hip_ext.h>
-
 #include "vr_internal.h"
 
 namespace vr {
@@ -482,8 +480,7 @@ hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow
     const dim3 grid((uint32_t)((seg + (lined ? 0 : 120) + wire - 1) / wire), k.rows), block(64u * (uint32_t)nranks);
     hipEvent_t ev0 = off == 0 ? tl_kernel_events.start : nullptr;
     hipEvent_t ev1 = off + seg >= chunk_bytes ? tl_kernel_events.stop : nullptr;
-    const hipError_t e = ev0 || ev1 ? hipExtLaunchKernel(k.fn, grid, block, kargs, lds, s, ev0, ev1, 0)
-                                    : hipLaunchKernel(k.fn, grid, block, kargs, lds, s);
+    const hipError_t e = launch_kernel(k.fn, grid, block, kargs, lds, s, ev0, ev1);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -15,6 +15,7 @@ CPP_TEST = os.path.join(ROOT, "tests", "cpp", "test_host_api")
 GRAPH_TEST = os.path.join(ROOT, "tests", "cpp", "test_graph")
 LAYOUT_TEST = os.path.join(ROOT, "tests", "cpp", "test_wire_layout")
 VERIFY_TEST = os.path.join(ROOT, "tests", "cpp", "test_verify")
+LAUNCH_TEST = os.path.join(ROOT, "tests", "cpp", "test_launch_errors")
 
 
 def run(cmd, **kw):
@@ -38,6 +39,12 @@ def test_host_side_checks_of_the_cpp_header():
     832-838) and the element arithmetic under them, against the oracle; CPU only."""
     r = run([VERIFY_TEST], timeout=120)
     assert r.returncode == 0 and "verify ok" in r.stdout, r.stdout[-2000:]
+
+
+def test_a_refused_launch_leaves_no_error_behind():
+    """The runtime's last error after launches that it refuses; CPU only."""
+    r = run([LAUNCH_TEST], timeout=120)
+    assert r.returncode == 0 and " 0 failures" in r.stdout, r.stdout
 
 
 def test_cli_rejects_bad_arguments_like_the_reference():
