@@ -157,6 +157,7 @@ struct GroupPlan {
   GroupPolicy policy;
   int unroll;       // 16-byte vectors per lane and message: 1, or 2 at 8 and 16 ranks
   int wgs_per_cu;   // residency cap, 0 = none
+  size_t segment_bytes = (size_t)1 << 30;   // bytes of a chunk one launch covers (32-bit offsets); multiple of 16
 };
 hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow, int nranks, DType dtype,
                              const PtrTable &in, const PtrTable &out, size_t chunk_bytes, const GroupPlan &plan,

@@ -33,7 +33,6 @@
 // another wave has given up) a wave records a time-out in the status word and
 // runs to completion without waiting again, so the grid always drains.
 
-
 #include <mutex>
 #include <unordered_map>
 

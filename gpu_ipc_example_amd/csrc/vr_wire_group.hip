@@ -472,7 +472,7 @@ hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow
   a.spin_limit = spin_limit;
   a.status = status;
   void *kargs[] = {&a};
-  const size_t seg_max = (size_t)1 << 30;   // 32-bit offsets
+  const size_t seg_max = plan.segment_bytes;
   for (size_t off = 0; off < chunk_bytes; off += seg_max) {
     const size_t seg = chunk_bytes - off < seg_max ? chunk_bytes - off : seg_max;
     a.seg_off = off;

@@ -167,8 +167,10 @@ static int group_launch(vr_ctx *c, hipStream_t s, const AlgoInfo *a, const PtrTa
   bool in_place = !a->allgather;
   for (int r = 0; r < N; ++r) in_place = in_place && in.p[r] == out.p[r];
   const size_t reads = (size_t)N * chunk_bytes * (a->allgather ? 1 : N);
-  const hipError_t e = launch_wire_group(s, c->dev, flow, N, c->dtype, in, out, chunk_bytes,
-                                         group_plan(flow, N, reads, in_place), spin_limit_of(c), c->status);
+  GroupPlan plan = group_plan(flow, N, reads, in_place);
+  if (c->tune.segment_kib != -1) plan.segment_bytes = (size_t)c->tune.segment_kib << 10;
+  const hipError_t e = launch_wire_group(s, c->dev, flow, N, c->dtype, in, out, chunk_bytes, plan, spin_limit_of(c),
+                                         c->status);
   return e == hipSuccess ? VR_OK : fail_hip(e, "launch_wire_group");
 }
 

@@ -334,7 +334,8 @@ int vr_ctx_set_spin_limit(vr_ctx *ctx, uint64_t polls);
  * "f16_wide" (1 = binary16 adds computed through
  * binary32 and rounded back after every add: the same bits, a longer ALU section),
  * "segment_kib" (KiB of a chunk one launch
- * covers; chunks longer than this, at most 1 GiB, take several launches);
+ * covers, also of the wire transport's through LDS; chunks longer than this, at most 1 GiB,
+ * take several launches);
  * for the wire transport, where setting any of them also moves launches that hold all
  * ranks from LDS to scratch memory, "wire_fenced" (how the Rt64_128 families, i.e. simple,
  * bisect, parallel, simple_pcie_p, simple_ring, simple_pcie, simple_transmit,

@@ -98,3 +98,31 @@ def test_allgather_beyond_half_the_cache(oracle):
     for r, got in enumerate(run_allgather_wire(ctx, "allgather_simple", ins, False)):
         assert (got == want).all(), r
     ctx.close()
+
+
+@pytest.mark.parametrize("nranks,algo", [(2, "simple"), (8, "parallel"), (4, "bisect"), (16, "bisect"), (8, "simple_transmit"),
+                                         (8, "simple_ring"), (8, "simple_pcie")])
+def test_chunks_of_several_launches(oracle, nranks, algo):
+    """Chunks longer than one launch covers: whole and ragged last segments, starts of segments
+    inside a vector (offset 8) and inside a line."""
+    msg = 16 if algo in ("simple_ring", "simple_pcie") else 8
+    ctx = vr.VirtualRanks(nranks)
+    for kib in (1, 3):
+        ctx.set_tuning(segment_kib=kib)
+        for k, chunk in enumerate((1024 * kib - msg, 1024 * kib, 1024 * kib + msg, 4 * 1024 * kib, 4 * 1024 * kib + 5 * msg)):
+            for inplace in (True, False):
+                for offset in (0, 8) if msg == 8 else (0, 16):
+                    run(oracle, ctx, algo, nranks * chunk // 2, F16, inplace, offset, 80_000 + 100 * k)
+    ctx.close()
+
+
+def test_gathers_of_several_launches(oracle):
+    ctx = vr.VirtualRanks(8)
+    ctx.set_tuning(segment_kib=1)
+    for n in (504, 512, 520, 8 * 643):
+        ins = [oracle.generate_dt(F16, n, 81_000 + r, DIST_NORMAL, 0.0, 1.0) for r in range(8)]
+        want = oracle.allgather(ins)
+        for alias in (False, True):
+            for r, got in enumerate(run_allgather_wire(ctx, "allgather_simple", ins, alias)):
+                assert (got == want).all(), (n, r, alias)
+    ctx.close()
