@@ -128,10 +128,12 @@ int main() {
     VRCK(vr_ctx_check(ctx, stream));
   }
 
-  // The allocation-free wire all-reduce clears its sinks in every call and starts
-  // its flags from 1, so a captured call replays correctly: six replays with
-  // eager work in between, each compared with the oracle.
-  {
+  // The allocation-free wire all-reduce keeps its messages in LDS, or, with a wire_* key
+  // set, clears its sinks in every call and starts its flags from 1, so a captured call
+  // replays correctly: six replays with eager work in between, each compared with the
+  // oracle.  Through LDS, with the reference's messages and with flag words.
+  for (int fenced : {-1, 0, 4}) {
+    VRCK(vr_ctx_set_tuning(ctx, "wire_fenced", fenced));
     int parallel_id = -1;
     VRCK(vr_algo_from_string("parallel", &parallel_id));
     const std::vector<uint16_t> &sum = s1;       // the rotated-order sum of the inputs
@@ -152,13 +154,14 @@ int main() {
         HIPCK(hipMemcpy(got.data(), mid[r], n * 2, hipMemcpyDeviceToHost));
         const size_t bad = vro_count_mismatch(got.data(), sum.data(), n);
         if (bad) {
-          printf("static replay %d rank %d: %zu mismatches\n", replay, r, bad);
+          printf("static replay %d rank %d wire_fenced %d: %zu mismatches\n", replay, r, fenced, bad);
           ++failures;
         }
       }
     }
     (void)hipGraphExecDestroy(e3);
     (void)hipGraphDestroy(g3);
+    VRCK(vr_ctx_set_tuning(ctx, "wire_fenced", -1));
   }
 
   // A streaming launch under capture: two ranks of 80 MiB, out of place, run as a one-trip

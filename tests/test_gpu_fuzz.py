@@ -44,6 +44,10 @@ def test_random_cases(oracle, seed):
         knobs.update(oneshot=rng2.choice((-1, -1, 0, 1)), wgs_per_cu=rng2.choice((-1, 0, 1, 2, 4, 8)),
                      block=rng2.choice((-1, -1, 64, 256, 512, 1024)),
                      deal=rng2.choice((-1, -1, 0, 1, 2, nranks)))
+        # (half of the wire cases through LDS: no wire_* setting, no grid)
+        if transport == vr.TRANSPORT_WIRE and rng2.random() < 0.5:
+            knobs.update({k: -1 for k in knobs if k.startswith("wire_")})
+            grid = None
         ctxs[nranks].set_tuning(**knobs)
         ins = H.make_inputs(oracle, nranks, n, 10_000 * seed + 37 * case,
                             p1=rng.choice((0.02, 1.0, 30.0, 3000.0)))

@@ -1,6 +1,8 @@
-"""GPU parity tests of the wire transport (message passing through scratch with
-flags, one persistent kernel holding every virtual rank's work-groups).  Same
-oracle, same bit-exact bar as the direct transport."""
+"""GPU parity tests of the wire transport.  Same oracle, same bit-exact bar as the
+direct transport.  A call that holds all ranks and leaves every wire_* setting and
+the grid alone passes its messages through LDS; any wire_* setting (SCRATCH: one
+that changes nothing else) or a grid makes it pass them through scratch with flags,
+one persistent kernel holding every virtual rank's work-groups."""
 import numpy as np
 import pytest
 
@@ -10,6 +12,18 @@ from tests.oracle_lib import DIST_NORMAL, DIST_UNIFORM
 
 pytestmark = pytest.mark.gpu
 WIRE = vr.TRANSPORT_WIRE
+THROUGH_LDS, SCRATCH = dict(), dict(wire_ahead=4)       # 4 is what the library takes by itself
+
+
+@pytest.fixture
+def tuned(ctxs):
+    """Settings on the shared eight-rank context, taken back when the test ends."""
+    def set_(kw):
+        keys.update(kw)
+        ctxs[8].set_tuning(**kw)
+    keys = {}
+    yield set_
+    ctxs[8].set_tuning(**{k: -1 for k in keys})
 
 
 @pytest.fixture(scope="module")
@@ -89,11 +103,13 @@ def test_result_independent_of_grid(ctxs, oracle, groups):
             H.assert_all_ranks_equal(oracle, got, want, "%s g=%d w=%d" % (algo, groups, subgroups))
 
 
-def test_many_launches_reuse_slots_and_flags(ctxs, oracle):
-    """Back-to-back launches without host synchronisation: slot rings wrap, the
-    sequence number keeps the flags apart."""
+@pytest.mark.parametrize("form", [THROUGH_LDS, SCRATCH])
+def test_many_launches_reuse_slots_and_flags(ctxs, oracle, tuned, form):
+    """Back-to-back launches without host synchronisation: slot rings in scratch wrap, the
+    sequence number keeps their flags apart."""
     from gpu_ipc_example_amd.binding import DeviceBuffer
     ctx = ctxs[8]
+    tuned(form)
     n = 8 * 4096 * 6            # several steps per launch at the automatic grid
     for algo in ("small", "simple", "bisect", "small_ring", "simple_pcie", "simple_transmit"):
         base = H.make_inputs(oracle, 8, n, 900)
@@ -132,10 +148,12 @@ def test_sequence_number_moving_backwards_is_safe(ctxs, oracle):
     assert e.value.code == "INVALID"
 
 
-def test_sequence_number_wrap_never_uses_flag_zero(ctxs, oracle):
-    """A 32-bit counter that would run through 0 restarts from 1 on clean scratch."""
+@pytest.mark.parametrize("form", [THROUGH_LDS, SCRATCH])
+def test_sequence_number_wrap_never_uses_flag_zero(ctxs, oracle, tuned, form):
+    """A 32-bit counter that would run through 0 restarts from 1, on clean scratch."""
     import ctypes as C
     ctx = ctxs[8]
+    tuned(form)
     n = 8 * 4096 * 8
     ins = H.make_inputs(oracle, 8, n, 88)
     want = oracle.rotated(ins)
@@ -184,11 +202,14 @@ def test_counter_that_wraps_in_a_call_that_uses_no_scratch(oracle, transport):
     ctx.close()
 
 
-def test_poll_timeout_is_reported_and_recoverable(ctxs, oracle):
+@pytest.mark.parametrize("form", [THROUGH_LDS, SCRATCH])
+def test_poll_timeout_is_reported_and_recoverable(oracle, form):
     """A spin limit of one poll makes some wave give up before its message has
     arrived; every wave still runs to completion, the context reports the
-    time-out, and the next launch works."""
+    time-out, and the next launch works: through scratch, where messages were left
+    half delivered, from cleared sinks."""
     ctx = vr.VirtualRanks(8)
+    ctx.set_tuning(**form)
     ins = H.make_inputs(oracle, 8, 1 << 20, 31)
     ctx.set_spin_limit(1)
     timed_out = False
@@ -200,15 +221,16 @@ def test_poll_timeout_is_reported_and_recoverable(ctxs, oracle):
             timed_out = True
     assert timed_out
     ctx.set_spin_limit(0)
-    got, _ = H.run_allreduce(ctx, "simple_ring", ins, transport=WIRE)
-    H.assert_all_ranks_equal(oracle, got, oracle.rotated(ins))
+    for algo in ("simple_ring", "small_ring", "bisect"):
+        got, _ = H.run_allreduce(ctx, algo, ins, transport=WIRE)
+        H.assert_all_ranks_equal(oracle, got, H.expected(oracle, algo, ins), algo)
     ctx.close()
 
 
-@pytest.mark.parametrize("fenced", [-1, 0])
+@pytest.mark.parametrize("fenced", [-1, 0, 4])
 def test_config3_bisect_32mib_wire(ctxs, oracle, fenced):
-    """The headline shape through scratch: flag words (the library's choice) and the
-    reference's 128-byte messages."""
+    """The headline shape through LDS (the library's choice) and through scratch: with the
+    reference's 128-byte messages (0) and with flag words (4)."""
     ins = H.make_inputs(oracle, 8, 16777216, 3000, DIST_NORMAL, 0.0, 0.02)
     ctxs[8].set_tuning(wire_fenced=fenced)
     try:
@@ -226,12 +248,14 @@ def test_parallel_defaults_to_wire_and_sweep_sizes(ctxs, oracle):
         H.assert_all_ranks_equal(oracle, got, oracle.rotated(ins), "n=%d" % n)
 
 
-@pytest.mark.parametrize("log2_elems,fenced", [(24, -1), (25, -1), (26, -1), (27, -1), (24, 0), (27, 0)])
+@pytest.mark.parametrize("log2_elems,fenced", [(24, -1), (25, -1), (26, -1), (27, -1), (24, 0), (27, 0),
+                                               (24, 4), (27, 4)])
 def test_config5_parallel_large_sizes(ctxs, oracle, log2_elems, fenced):
     """The sweep's named protocol on its default (wire) transport at 32, 64, 128 and
     256 MiB per rank: N(0,1) inputs, rank 0 compared in full with the rotated-order
-    oracle, the other ranks by equality with rank 0.  With the library's own choice of
-    format (flag words) and with the reference's 256-byte messages (fenced 0)."""
+    oracle, the other ranks by equality with rank 0.  Through LDS (the library's own
+    choice) and through scratch, with the reference's 256-byte messages (fenced 0) and
+    with flag words (4)."""
     n = 1 << log2_elems
     ins = H.make_inputs(oracle, 8, n, 5000 + log2_elems)
     want = oracle.rotated(ins)
@@ -347,8 +371,8 @@ def test_eight_byte_messages_for_the_128_byte_families(oracle, algo):
 
 @pytest.mark.parametrize("cooperative", [0, 1])
 def test_plain_and_cooperative_launch(oracle, cooperative):
-    """By default the launch is plain when the occupancy query proves the grid
-    co-resident; both forms can be forced."""
+    """Launches through scratch are plain by default, the occupancy query having proved the
+    grid co-resident; both forms can be forced."""
     ctx = vr.VirtualRanks(8)
     ctx.set_tuning(wire_cooperative=cooperative)
     for algo in ("small", "simple", "bisect", "small_ring"):

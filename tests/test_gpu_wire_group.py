@@ -78,10 +78,11 @@ def test_allgather_edges(oracle, nranks):
 
 
 @pytest.mark.parametrize("nranks,algo,mib,inplace", [(4, "simple_ring", 194, True), (4, "bisect", 194, False),
-                                                     (8, "simple", 71, True)])
+                                                     (8, "simple", 71, True), (16, "bisect", 98, False)])
 def test_capped_and_resident_launches(oracle, nranks, algo, mib, inplace):
     """Just inside the sizes (bytes of all ranks' inputs) that cap the work-groups per compute unit,
-    and the largest that stay cacheable in place, with a chunk that ends inside a wire."""
+    the largest that stay cacheable in place, and sixteen ranks with one vector per lane, with a
+    chunk that ends inside a wire."""
     ctx = vr.VirtualRanks(nranks)
     msg = 16 if algo == "simple_ring" else 8
     chunk = (mib << 20) // nranks ** 2 // 16 * 16 + 3 * msg
