@@ -74,7 +74,8 @@ CFG2_KERNEL_TRACE = (4.20, "direct_allreduce_small_8x1MiB_kernel_trace.md")
 
 # --transport: how the virtual ranks exchange data (0 = the protocol's default).
 TRANSPORT = 0
-# --transport static: vr_allreduce_static (wire transport through the library's fixed scratch region)
+# --transport static: vr_allreduce_static (wire transport without an allocation: through LDS, or through the
+# library's fixed scratch region where --tune sets a wire_* key)
 STATIC = False
 
 
@@ -458,7 +459,7 @@ def latency_block(vr, binding, want_check, gpu_results, iters):
     groups = max(10, iters // 20)
     b2b, host_c = c2.time_allreduce_grouped(algo, ptrs, ne, groups, 20, transport=TRANSPORT)
     b2b = b2b * 1e3
-    # the same call through the Python binding (ctypes marshalling on top of the C call)
+    # the same call through the Python binding (its argument conversion on top of the C call)
     t0 = time.perf_counter()
     for _ in range(iters):
         c2.allreduce(algo, ptrs, ne, transport=TRANSPORT)
@@ -478,7 +479,7 @@ def latency_block(vr, binding, want_check, gpu_results, iters):
                                   "note": "hipEventRecord before and after each launch: adds the event "
                                           "commands' own time to the kernel's"},
         "back_to_back_us_per_launch": round(float(np.median(b2b)), 3),
-        "host_call_us": {"c_abi": round(host_c, 3), "through_ctypes": round(host_py, 3),
+        "host_call_us": {"c_abi": round(host_c, 3), "from_python": round(host_py, 3),
                          "note": "host wall time for one vr_allreduce call to return (validation, launch "
                                  "heuristics, kernel enqueue), mean over back-to-back calls; c_abi is "
                                  "measured inside the library's own loop"},
@@ -522,8 +523,8 @@ def allgather_block(vr, binding, want_check, gpu_results):
 
 
 def cfg5_block(vr, binding):
-    """Config 5 at three sizes: its named protocol `parallel` (message passing through
-    scratch) and the direct kernel (`simple`), in place on one buffer set as the
+    """Config 5 at three sizes: its named protocol `parallel` (message passing)
+    and the direct kernel (`simple`), in place on one buffer set as the
     reference's own run protocol has it (main.cpp:67-108)."""
     n = 8
     sizes = [1 << 20, 32 << 20, 256 << 20]
@@ -559,9 +560,9 @@ def main():
     ap.add_argument("--dtype", default="f16", choices=["f16", "bf16"],
                     help="element type of the adds (the reference instantiates both)")
     ap.add_argument("--transport", default="default", choices=["default", "direct", "wire", "static"],
-                    help="direct: one pass over HBM; wire: the reference's message passing through "
-                         "scratch; default: wire for 'parallel', direct otherwise; static: the "
-                         "allocation-free entry point (wire transport through the library's fixed region)")
+                    help="direct: one pass over HBM; wire: the reference's message passing, "
+                         "through LDS, or through scratch where --tune sets a wire_* key; default: wire for 'parallel', direct otherwise; static: the "
+                         "allocation-free entry point (wire transport; its scratch is the library's fixed region)")
     ap.add_argument("--inplace", action="store_true",
                     help="reference semantics: results overwrite the inputs (values saturate "
                          "after a few steps; traffic is identical)")

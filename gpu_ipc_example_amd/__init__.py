@@ -3,7 +3,7 @@
 The product is the C ABI in ``include/vrank_allreduce.h`` (built into
 ``libvrank_allreduce.so`` from ``csrc/``) and the C++ host header
 ``include/vrank/allreduce.hpp``.  This package is the Python-side binding of that
-C ABI (ctypes) used by the tests and the benchmark.
+C ABI (ctypes, and a CPython module for the collective calls) used by the tests and the benchmark.
 """
 from .binding import (  # noqa: F401
     ALGOS,

@@ -420,7 +420,8 @@ static Tuning default_tuning(int nranks, const AlgoInfo *a, size_t read_bytes, s
     // 9 MiB 4.5 us, the other launch 4.7), where both are bound by their start; beyond, the other protocols' launch is the faster
     // (out of place, 8 ranks, one / three sets of buffers: 16 MiB 5.9 / 7.3 -> 4.4 / 6.4 us,
     // 32 MiB 11.6 / 11.7 -> 8.1 / 11.0, 64 MiB 21.1 / 28.7 -> 20.4 / 20.2, 96 MiB 30.2 / 43.3 ->
-    // 29.6 / 34.9; in place 32 MiB 8.8 / 12.2 -> 8.0 / 11.3, 96 MiB even).
+    // 29.6 / 34.9; in place 32 MiB 8.8 / 12.2 -> 8.0 / 11.3, 96 MiB even; at 2 and 4 ranks with inputs
+    // that change, calls of 24 MiB are 3 to 11 % faster, of 96 MiB out of place 15 to 20 %, in place even).
     t.waves_per_cu = 8;
     t.oneshot = 1;
     t.nt_load = 0;

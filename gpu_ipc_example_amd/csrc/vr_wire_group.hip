@@ -16,8 +16,8 @@
 // times the algorithmic bytes at the L2 / fabric boundary, which carries about
 // 8 TB/s however much of it the memory-side cache serves; here only inputs and
 // outputs cross it.  ParallelTransmit, 8 ranks in place: 256 MiB per rank
-// 2196 -> 688 us (6.2 TB/s), 1 MiB per rank 14.4 -> 5.6 us (the host's pace);
-// RingTransmit, 4 x 8 MB: 39.3 -> 11.1 us; ring all-gather, 8 x 1 MB: 51 -> 12.2 us.
+// 2196 -> 681 us (6.3 TB/s), 1 MiB per rank 14.5 -> 4.2 us (bfloat16 4.65);
+// RingTransmit, 4 x 8 MB: 39.4 -> 10.8 us; ring all-gather, 8 x 1 MB: 51.6 -> 12.2 us.
 //
 // One wire per work-group and no loop: the hardware starts work-groups in index
 // order, so a launch sweeps the chunks front to back with all compute units close

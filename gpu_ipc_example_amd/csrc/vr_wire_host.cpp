@@ -107,18 +107,22 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
   const size_t MiB = (size_t)1 << 20;
   GroupPlan p = {GROUP_MIXED, 1, 0};
   // Cache policies, us per pass on one / three / ten sets of buffers in turn:
-  //  * in place up to 72 MiB, of which three sets fit the memory-side cache, everything stays
-  //    cacheable (8 x 4 MiB 9.1 / 12.9 / 16.0, streamed 13.9 / 15.9 / 15.9; 9 MiB per rank on 8, one
+  //  * in place up to 72 MiB everything stays cacheable: what else a caller's program touches
+  //    between two calls is not known here, so room is left for twice as much again (three sets
+  //    fit the memory-side cache) (8 x 4 MiB 9.1 / 12.9 / 16.0, streamed 13.9 / 15.9 / 15.9; 9 MiB per rank on 8, one
   //    and three sets: parallel 23.4 / 23.8, streamed 27.6 / 27.9, ring 8 x 8 MiB + 16 B
   //    20.7 / 20.5, streamed 27.2 / 27.3), beyond it streaming wins as soon as the buffers do
   //    not all fit (8 x 10 MiB: simple 26.3 / 33.5, streamed 30.4 / 30.5; 8 x 16 MiB
-  //    39.5 / 50.5 / 53.2, streamed 49.9 / 48.9 / 49.4);
+  //    39.5 / 50.5 / 53.2, streamed 49.9 / 48.9 / 49.4).  (The direct transport, which stays
+  //    cacheable up to 255 MiB, takes 41.5 there on one set and 52.0 with inputs that change, parallel 53.4
+  //    and 49.3.)
   //  * out of place up to half the memory-side cache of inputs: results are streamed past
   //    inputs that may stay (8 x 16 MiB 41.3 / 49.3 / 50.5, everything streamed
   //    50.2 / 50.2 / 49.4), beyond it everything streams (8 x 128 MiB 355, 351 us);
   //  * all-gather: results are streamed past the inputs at every size, they are N times as
   //    long (2 x 64 MiB 58.2 / 65.9, everything streamed 68.0 / 66.9; 8 x 16 MiB 193 / 222, streamed
-  //    238 / 230).
+  //    238 / 230; with inputs that change, 256 and 512 MiB of them: 8 x 32 MiB 399, streamed 416, 8 x 64
+  //    810, 821, 2 x 128 and 4 x 128 even).
   if (in_place) p.policy = reads <= 72 * MiB ? GROUP_RESIDENT : GROUP_STREAM;
   else if (reads > 128 * MiB && flow != WIRE_ALLGATHER) p.policy = GROUP_STREAM;
   // Two vectors per lane at 8 and 16 ranks, where that is the faster (fewer waves for the
@@ -148,7 +152,9 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
       // 8.4, two: 9.9; 8 x 32 MiB 97.7, two: 108.8
       if (nranks == 8 && reads >= 32 * MiB && reads <= 192 * MiB) p.unroll = 2;
       // Ring, four ranks, streaming: 48 KiB of loads per CU in flight instead of 128.
-      // 4 x 64 MiB 106 -> 94 us, 4 x 128 MiB 190.5 -> 169.5; 4 x 32 MiB 50.7, capped 50.9
+      // 4 x 64 MiB 106 -> 94 us, 4 x 128 MiB 190.5 -> 169.5; 4 x 32 MiB 50.7, capped 50.9.  (Eight
+      // ranks with one vector: their 64 KiB of slots hold a compute unit at two work-groups anyway;
+      // with two vectors no cap was timed.)
       if (flow == WIRE_RING && nranks == 4 && reads >= 192 * MiB) p.wgs_per_cu = 3;
       break;
     case WIRE_ALLGATHER:   // one vector: 8 x 4 MiB 49.0, two: 59.1 us
@@ -306,14 +312,17 @@ static int wire_launch(vr_ctx *c, hipStream_t s, const AlgoInfo *a, const PtrTab
     return fail(VR_ERR_INVALID, "sequence number 0 cannot be told from freshly zeroed scratch");
   const WireSinks &k = *wlch.sinks;
   const int N = c->nranks;
-  // The flag values of a launch are kernel arguments, and whether the sinks must
-  // be cleared first is decided here on the host: a captured launch would replay
-  // with stale flags.  (With always_clear every replay starts from clean sinks.)
+  // The flag values of a launch through scratch are kernel arguments, and whether the sinks
+  // must be cleared first is decided here on the host: a captured launch would replay with
+  // stale flags.  (With always_clear every replay starts from clean sinks.)  Launches through
+  // LDS keep no flags, but which form a call takes depends on the context's settings and the
+  // grid, so both are refused alike.
   if (!wlch.always_clear) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
-      return fail(VR_ERR_INVALID, "the wire transport cannot be captured into a graph: its flag values "
-                                  "are per-launch kernel arguments (capture the direct transport)");
+      return fail(VR_ERR_INVALID, "the wire transport cannot be captured into a graph: flag values "
+                                  "are per-launch kernel arguments (capture the direct transport or "
+                                  "vr_allreduce_static)");
     (void)hipGetLastError();
   }
   // Sinks the library owns (a launch against a caller's sinks leaves its messages there).
@@ -455,10 +464,11 @@ extern "C" int vr_allreduce_static(vr_ctx *ctx, void *stream, int algo, void *co
     return fail(VR_ERR_INVALID, "vr_allreduce_static has no room for SimpleTransmit's 2 MiB sender sections");
   WireSinks k;
   if (int rc = static_sinks(ctx, &k)) return rc;
-  // The region is shared by every context on the device and keeps the last
-  // call's messages: every call first clears the slots it is about to use (a
-  // fill kernel on the stream), so the flags can start from 1 each time.  The
-  // time-out word is the context's own, like that of its other wire launches.
+  // A context that sets a wire_* key sends its messages through the region (others use LDS and
+  // neither read nor write it).  It is shared by every context on the device and keeps the
+  // last call's messages: every call first clears the slots it is about to use (a fill kernel
+  // on the stream), so the flags can start from 1 each time.  The time-out word is the
+  // context's own, like that of its other wire launches.
   const WireLaunch wlch = {&k, nullptr, ctx->status, 0, ctx->nranks, true};
   uint32_t seq = 1, used = 0;
   return wire_launch(ctx, (hipStream_t)stream, p.a, p.in, p.out, p.chunk_elems * 2, p.vec_halves, &seq,

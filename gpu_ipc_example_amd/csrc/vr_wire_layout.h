@@ -118,7 +118,8 @@ struct Span {
   VR_HD bool half() const { return straddles && off == 0; }
   // Its load takes the 16 bytes from the chunk's start on, so that no byte outside the buffer
   // is read.  The half that counts comes, is added up (the lane does so in every rank) and is
-  // stored as the lower one.
+  // stored as the lower one.  (Moved up to its place after the load instead, simple_transmit at
+  // 8 x 4 MiB took 15.6 us for 14.8.)
   VR_HD uint32_t first_load() const { return half() ? 8u : off; }
 };
 // The chunk's bytes [base, base + seg_bytes) of each buffer; `lines` as lines_of forms it

@@ -278,18 +278,18 @@ int vr_ipc_barrier(int rank, int world, const char *instance, int generation);
 
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory: code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc.  A wire-transport vr_allreduce whose sinks live in a fixed
- * region of device memory that is part of the library's code object (about
- * 32 MiB per GPU, held until the process ends) instead of scratch reserved by the
- * context.  Calls no hipMalloc / hipFree and does not synchronise.
+ * forbid hipMalloc.  A wire-transport vr_allreduce that needs no scratch reserved by
+ * the context.  Calls no hipMalloc / hipFree and does not synchronise.
  * Limits: at most 8 ranks, at most 256 MiB (134217728 elements) per rank, every
- * all-reduce algo except simple_transmit; 32 to 128 wires per rank.  Beyond them:
- * VR_ERR_INVALID.  Every context on a GPU shares that GPU's region and each call
- * first clears the message slots it is about to use (a fill kernel on `stream`),
- * so calls that overlap in time on one GPU race: keep them on one stream or
- * otherwise ordered.  (A call whose context leaves every "wire_*" setting alone keeps
- * its messages in LDS: it neither touches the region nor clears anything.)  A time-out is recorded in the calling context's own status
- * word and reported by vr_ctx_check like those of vr_allreduce. */
+ * all-reduce algo except simple_transmit.  Beyond them: VR_ERR_INVALID.
+ * A call whose context leaves every "wire_*" setting alone keeps its messages in LDS and
+ * shares nothing with other calls.  With such a setting the sinks live in a fixed region
+ * of device memory that is part of the library's code object (about 32 MiB per GPU,
+ * held until the process ends; 32 to 128 wires per rank).  Every context on a GPU shares
+ * that GPU's region and each call through it first clears the message slots it is about
+ * to use (a fill kernel on `stream`), so such calls that overlap in time on one GPU race:
+ * keep them on one stream or otherwise ordered.  A time-out is recorded in the calling
+ * context's own status word and reported by vr_ctx_check like those of vr_allreduce. */
 int vr_allreduce_static(vr_ctx *ctx, void *stream, int algo, void *const bufs[], void *const outs[],
                         size_t nelems);
 

@@ -23,7 +23,7 @@ def run_pair(oracle, nranks, algo, sizes, seed, form):
     ctx.reserve_wire()
     for k, n in enumerate(sizes):
         ins = H.make_inputs(oracle, nranks, n, seed + 10 * k)
-        # existing entry point, context-owned scratch
+        # existing entry point: LDS or context-owned scratch
         ref = H.RankBuffers(nranks, n)
         ref.upload(ins)
         ctx.allreduce(algo, ref.ptrs, n, transport=vr.TRANSPORT_WIRE)
