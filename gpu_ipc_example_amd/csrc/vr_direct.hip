@@ -92,11 +92,10 @@ __device__ __forceinline__ void st_low(__amdgpu_buffer_rsrc_t r, h8 v) {
 struct TileStart {
   uint32_t head, skew;
 };
-// `lines` (lines_of): place of the first output in its line, and head_mask in the second
-// byte: an argument of its own, so that nothing waits for the pointer table.
-__device__ __forceinline__ TileStart tile_start(uint32_t lines, size_t base) {
-  const uint32_t at = (lines & 0xffu) + (uint32_t)base;
-  const uint32_t head = at & (lines >> 8);
+// `line`: place of the first output in its line; `base`: the chunk's start, from the outputs'.
+__device__ __forceinline__ TileStart tile_start(uint32_t line, uint32_t head_mask, size_t base) {
+  const uint32_t at = line + (uint32_t)base;
+  const uint32_t head = at & head_mask;
   return {head, (at + head) & 112u};
 }
 
@@ -126,19 +125,25 @@ __device__ __forceinline__ void rotate_left(T (&t)[M], int a) {
   }
 }
 
+// Pointer k of the launch: inputs, then outputs.
+template <int N>
+__device__ __forceinline__ char *ptr_of(const DirectArgs<N> &a, int k) {
+  return reinterpret_cast<char *>(a.address(k));
+}
+
 // op[k] = the input that is the k-th operand of the chain for the chunk owned by
 // `owner`.  All N pointers are fetched with static indices (one scalar load of the
 // whole table) and permuted in registers: a table lookup per operand would be N
 // dependent scalar loads at the head of every work-group.
 template <int N, int ORDER>
-__device__ __forceinline__ void select_operands(const PtrTable &in, int owner, const char *(&op)[N]) {
+__device__ __forceinline__ void select_operands(const DirectArgs<N> &a, int owner, const char *(&op)[N]) {
   if constexpr (ORDER == ORDER_COPY) {
 #pragma unroll
-    for (int k = 0; k < N; ++k) op[k] = static_cast<const char *>(in.p[k]);
+    for (int k = 0; k < N; ++k) op[k] = ptr_of(a, k);
   } else if constexpr (ORDER == ORDER_ROTATED) {
     // own chunk first, then rank+1, rank+2, ...
 #pragma unroll
-    for (int k = 0; k < N; ++k) op[k] = static_cast<const char *>(in.p[k]);
+    for (int k = 0; k < N; ++k) op[k] = ptr_of(a, k);
     rotate_left<N>(op, owner);
   } else {
     // pair sums in the order l, l+1, ... (mod N/2); inside a pair the rank of the
@@ -148,8 +153,8 @@ __device__ __forceinline__ void select_operands(const PtrTable &in, int owner, c
     const char *ev[B], *od[B];
 #pragma unroll
     for (int j = 0; j < B; ++j) {
-      ev[j] = static_cast<const char *>(in.p[2 * j]);
-      od[j] = static_cast<const char *>(in.p[2 * j + 1]);
+      ev[j] = ptr_of(a, 2 * j);
+      od[j] = ptr_of(a, 2 * j + 1);
     }
     rotate_left<B>(ev, l);
     rotate_left<B>(od, l);
@@ -196,14 +201,10 @@ __device__ __forceinline__ h8 reduce_operands(const h8 (&x)[N]) {
   }
 }
 
-// One launch covers bytes [seg_off, seg_off + seg_bytes) of every chunk;
-// chunk_pitch is the full chunk length (the distance between chunk starts).
+// One launch covers seg_bytes of every chunk (DirectArgs).
 template <int N, int ORDER, int DT, int UNROLL, int LD_AUX, int ST_AUX>
-__global__ __launch_bounds__(1024) void k_direct_allreduce(PtrTable in, PtrTable out,
-                                                           size_t chunk_pitch, size_t seg_off,
-                                                           uint32_t seg_bytes,
-                                                           uint32_t blocks_per_rank, uint32_t deal_log2,
-                                                           uint32_t row, uint32_t lines) {
+__global__ __launch_bounds__(1024) void k_direct_allreduce(DirectArgs<N> a) {
+  const uint32_t deal_log2 = a.deal_log2(), row = a.row();
   // 2^deal_log2 chunks ("deal") are worked on at a time: row y of the grid, deal *
   // blocks_per_rank work-groups, belongs to owners y * deal ... y * deal + deal - 1,
   // round robin (rows are dispatched one after the other).  deal = N: work-group b
@@ -212,24 +213,22 @@ __global__ __launch_bounds__(1024) void k_direct_allreduce(PtrTable in, PtrTable
   const uint32_t deal = 1u << deal_log2;
   const int owner = owner_of_group<N, ORDER>((int)(blockIdx.y * deal + (blockIdx.x & (deal - 1))));
   const uint32_t jblock = blockIdx.x >> deal_log2;
-  size_t base = (size_t)chunk_of_owner<N, ORDER>(owner) * chunk_pitch + seg_off;
-  const TileStart ts = tile_start(lines, base);
+  size_t base = (size_t)chunk_of_owner<N, ORDER>(owner) * a.pitch();
+  const TileStart ts = tile_start(a.line(), a.head_mask(), base);
   base += ts.head;
-  seg_bytes -= ts.head;
+  const uint32_t seg_bytes = a.seg_bytes - ts.head;
 
   const char *op[N];
-  select_operands<N, ORDER>(in, owner, op);
+  select_operands<N, ORDER>(a, owner, op);
   __amdgpu_buffer_rsrc_t src[N], dst[N];
 #pragma unroll
   for (int k = 0; k < N; ++k) {
     src[k] = make_rsrc(op[k] + base, seg_bytes);
-    dst[k] = make_rsrc(static_cast<char *>(out.p[k]) + base, seg_bytes);
+    dst[k] = make_rsrc(ptr_of(a, N + k) + base, seg_bytes);
   }
   const uint32_t lane = threadIdx.x * 16u - ts.skew;
-  // `row` = bytes one unroll step spans, blockDim.x * 16: an argument, so that it
-  // arrives with the others instead of through a separate load of the launch's dimensions
   const uint32_t tile = row * UNROLL;
-  const uint32_t stride = tile * blocks_per_rank;
+  const uint32_t stride = tile * a.blocks_per_rank;
   // Every work-group has a first tile (the host launches at most one work-group per tile),
   // so the loop tests at its end and nothing separates the kernel's argument loads.
   uint32_t t = jblock * tile;
@@ -268,7 +267,7 @@ __global__ __launch_bounds__(1024) void k_direct_allreduce(PtrTable in, PtrTable
       for (int k = 0; k < N; ++k) x[k] = ld_low<LD_AUX>(make_rsrc(op[k] + base - 8, 8));
       const h8 acc = reduce_operands<N, ORDER, DT>(x);
 #pragma unroll
-      for (int k = 0; k < N; ++k) st_low<ST_AUX>(make_rsrc(static_cast<char *>(out.p[k]) + base - 8, 8), acc);
+      for (int k = 0; k < N; ++k) st_low<ST_AUX>(make_rsrc(ptr_of(a, N + k) + base - 8, 8), acc);
     }
   }
 }
@@ -276,16 +275,11 @@ __global__ __launch_bounds__(1024) void k_direct_allreduce(PtrTable in, PtrTable
 // All-gather: the groups of rank p read p's slice once and store it into slot p
 // of every rank's output (allgather.hpp:79-100 collapsed to one hop).
 template <int N, int UNROLL, int LD_AUX, int ST_AUX>
-__global__ __launch_bounds__(1024) void k_direct_allgather(PtrTable in, PtrTable out,
-                                                           size_t slice_pitch, size_t seg_off,
-                                                           uint32_t seg_bytes,
-                                                           uint32_t blocks_per_rank, uint32_t deal_log2,
-                                                           uint32_t row, uint32_t lines) {
+__global__ __launch_bounds__(1024) void k_direct_allgather(DirectArgs<N> a) {
   // 2^deal_log2 source slices are worked on at a time (see k_direct_allreduce): deal = N
   // gives work-group b to source b % N throughout, deal = 1 lets all work-groups sweep
   // one source's slice after the other.
-  const uint32_t run_log2 = deal_log2 >> 8;   // second byte: tiles per XCD run (see below)
-  deal_log2 &= 0xff;
+  const uint32_t run_log2 = a.run_log2(), deal_log2 = a.deal_log2(), row = a.row(), seg_bytes = a.seg_bytes;
   const uint32_t deal = 1u << deal_log2;
   const int p = (int)(blockIdx.y * deal + (blockIdx.x & (deal - 1)));
   uint32_t jblock = blockIdx.x >> deal_log2;
@@ -294,19 +288,20 @@ __global__ __launch_bounds__(1024) void k_direct_allgather(PtrTable in, PtrTable
   // consecutive tiles (the ragged last group of a slice stays as it is).
   if (run_log2) {
     const uint32_t group = 8u << run_log2, first = jblock & ~(group - 1), r = jblock & (group - 1);
-    if (first + group <= blocks_per_rank) jblock = first + ((r & 7u) << run_log2) + (r >> 3);
+    if (first + group <= a.blocks_per_rank) jblock = first + ((r & 7u) << run_log2) + (r >> 3);
   }
   // the source pointer picked from the whole table with scalar selects: a look-up
   // by p would be a second, dependent scalar load at the head of every work-group
   uintptr_t picked = 0;
 #pragma unroll
-  for (int k = 0; k < N; ++k) picked |= p == k ? reinterpret_cast<uintptr_t>(in.p[k]) : (uintptr_t)0;
-  const char *src_ptr = reinterpret_cast<const char *>(picked) + seg_off;
+  for (int k = 0; k < N; ++k) picked |= p == k ? reinterpret_cast<uintptr_t>(ptr_of(a, k)) : (uintptr_t)0;
+  const char *src_ptr = reinterpret_cast<const char *>(picked);
+  const size_t slot = (size_t)p * a.pitch();
   const __amdgpu_buffer_rsrc_t src = make_rsrc(src_ptr, seg_bytes);
   __amdgpu_buffer_rsrc_t dst[N];
 #pragma unroll
   for (int r = 0; r < N; ++r) {
-    char *d = static_cast<char *>(out.p[r]) + (size_t)p * slice_pitch + seg_off;
+    char *d = ptr_of(a, N + r) + slot;
     // The reference skips the store when a rank's input already is its own
     // output slot (sequential_transmit.hpp:496-497).  Here such a destination gets
     // a resource of length zero, so the hardware drops its stores: no branch sits
@@ -315,10 +310,10 @@ __global__ __launch_bounds__(1024) void k_direct_allgather(PtrTable in, PtrTable
     dst[r] = make_rsrc(d, d == src_ptr ? 0u : seg_bytes);
   }
   // every address is a multiple of the 16-byte messages, so no vector straddles a start
-  const TileStart ts = tile_start(lines, (size_t)p * slice_pitch + seg_off);
+  const TileStart ts = tile_start(a.line(), 0, slot);
   const uint32_t lane = threadIdx.x * 16u - ts.skew;
   const uint32_t tile = row * UNROLL;
-  const uint32_t stride = tile * blocks_per_rank;
+  const uint32_t stride = tile * a.blocks_per_rank;
   uint32_t t = jblock * tile;   // every work-group has a first tile, as in k_direct_allreduce
   do {
     h8 x[UNROLL];
@@ -455,20 +450,16 @@ hipError_t launch_kernel(const void *fn, dim3 grid, dim3 block, void **kargs, ui
   return e;
 }
 
-template <typename... P>
-static hipError_t launch(void (*kernel)(P...), dim3 grid, dim3 block, uint32_t lds, hipStream_t s, hipEvent_t ev0,
-                         hipEvent_t ev1, P... args) {
-  void *kargs[] = {&args...};
+template <typename P>
+static hipError_t launch(void (*kernel)(P), dim3 grid, dim3 block, uint32_t lds, hipStream_t s, hipEvent_t ev0,
+                         hipEvent_t ev1, P &args) {
+  void *kargs[] = {&args};
   return launch_kernel(reinterpret_cast<const void *>(kernel), grid, block, kargs, lds, s, ev0, ev1);
 }
 
 // Bytes the tiles of a chunk may have to start early to lie on the outputs' lines (tile_start).
 static size_t skew_of(const PtrTable &out, size_t pitch, size_t seg_off) {
   return (((uintptr_t)out.p[0] | pitch | seg_off) & 127u) ? 120 : 0;
-}
-
-uint32_t lines_of(const PtrTable &out, uint32_t head_mask) {
-  return ((uint32_t)(uintptr_t)out.p[0] & 127u) | head_mask << 8;
 }
 
 // 8 where a chunk that starts in the middle of 16 bytes does so in every buffer, else 0.
@@ -482,25 +473,25 @@ uint32_t head_mask_of(int nranks, const PtrTable &in, const PtrTable &out) {
 template <int N, int ORDER, int DT, int UNROLL>
 static hipError_t launch_ar_segments(hipStream_t s, const DeviceInfo &dev, const Tuning &t,
                                      const PtrTable &in, const PtrTable &out, size_t chunk_bytes) {
-  const uint32_t row = (uint32_t)t.block * 16u;   // bytes one unroll step of a work-group spans
-  const size_t tile = (size_t)row * UNROLL;
+  const size_t tile = (size_t)t.block * 16 * UNROLL;
   const size_t seg_max = segment_of(t);
   const uint32_t lds = lds_cap_bytes(dev, t.wgs_per_cu);
   // chunks dealt at a time: a divisor of N, N itself unless the launch says otherwise
   const uint32_t deal = (t.deal > 0 && t.deal <= N && N % t.deal == 0) ? (uint32_t)t.deal : (uint32_t)N;
-  const uint32_t lines = lines_of(out, ORDER == ORDER_COPY ? 0u : head_mask_of(N, in, out));
+  const uint32_t head_mask = ORDER == ORDER_COPY ? 0u : head_mask_of(N, in, out);
   const uint32_t deal_log2 = (uint32_t)__builtin_ctz(deal);   // N is a power of two, so are its divisors
   for (size_t off = 0; off < chunk_bytes; off += seg_max) {
     const size_t seg = chunk_bytes - off < seg_max ? chunk_bytes - off : seg_max;
     const uint32_t bpr = blocks_per_rank_for(dev, t, N, seg + skew_of(out, chunk_bytes, off), tile);
     const dim3 grid(bpr * deal, N / deal), block(t.block);
+    DirectArgs<N> args = direct_args<N>(in.p, out.p, chunk_bytes, off, seg, t.block, bpr, deal_log2, 0, head_mask);
     // kernel-attached profiling events: start on the first segment, stop on the last
     hipEvent_t ev0 = off == 0 ? tl_kernel_events.start : nullptr;
     hipEvent_t ev1 = off + seg >= chunk_bytes ? tl_kernel_events.stop : nullptr;
     hipError_t e = with_policy(t, [&](auto ld_aux, auto st_aux) {
       auto kernel = k_direct_allreduce<N, ORDER, DT, UNROLL, decltype(ld_aux)::value, decltype(st_aux)::value>;
       if (hipError_t a = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), dev, lds); a != hipSuccess) return a;
-      return launch(kernel, grid, block, lds, s, ev0, ev1, in, out, chunk_bytes, off, (uint32_t)seg, bpr, deal_log2, row, lines);
+      return launch(kernel, grid, block, lds, s, ev0, ev1, args);
     });
     if (e != hipSuccess) return e;
   }
@@ -558,24 +549,24 @@ hipError_t launch_direct_allreduce(hipStream_t s, const DeviceInfo &dev, const T
 template <int N, int UNROLL>
 static hipError_t launch_ag_segments(hipStream_t s, const DeviceInfo &dev, const Tuning &t,
                                      const PtrTable &in, const PtrTable &out, size_t slice_bytes) {
-  const uint32_t row = (uint32_t)t.block * 16u;   // bytes one unroll step of a work-group spans
-  const size_t tile = (size_t)row * UNROLL;
+  const size_t tile = (size_t)t.block * 16 * UNROLL;
   const size_t seg_max = segment_of(t);
   const uint32_t lds = lds_cap_bytes(dev, t.wgs_per_cu);
   const uint32_t deal = (t.deal > 0 && t.deal <= N && N % t.deal == 0) ? (uint32_t)t.deal : (uint32_t)N;
-  uint32_t deal_log2 = (uint32_t)__builtin_ctz(deal);
+  const uint32_t deal_log2 = (uint32_t)__builtin_ctz(deal);
   // tiles per XCD run: only where a row of the grid is one source's slice and a one-trip launch
-  if (t.run > 1 && deal == 1 && t.oneshot) deal_log2 |= (uint32_t)__builtin_ctz((unsigned)t.run) << 8;
+  const uint32_t run_log2 = t.run > 1 && deal == 1 && t.oneshot ? (uint32_t)__builtin_ctz((unsigned)t.run) : 0u;
   for (size_t off = 0; off < slice_bytes; off += seg_max) {
     const size_t seg = slice_bytes - off < seg_max ? slice_bytes - off : seg_max;
     const uint32_t bpr = blocks_per_rank_for(dev, t, N, seg + skew_of(out, slice_bytes, off), tile);
     const dim3 grid(bpr * deal, N / deal), block(t.block);
+    DirectArgs<N> args = direct_args<N>(in.p, out.p, slice_bytes, off, seg, t.block, bpr, deal_log2, run_log2, 0);
     hipEvent_t ev0 = off == 0 ? tl_kernel_events.start : nullptr;
     hipEvent_t ev1 = off + seg >= slice_bytes ? tl_kernel_events.stop : nullptr;
     hipError_t e = with_policy(t, [&](auto ld_aux, auto st_aux) {
       auto kernel = k_direct_allgather<N, UNROLL, decltype(ld_aux)::value, decltype(st_aux)::value>;
       if (hipError_t a = allow_dynamic_lds(reinterpret_cast<const void *>(kernel), dev, lds); a != hipSuccess) return a;
-      return launch(kernel, grid, block, lds, s, ev0, ev1, in, out, slice_bytes, off, (uint32_t)seg, bpr, deal_log2, row, lines_of(out, 0));
+      return launch(kernel, grid, block, lds, s, ev0, ev1, args);
     });
     if (e != hipSuccess) return e;
   }

@@ -6,12 +6,13 @@
 #include <stdint.h>
 
 #include "vrank_allreduce.h"
+#include "vr_launch_args.h"
 #include "vr_wire_layout.h"
 
 namespace vr {
 
-// Device pointers of all virtual ranks, passed to kernels by value (like the
-// reference functor's by-value pointer tables, parallel_transmit.hpp:134-145).
+// Device pointers of all virtual ranks (the reference functor's by-value pointer tables,
+// parallel_transmit.hpp:134-145).
 struct PtrTable {
   void *p[VR_MAX_RANKS];
 };
@@ -88,8 +89,6 @@ hipError_t launch_copy(hipStream_t s, const DeviceInfo &dev, const Tuning &t, vo
 
 // 8 where a chunk that starts in the middle of 16 bytes does so in every buffer, else 0.
 uint32_t head_mask_of(int nranks, const PtrTable &in, const PtrTable &out);
-// Place of the first output in its 128-byte line, and head_mask in the second byte.
-uint32_t lines_of(const PtrTable &out, uint32_t head_mask);
 // Residency cap of a launch: bytes of dynamic LDS (never touched) with which at most `wgs`
 // work-groups share a compute unit; 0 = no cap.  And the allowance a kernel needs before
 // it may ask for more than 48 KiB.

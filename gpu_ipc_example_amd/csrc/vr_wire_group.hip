@@ -42,21 +42,20 @@ typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kStreamLoad = 2;        // nt
 constexpr int kStreamStore = 2 | 16;  // nt sc1
 
-// One launch covers bytes [seg_off, seg_off + seg_bytes) of every chunk.
-struct Args {
-  PtrTable in, out;
-  size_t pitch;           // bytes per rank-chunk (all-gather: of one slice)
-  size_t seg_off;
-  uint32_t seg_bytes;
-  uint32_t lines;         // see lines_of
-  uint32_t spin_limit;
-  uint32_t *status;       // non-zero once any poll gave up
-};
-
 struct Poll {
   uint32_t limit;
-  uint32_t *status;
+  __attribute__((address_space(1))) uint32_t *status;   // (device memory) non-zero once any poll gave up
   bool dead;
+  // Before the first wait: the limit and the time-out word out of the arguments, not sooner than
+  // here (ahead of a wave's first load, where the compiler likes to put it, it delays the load).
+  template <int N>
+  __device__ __forceinline__ void arm(const GroupArgs<N> &a) {
+    uint32_t rest = a.rest;
+    asm volatile("" : "+s"(rest));
+    limit = a.spin_limit(rest);
+    status = reinterpret_cast<__attribute__((address_space(1))) uint32_t *>(a.status_address(rest, a.status_lo));
+    dead = false;
+  }
   // Waits until `ready` holds in every lane.
   template <typename F>
   __device__ __forceinline__ void until(F &&ready) {
@@ -88,9 +87,9 @@ struct Msg {
 enum Starts : int { ON_LINES, ON_VECTORS, ON_HALVES };
 template <Starts S>
 struct Span : wl::Span {};
-template <Starts S, int U>
-static __device__ __forceinline__ Span<S> span_of(const Args &a, uint32_t chunk, uint32_t lane) {
-  return {wl::wire_span(S == ON_LINES, chunk * a.pitch + a.seg_off, a.seg_bytes, a.lines,
+template <Starts S, int U, int N>
+static __device__ __forceinline__ Span<S> span_of(const GroupArgs<N> &a, uint32_t chunk, uint32_t lane) {
+  return {wl::wire_span(S == ON_LINES, chunk * a.pitch(), S == ON_LINES ? a.seg : a.seg & 0x7fffffffu, S == ON_LINES ? 0 : a.lines(),
                         blockIdx.x * (1024u * U) + lane * 16u, blockIdx.x == 0)};
 }
 template <Starts S>
@@ -186,12 +185,12 @@ struct Sinks {
   extern __shared__ u32x4 lds[];                                                              \
   const uint32_t lane = threadIdx.x & 63u;                                                    \
   const int r = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));                      \
-  const char *const src = static_cast<const char *>(a.in.p[r]);                               \
-  char *const dst = static_cast<char *>(a.out.p[r]);                                          \
+  const char *const src = reinterpret_cast<const char *>(a.rank[r].in());                      \
+  char *const dst = reinterpret_cast<char *>(a.rank[r].out());                                 \
   /* every argument arrives behind one wait */                                                \
-  asm volatile("" ::"s"(src), "s"(dst), "s"(a.pitch), "s"(a.seg_off), "s"(a.seg_bytes), "s"(a.lines), \
-               "s"(a.spin_limit));                                                            \
-  Poll poll{a.spin_limit, a.status, false}
+  asm volatile("" ::"s"(src), "s"(dst), "s"(a.pitch_lo), "s"(a.seg), "s"(a.status_lo), "s"(a.rest), \
+               "s"(S == ON_LINES ? 0 : a.rank[0].out_lo));                                    \
+  Poll poll
 
 // ---- ParallelTransmit (parallel_transmit.hpp:63-131) -----------------------------------
 // Row y of the grid sweeps chunk y; the wave of rank y owns the column's reduction.
@@ -200,13 +199,14 @@ template <int N, int U>
 using ParallelSinks = Sinks<U, N, 2 * N>;
 
 template <int N, int DT, int U, Starts S, int LD, int ST>
-__global__ __launch_bounds__(64 * N) void k_group_parallel(Args a) {
+__global__ __launch_bounds__(64 * N) void k_group_parallel(GroupArgs<N> a) {
   VR_GROUP_PROLOGUE;
   const ParallelSinks<N, U> sk(lds, lane);
   const int y = (int)blockIdx.y;
   const auto at = span_of<S, U>(a, y, lane);
   Msg<U> v = load<U, LD>(src, at);
   sk.ready();
+  poll.arm(a);
   if (r != y) {
     sk.put(r, v);
     sk.publish();
@@ -235,13 +235,14 @@ template <int N, int U>
 using SequentialSinks = Sinks<U, N * N, 2 * N * N>;
 
 template <int N, int DT, int U, Starts S, int LD, int ST>
-__global__ __launch_bounds__(64 * N) void k_group_sequential(Args a) {
+__global__ __launch_bounds__(64 * N) void k_group_sequential(GroupArgs<N> a) {
   VR_GROUP_PROLOGUE;
   const SequentialSinks<N, U> sk(lds, lane);
   Msg<U> x[N];                                             // x[i]: chunk of rank r + i
 #pragma unroll
   for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<S, U>(a, (r + i) % N, lane));
   sk.ready();
+  poll.arm(a);
 #pragma unroll
   for (int i = 1; i < N; ++i) sk.put((r + i) % N * N + r, x[i]);
   sk.publish();
@@ -306,7 +307,7 @@ struct Ring {
 };
 
 template <int N, int DT, int U, Starts S, int LD, int ST>
-__global__ __launch_bounds__(64 * N) void k_group_ring(Args a) {
+__global__ __launch_bounds__(64 * N) void k_group_ring(GroupArgs<N> a) {
   VR_GROUP_PROLOGUE;
   const RingSinks<N, U> sk(lds, lane);
   Msg<U> x[N];                                             // x[i]: chunk of rank r - i
@@ -314,6 +315,7 @@ __global__ __launch_bounds__(64 * N) void k_group_ring(Args a) {
   for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<S, U>(a, (r + N - i) % N, lane));
   const Ring<N, U> ring{sk, poll, r, (r + 1) % N};
   sk.ready();
+  poll.arm(a);
   ring.send(0, x[0]);
 #pragma unroll
   for (int i = 1; i < N; ++i) {                            // reduce and forward; the last add starts the gather ring
@@ -330,15 +332,16 @@ __global__ __launch_bounds__(64 * N) void k_group_ring(Args a) {
 }
 
 template <int N, int DT, int U, Starts S, int LD, int ST>
-__global__ __launch_bounds__(64 * N) void k_group_allgather(Args a) {
+__global__ __launch_bounds__(64 * N) void k_group_allgather(GroupArgs<N> a) {
   VR_GROUP_PROLOGUE;
   const RingSinks<N, U> sk(lds, lane);
   const auto own = span_of<S, U>(a, r, lane);
   // the input is one slice long: the same bytes of it as of the own slot
-  const char *slot0 = src - (size_t)r * a.pitch;
+  const char *slot0 = src - (size_t)r * a.pitch();
   Msg<U> v = load<U, LD>(slot0, own);
   const Ring<N, U> ring{sk, poll, r, (r + 1) % N};
   sk.ready();
+  poll.arm(a);
   ring.send(0, v);
   // the own slot needs no store when it is the input (sequential_transmit.hpp:496-497)
   if (slot0 != dst) store<U, ST>(dst, own, v);
@@ -358,7 +361,7 @@ template <int N, int U>
 using BisectSinks = Sinks<U, 2 * N, 4 * N>;
 
 template <int N, int DT, int U, Starts S, int LD, int ST>
-__global__ __launch_bounds__(64 * N) void k_group_bisect(Args a) {
+__global__ __launch_bounds__(64 * N) void k_group_bisect(GroupArgs<N> a) {
   constexpr int B = N / 2;
   VR_GROUP_PROLOGUE;
   const BisectSinks<N, U> sk(lds, lane);
@@ -368,6 +371,7 @@ __global__ __launch_bounds__(64 * N) void k_group_bisect(Args a) {
   const Msg<U> f = load<U, LD>(src, far);
   Msg<U> v = load<U, LD>(src, close);
   sk.ready();
+  poll.arm(a);
   sk.put(pair, f);                                         // scatterFar
   sk.publish();
   sk.raise(pair, 1);
@@ -464,23 +468,30 @@ hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow
   const uint32_t cap = lds_cap_bytes(dev, plan.wgs_per_cu);
   if (cap > lds) lds = cap;
   if (hipError_t e = allow_dynamic_lds(k.fn, dev, lds); e != hipSuccess) return e;
-  Args a;
-  a.in = in;
-  a.out = out;
-  a.pitch = chunk_bytes;
-  a.lines = lines_of(out, flow == WIRE_PARALLEL || flow == WIRE_BISECT || flow == WIRE_SIMPLE ? head_mask_of(nranks, in, out) : 0u);
-  a.spin_limit = spin_limit;
-  a.status = status;
-  void *kargs[] = {&a};
+  // (0 where every chunk starts on a line: those kernels take GroupArgs::seg as it is)
+  const uint32_t head_mask =
+      !lined && (flow == WIRE_PARALLEL || flow == WIRE_BISECT || flow == WIRE_SIMPLE) ? head_mask_of(nranks, in, out) : 0u;
   const size_t seg_max = plan.segment_bytes;
   for (size_t off = 0; off < chunk_bytes; off += seg_max) {
     const size_t seg = chunk_bytes - off < seg_max ? chunk_bytes - off : seg_max;
-    a.seg_off = off;
-    a.seg_bytes = (uint32_t)seg;
     const dim3 grid((uint32_t)((seg + (lined ? 0 : 120) + wire - 1) / wire), k.rows), block(64u * (uint32_t)nranks);
     hipEvent_t ev0 = off == 0 ? tl_kernel_events.start : nullptr;
     hipEvent_t ev1 = off + seg >= chunk_bytes ? tl_kernel_events.stop : nullptr;
-    const hipError_t e = launch_kernel(k.fn, grid, block, kargs, lds, s, ev0, ev1);
+    hipError_t e = hipErrorInvalidValue;
+    switch (nranks) {
+#define VR_CASE(NN)                                                                                            \
+  case NN: {                                                                                                   \
+    GroupArgs<NN> a = group_args<NN>(in.p, out.p, chunk_bytes, off, seg, head_mask, spin_limit, status);       \
+    void *kargs[] = {&a};                                                                                      \
+    e = launch_kernel(k.fn, grid, block, kargs, lds, s, ev0, ev1);                                             \
+    break;                                                                                                     \
+  }
+      VR_CASE(2)
+      VR_CASE(4)
+      VR_CASE(8)
+      VR_CASE(16)
+#undef VR_CASE
+    }
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -122,9 +122,10 @@ struct Span {
   // 8 x 4 MiB took 15.6 us for 14.8.)
   VR_HD uint32_t first_load() const { return half() ? 8u : off; }
 };
-// The chunk's bytes [base, base + seg_bytes) of each buffer; `lines` as lines_of forms it
-// (vr_direct.hip); `off` = the lane's place counted from the start of the first wire.  `lined` =
-// every chunk starts on a line.
+// The chunk's bytes [base, base + seg_bytes) of each buffer; `lines` = place of the first output
+// in its line and, in the second byte, 8 where a chunk that starts in the middle of 16 bytes does
+// so in every buffer, else 0; `off` = the lane's place counted from the start of the first wire.
+// `lined` = every chunk starts on a line.
 VR_HD Span wire_span(bool lined, size_t base, uint32_t seg_bytes, uint32_t lines, uint32_t off, bool first_wire) {
   if (lined) return Span{base, seg_bytes, off, false};
   const uint32_t addr = (lines & 0xffu) + (uint32_t)base, head = addr & (lines >> 8);

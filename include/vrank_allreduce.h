@@ -313,7 +313,8 @@ int vr_allgather_grid(vr_ctx *ctx, void *stream, int algo, int transport, const 
  * scratch has been zeroed again; sinks a caller handed to the rank-group launches
  * are the caller's to zero. */
 int vr_ctx_check(vr_ctx *ctx, void *stream);
-/* Poll budget of the wire transport's bounded spin (0 = library default). */
+/* Poll budget of the wire transport's bounded spin (0 = library default).  Launches that hold
+ * all ranks take it rounded up to 10 significant bits. */
 int vr_ctx_set_spin_limit(vr_ctx *ctx, uint64_t polls);
 
 /* Tuning knobs for the direct kernels (benchmark sweeps).  Unknown keys are

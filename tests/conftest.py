@@ -19,6 +19,7 @@ def pytest_configure(config):
              os.path.join(ROOT, "tests", "cpp", "test_host_api"),
              os.path.join(ROOT, "tests", "cpp", "test_graph"),
              os.path.join(ROOT, "tests", "cpp", "test_wire_layout"),
+             os.path.join(ROOT, "tests", "cpp", "test_launch_args"),
              os.path.join(ROOT, "tests", "cpp", "test_verify"),
              os.path.join(ROOT, "tests", "cpp", "test_launch_errors")]
     if not all(os.path.exists(p) for p in built):

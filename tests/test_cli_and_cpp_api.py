@@ -14,6 +14,7 @@ CLI = os.path.join(ROOT, "gpu_ipc_example_amd", "vr_main")
 CPP_TEST = os.path.join(ROOT, "tests", "cpp", "test_host_api")
 GRAPH_TEST = os.path.join(ROOT, "tests", "cpp", "test_graph")
 LAYOUT_TEST = os.path.join(ROOT, "tests", "cpp", "test_wire_layout")
+ARGS_TEST = os.path.join(ROOT, "tests", "cpp", "test_launch_args")
 VERIFY_TEST = os.path.join(ROOT, "tests", "cpp", "test_verify")
 LAUNCH_TEST = os.path.join(ROOT, "tests", "cpp", "test_launch_errors")
 
@@ -32,6 +33,12 @@ def test_wire_sinks_hold_every_slot_the_kernels_index():
     slot functions: each message slot and flag word lies inside the sink."""
     r = run([LAYOUT_TEST], timeout=120)
     assert r.returncode == 0 and " 0 failures" in r.stdout, r.stdout
+
+
+def test_packed_kernel_arguments_come_out_as_they_went_in():
+    """Addresses up to 48 bits, chunks beyond 4 GiB and every field's range ends; CPU only."""
+    r = run([ARGS_TEST], timeout=120)
+    assert r.returncode == 0 and "launch arguments ok" in r.stdout, r.stdout[-2000:]
 
 
 def test_host_side_checks_of_the_cpp_header():
