@@ -80,23 +80,27 @@ __device__ __forceinline__ void st_low(__amdgpu_buffer_rsrc_t r, h8 v) {
 }
 
 // Where the tiles of a chunk lie.  Chunks may start at any multiple of 8 bytes, but tiles
-// are laid on 128-byte lines of the outputs and vectors on 16 bytes: a tile that starts
-// inside a line makes two work-groups, on two XCDs, write parts of it.  (With 8 bytes per
-// lane and tiles counted from the chunk's start: bisect, 16 x 12 MB bfloat16 of odd length
-// 112.5 us, now 69.8; simple, 4 x 20 MB in place 26.0, now 23.8.)
+// are laid on kTilePlace bytes of the outputs and vectors on 16 bytes: a tile that starts
+// inside a 128-byte line makes two work-groups, on two XCDs, write parts of it, and one that
+// starts inside the 256 bytes that memory channels take in turn reaches one channel more.  (With
+// 8 bytes per lane and tiles counted from the chunk's start: bisect, 16 x 12 MB bfloat16 of odd
+// length 112.5 us, on lines 69.8; simple, 4 x 20 MB in place 26.0, 23.8.  On 128 / 256 / 512 / 1024
+// bytes: simple, 8 x 32 MiB less 64 bytes 85.0 / 85.3 / 85.6 / 83.5 us, 82.1 at 32 MiB; 4 x 40 MB
+// 51.8 / 51.8 / 51.6 / 51.2; bisect, 8 x 16 MiB less 64 in place 51.2 / 50.8 / 50.6 / 50.6.)
 //   head: bytes (0 or 8) of the chunk ahead of its first whole vector.  `head_mask` is 0 where
 //         the buffers disagree modulo 16: then a lane's 16 bytes are 8-byte aligned in some
 //         of them, which the hardware takes.
-//   skew: bytes of the first tile's line below the first vector; lanes there form offsets
+//   skew: bytes of the first tile below the first vector; lanes there form offsets
 //         below zero, which are beyond the buffer's length like those of the last tile.
+constexpr uint32_t kTilePlace = 1024;   // the smallest tile: one wave's vectors
 struct TileStart {
   uint32_t head, skew;
 };
-// `line`: place of the first output in its line; `base`: the chunk's start, from the outputs'.
-__device__ __forceinline__ TileStart tile_start(uint32_t line, uint32_t head_mask, size_t base) {
-  const uint32_t at = line + (uint32_t)base;
+// `place`: the first output's in kTilePlace bytes; `base`: the chunk's start, from the outputs'.
+__device__ __forceinline__ TileStart tile_start(uint32_t place, uint32_t head_mask, size_t base) {
+  const uint32_t at = place + (uint32_t)base;
   const uint32_t head = at & head_mask;
-  return {head, (at + head) & 112u};
+  return {head, (at + head) & (kTilePlace - 16u)};
 }
 
 // The chunk a protocol owner reduces.
@@ -214,7 +218,7 @@ __global__ __launch_bounds__(1024) void k_direct_allreduce(DirectArgs<N> a) {
   const int owner = owner_of_group<N, ORDER>((int)(blockIdx.y * deal + (blockIdx.x & (deal - 1))));
   const uint32_t jblock = blockIdx.x >> deal_log2;
   size_t base = (size_t)chunk_of_owner<N, ORDER>(owner) * a.pitch();
-  const TileStart ts = tile_start(a.line(), a.head_mask(), base);
+  const TileStart ts = tile_start(a.place(), a.head_mask(), base);
   base += ts.head;
   const uint32_t seg_bytes = a.seg_bytes - ts.head;
 
@@ -310,7 +314,7 @@ __global__ __launch_bounds__(1024) void k_direct_allgather(DirectArgs<N> a) {
     dst[r] = make_rsrc(d, d == src_ptr ? 0u : seg_bytes);
   }
   // every address is a multiple of the 16-byte messages, so no vector straddles a start
-  const TileStart ts = tile_start(a.line(), 0, slot);
+  const TileStart ts = tile_start(a.place(), 0, slot);
   const uint32_t lane = threadIdx.x * 16u - ts.skew;
   const uint32_t tile = row * UNROLL;
   const uint32_t stride = tile * a.blocks_per_rank;
@@ -457,9 +461,9 @@ static hipError_t launch(void (*kernel)(P), dim3 grid, dim3 block, uint32_t lds,
   return launch_kernel(reinterpret_cast<const void *>(kernel), grid, block, kargs, lds, s, ev0, ev1);
 }
 
-// Bytes the tiles of a chunk may have to start early to lie on the outputs' lines (tile_start).
+// Bytes the tiles of a chunk may have to start early to lie as they should (tile_start).
 static size_t skew_of(const PtrTable &out, size_t pitch, size_t seg_off) {
-  return (((uintptr_t)out.p[0] | pitch | seg_off) & 127u) ? 120 : 0;
+  return (((uintptr_t)out.p[0] | pitch | seg_off) & (kTilePlace - 1u)) ? kTilePlace - 8u : 0;
 }
 
 // 8 where a chunk that starts in the middle of 16 bytes does so in every buffer, else 0.

@@ -26,7 +26,7 @@ struct DirectArgs {
   uint32_t seg_bytes;         // bytes of every chunk the launch covers
   uint32_t blocks_per_rank;
   // bits 0-2 log2 of the chunks dealt at a time; 3-7 waves of a work-group; 8-14 place of the first
-  // output in its 128-byte line; 15 head mask / 8; 16-19 all-gather: log2 of the tiles per XCD run;
+  // output in its KiB, / 8; 15 head mask / 8; 16-19 all-gather: log2 of the tiles per XCD run;
   // 20-31 bits 32-43 of the pitch
   uint32_t shape;
 
@@ -35,7 +35,7 @@ struct DirectArgs {
   // bytes one unroll step of a work-group spans, 16 a lane (from the arguments, so that nothing
   // waits for a separate load of the launch's dimensions)
   VR_HD uint32_t row() const { return (shape >> 3 & 31u) << 10; }
-  VR_HD uint32_t line() const { return shape >> 8 & 127u; }
+  VR_HD uint32_t place() const { return shape >> 5 & 1016u; }
   VR_HD uint32_t head_mask() const { return shape >> 12 & 8u; }
   VR_HD uint32_t run_log2() const { return shape >> 16 & 15u; }
   VR_HD uint64_t pitch() const { return join48(shape >> 20, pitch_lo); }
@@ -57,7 +57,7 @@ DirectArgs<N> direct_args(void *const in[], void *const out[], size_t pitch, siz
   a.pitch_lo = (uint32_t)pitch;
   a.seg_bytes = (uint32_t)seg;
   a.blocks_per_rank = blocks_per_rank;
-  a.shape = deal_log2 | (uint32_t)block / 64u << 3 | (a.lo[N] & 127u) << 8 | (head_mask ? 1u : 0u) << 15 | run_log2 << 16 |
+  a.shape = deal_log2 | (uint32_t)block / 64u << 3 | (a.lo[N] >> 3 & 127u) << 8 | (head_mask ? 1u : 0u) << 15 | run_log2 << 16 |
             (uint32_t)((uint64_t)pitch >> 32) << 20;
   return a;
 }

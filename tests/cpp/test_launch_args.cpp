@@ -34,7 +34,7 @@ static void check(uint64_t in_base, uint64_t out_base, size_t pitch, size_t off,
       }
       EXPECT(a.pitch() == pitch && a.seg_bytes == seg && a.blocks_per_rank == 0xfedcba98u);
       EXPECT(a.deal_log2() == deal && a.row() == (uint32_t)block * 16u && a.run_log2() == run && a.head_mask() == head);
-      EXPECT(a.line() == (((uintptr_t)out[0] + off) & 127u));
+      EXPECT(a.place() == (((uintptr_t)out[0] + off) & 1023u));
     }
   for (uint64_t status : {(uint64_t)256, (uint64_t)0xffffffffff00, (uint64_t)0x7f1234567800}) {
     const GroupArgs<N> g = group_args<N>(in, out, pitch, off, seg, head, spin, (void *)(uintptr_t)status);

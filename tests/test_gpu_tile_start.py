@@ -1,4 +1,4 @@
-"""Tiles laid on the outputs' 128-byte lines: buffers that start anywhere on 8 bytes, chunks
+"""Tiles laid on KiBs (direct) and 128-byte lines of the outputs: buffers that start anywhere on 8 bytes, chunks
 that are any multiple of 8 bytes, buffers that disagree about their place in 16 bytes.  Bit for
 bit against the oracle, nothing written outside a buffer, inputs kept."""
 import numpy as np
@@ -11,13 +11,13 @@ from tests import vr_helpers as H
 pytestmark = pytest.mark.gpu
 
 
-def run(oracle, ctx, algo, n, offsets, out_offsets, transport, seed):
+def run(oracle, ctx, algo, n, offsets, out_offsets, transport, seed, slack=256):
     N = ctx.nranks
     ins = H.make_inputs(oracle, N, n, seed)
     want = H.expected(oracle, algo, ins)
     what = (algo, N, n, offsets, out_offsets, transport)
-    src = [DeviceBuffer(n * 2 + 256) for _ in range(N)]
-    dst = [DeviceBuffer(n * 2 + 256) for _ in range(N)] if out_offsets else src
+    src = [DeviceBuffer(n * 2 + slack) for _ in range(N)]
+    dst = [DeviceBuffer(n * 2 + slack) for _ in range(N)] if out_offsets else src
     for b in src + dst:
         b.fill(0xAB)
     for b, a, o in zip(src, ins, offsets):
@@ -26,7 +26,7 @@ def run(oracle, ctx, algo, n, offsets, out_offsets, transport, seed):
     ctx.allreduce(algo, [b.ptr + o for b, o in zip(src, offsets)], n, outs=outs, transport=transport)
     ctx.check()
     for r, (b, o) in enumerate(zip(dst, out_offsets or offsets)):
-        got = b.download(np.uint16, n + 128)
+        got = b.download(np.uint16, n + slack // 2)
         assert oracle.count_mismatch(got[o // 2:o // 2 + n], want) == 0, (what, r)
         assert (got[:o // 2] == 0xABAB).all() and (got[o // 2 + n:] == 0xABAB).all(), (what, r)
     if out_offsets:
@@ -51,6 +51,19 @@ def test_direct(oracle, nranks, algo):
             run(oracle, ctx, algo, n, [8 * (r % 3) for r in range(nranks)], [8 + 16 * (r % 2) for r in range(nranks)],
                 vr.TRANSPORT_DIRECT, 72_000 + chunk)
         ctx.set_tuning(**{key: -1 for key in kn})
+    ctx.close()
+
+
+@pytest.mark.parametrize("transport", [vr.TRANSPORT_DIRECT, vr.TRANSPORT_WIRE])
+@pytest.mark.parametrize("nranks,algo", [(2, "simple"), (8, "parallel"), (16, "bisect")])
+def test_places_within_a_kib(oracle, nranks, algo, transport):
+    """First tiles that hold 16 bytes of the chunk, or all but 16."""
+    ctx = vr.VirtualRanks(nranks)
+    for chunk in (8, 1024, 3 * 1024 + 520):
+        for off in (264, 1008, 1016):
+            n = nranks * chunk // 2
+            run(oracle, ctx, algo, n, [off] * nranks, None, transport, 76_000 + chunk, 2048)
+            run(oracle, ctx, algo, n, [8] * nranks, [off] * nranks, transport, 77_000 + chunk, 2048)
     ctx.close()
 
 
