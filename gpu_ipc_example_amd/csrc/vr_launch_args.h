@@ -77,12 +77,15 @@ struct GroupArgs {
                           // every chunk starts on a line: the kernels for that take the word as it is)
   uint32_t status_lo;     // address / 256 of the time-out word, lower 32 bits
   uint32_t rest;          // bits 0-7: upper ones of that address; 8-16: of the pitch; 17-26 and 27-31: spin
-                          // limit, 10 significant bits and how far they are shifted up
+                          // limit, 10 significant bits and how far they are shifted up; the all-gather,
+                          // which waits for no flag, has there what run_code forms
   VR_HD uint64_t pitch() const { return join48(rest >> 8 & 511u, pitch_lo); }
-  // place of the first output in its line, and the head mask in the second byte
-  VR_HD uint32_t lines() const { return (rank[0].out_lo & 127u) | seg >> 31 << 11; }
+  // place of the first output in its KiB, and the head mask from bit 8 on (wire_span)
+  VR_HD uint32_t lines() const { return (rank[0].out_lo & 1023u) | seg >> 31 << 11; }
   static VR_HD uint64_t status_address(uint32_t rest, uint32_t status_lo) { return join48(rest & 255u, status_lo) << 8; }
   static VR_HD uint32_t spin_limit(uint32_t rest) { return (rest >> 17 & 0x3ffu) << (rest >> 27); }
+  VR_HD uint32_t run_log2() const { return rest >> 17 & 7u; }
+  VR_HD uint32_t run_cols() const { return (rest >> 20) << (3 + run_log2()); }
 };
 static_assert(sizeof(GroupArgs<8>) <= kCheapArgBytes, "a launch's arguments cost the host more beyond");
 
@@ -94,6 +97,16 @@ inline uint32_t spin_code(uint32_t limit) {
   while (m > 0x3ffu) m = (m + 1) / 2, ++shift;
   if (m << shift > 0xffffffffull) --shift, m = 0x3ffu;   // 2^32 would not come out of the shift
   return (uint32_t)m << 17 | shift << 27;
+}
+
+// The all-gather's bits of GroupArgs::rest: log2 of the work-groups in a row on an XCD, at most 7,
+// and how many groups of 8 * run work-groups a row of `cols` holds (as many as 12 bits say; the
+// others stay in their order).
+inline uint32_t run_code(int run, uint32_t cols) {
+  uint32_t log2 = 0;
+  while (log2 < 7 && (2 << log2) <= run) ++log2;
+  const uint32_t groups = cols >> (3 + log2);
+  return log2 << 17 | (groups < 4095u ? groups : 4095u) << 20;
 }
 
 // The launch that covers [off, off + seg) of every chunk.  `status` is the start of an allocation,

@@ -3,30 +3,33 @@
 // The waves of one wire column talk to nobody but each other: one wave per rank,
 // N waves.  When a launch holds all N ranks those N waves are made ONE work-group,
 // so they share a compute unit and its LDS, and the sinks of the column's ranks
-// live there: message slots and flag words at work-group scope, no scratch in
-// device memory, no polling across the chip, no co-residency demand on the grid.
-// The stages stay the reference's: every wave loads its own rank's input only,
-// scatters messages into the owners' sinks, the owner polls the flags, adds in the
-// protocol's order and gathers the sum into its peers' sinks, and every wave stores
-// its own rank's output only (parallel_transmit.hpp:63-131, sequential_transmit.hpp:
-// 83-207, 429-516, simple_transmit.hpp:16-179, bisect_transmit.hpp:286-424).
+// live there: message slots at work-group scope, no scratch in device memory, no
+// polling across the chip, no co-residency demand on the grid.  Every wave loads its
+// own rank's input only and stores its own rank's output only; between them the messages
+// are scattered, added up in the protocol's order and gathered.
 // Launches that hold some of the ranks keep their sinks in memory (vr_wire.hip).
+//
+// Two forms.  The all-to-all protocols (and, without the sums, the all-gather) are two steps
+// at most that all waves of the column take together, so the work-group's barrier says that
+// the messages are there.  RingTransmit's hops wait for one neighbour each, which a flag
+// word per rank says.  Its polls are bounded as in vr_wire.hip: after `spin_limit`
+// unsuccessful polls (or once another wave has given up) a wave records a time-out in the
+// status word and runs to its end without waiting again.
 //
 // What bounds it: HBM, like the direct transport.  Messages through memory cost 2.75
 // times the algorithmic bytes at the L2 / fabric boundary, which carries about
 // 8 TB/s however much of it the memory-side cache serves; here only inputs and
-// outputs cross it.  ParallelTransmit, 8 ranks in place: 256 MiB per rank
-// 2196 -> 681 us (6.3 TB/s), 1 MiB per rank 14.5 -> 4.2 us (bfloat16 4.65);
-// RingTransmit, 4 x 8 MB: 39.4 -> 10.8 us; ring all-gather, 8 x 1 MB: 51.6 -> 12.2 us.
+// outputs cross it.  ParallelTransmit, 8 ranks in place: 256 MiB per rank 2196 us through memory,
+// 670 us (6.4 TB/s); RingTransmit, 4 x 8 MB: 39.4, 10.8 us; all-gather, 8 x 1 MB: 51.6, 11.6 us.
+// Small launches are bound by the chain from a wave's load to its store.  With flag words for
+// every message, the owner's N - 1 additions in one wave and a copy of the sum for each peer it was
+// longer: parallel, 8 x 1 MiB bfloat16 4.62 us, now 3.72, of 64 bytes less 5.51, now 3.93; 8 x 8 MiB less
+// 64 28.5, now 24.7; simple_pcie, 8 x 5 MB 16.6, now 12.9; small, 8 x 1.9 MB out of place 6.8, now 6.2.
 //
 // One wire per work-group and no loop: the hardware starts work-groups in index
 // order, so a launch sweeps the chunks front to back with all compute units close
 // together (as the direct transport's one-trip grids).  A wave's message is U x 16
 // bytes per lane; the host picks U and the cache policies (group_plan).
-//
-// Polls are bounded as there: after `spin_limit` unsuccessful polls (or once another
-// wave has given up) a wave records a time-out in the status word and runs to its
-// end without waiting again.
 
 #include "vr_internal.h"
 
@@ -81,16 +84,18 @@ struct Msg {
 };
 
 // Where a chunk lies in every rank's buffer (wl::wire_span), by what chunks are known to start
-// on.  ON_LINES: none of the arithmetic for other starts (the extra scalar instructions of eight
+// on.  GRAIN: what wires are laid on, 128-byte lines or, where a row of the grid sweeps one chunk,
+// KiBs (parallel, 8 x 8 MiB less 64 bytes 28.6 -> 27.1 us, bisect 8 x 16 MiB less 64 56.2 -> 54.7; ring and
+// all-gather, which have a wire more then, lose 1 %).  ON_LINES: none of the arithmetic for other starts (the extra scalar instructions of eight
 // waves per 8 KiB cost 7 % at 8 x 32 MiB).  ON_VECTORS: messages of 16 bytes, no vector straddles
 // a start.
 enum Starts : int { ON_LINES, ON_VECTORS, ON_HALVES };
 template <Starts S>
 struct Span : wl::Span {};
-template <Starts S, int U, int N>
-static __device__ __forceinline__ Span<S> span_of(const GroupArgs<N> &a, uint32_t chunk, uint32_t lane) {
+template <Starts S, int U, int GRAIN, int N>
+static __device__ __forceinline__ Span<S> span_of(const GroupArgs<N> &a, uint32_t chunk, uint32_t lane, uint32_t col = blockIdx.x) {
   return {wl::wire_span(S == ON_LINES, chunk * a.pitch(), S == ON_LINES ? a.seg : a.seg & 0x7fffffffu, S == ON_LINES ? 0 : a.lines(),
-                        blockIdx.x * (1024u * U) + lane * 16u, blockIdx.x == 0)};
+                        col * (1024u * U) + lane * 16u, col == 0, GRAIN)};
 }
 template <Starts S>
 static __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *base, const Span<S> &s) {
@@ -117,13 +122,19 @@ static __device__ __forceinline__ Msg<U> load(const void *base, const Span<S> &s
 template <int U, int ST, Starts S>
 static __device__ __forceinline__ void store(void *base, const Span<S> &s, const Msg<U> &m) {
   const __amdgpu_buffer_rsrc_t rs = rsrc(base, s);
+  // (a scalar branch: only a chunk's first wire has a vector that straddles its start)
+  if (S == ON_HALVES && s.straddles) {
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    if (S == ON_HALVES && u == 0 && s.half())
-      __builtin_amdgcn_raw_buffer_store_b64(u32x2{m.d[0].x, m.d[0].y}, rs, 8u, 0, ST);
-    else
-      __builtin_amdgcn_raw_buffer_store_b128(m.d[u], rs, vec_off(s, u), 0, ST);
+    for (int u = 0; u < U; ++u) {
+      if (u == 0 && s.off == 0)
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{m.d[0].x, m.d[0].y}, rs, 8u, 0, ST);
+      else
+        __builtin_amdgcn_raw_buffer_store_b128(m.d[u], rs, vec_off(s, u), 0, ST);
+    }
+    return;
   }
+#pragma unroll
+  for (int u = 0; u < U; ++u) __builtin_amdgcn_raw_buffer_store_b128(m.d[u], rs, vec_off(s, u), 0, ST);
 }
 // v = m + v, the received message on the left (rt64_128.hpp:947-957)
 template <int DT, int U>
@@ -144,12 +155,6 @@ struct Sinks {
     flags = reinterpret_cast<uint32_t *>(lds + SLOTS * U * 64);
     if (threadIdx.x < (uint32_t)FLAGS) flags[threadIdx.x] = 0;   // never more than the work-group has lanes
   }
-  // All waves' flag words are zero from here on.
-  static __device__ __forceinline__ void ready() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-  }
   __device__ __forceinline__ void put(int slot, const Msg<U> &m) const {
 #pragma unroll
     for (int u = 0; u < U; ++u) slots[(slot * U + u) * 64 + lane] = m.d[u];
@@ -168,17 +173,6 @@ struct Sinks {
   __device__ __forceinline__ uint32_t look(int flag) const {
     return __hip_atomic_load(flags + flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
-  // Raises / awaits, with one access by the first N lanes, the N flag words from `first`
-  // on except number `self`.
-  template <int N>
-  __device__ __forceinline__ void raise_others(int first, int self, int stride = 1) const {
-    if (lane < (uint32_t)N && (int)lane != self)
-      __hip_atomic_store(flags + first + (int)lane * stride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  }
-  template <int N>
-  __device__ __forceinline__ void await_others(Poll &poll, int first, int self, int stride = 1) const {
-    poll.until([&] { return lane >= (uint32_t)N || (int)lane == self || look(first + (int)lane * stride) != 0; });
-  }
 };
 
 #define VR_GROUP_PROLOGUE                                                                    \
@@ -189,80 +183,104 @@ struct Sinks {
   char *const dst = reinterpret_cast<char *>(a.rank[r].out());                                 \
   /* every argument arrives behind one wait */                                                \
   asm volatile("" ::"s"(src), "s"(dst), "s"(a.pitch_lo), "s"(a.seg), "s"(a.status_lo), "s"(a.rest), \
-               "s"(S == ON_LINES ? 0 : a.rank[0].out_lo));                                    \
-  Poll poll
+               "s"(S == ON_LINES ? 0 : a.rank[0].out_lo))
 
-// ---- ParallelTransmit (parallel_transmit.hpp:63-131) -----------------------------------
-// Row y of the grid sweeps chunk y; the wave of rank y owns the column's reduction.
-// Peer p's slot carries its message to the owner and then the owner's sum back.
-template <int N, int U>
-using ParallelSinks = Sinks<U, N, 2 * N>;
+// Messages written before are in LDS for every wave of the work-group after.
+static __device__ __forceinline__ void meet() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
-template <int N, int DT, int U, Starts S, int LD, int ST>
-__global__ __launch_bounds__(64 * N) void k_group_parallel(GroupArgs<N> a) {
+// ---- ParallelTransmit, SequentialTransmit, SimpleTransmit, BisectPTransmit (parallel_transmit.hpp:
+// 63-131, sequential_transmit.hpp:83-207, simple_transmit.hpp:16-179, bisect_transmit.hpp:286-424) ----
+// Row c of the grid sweeps chunk c.  Every wave scatters its rank's message; the owner's additions,
+// N - 1 of them in a row, are shared out: each wave adds up an N-th of the message, in the
+// protocol's order, into the first slot, which all waves gather from.
+template <int N, int ORDER>
+static __device__ __forceinline__ int operand_of(int r, int c) {   // rank r's place in chunk c's order
+  if constexpr (ORDER == ORDER_ROTATED) return (r - c) & (N - 1);  // rank c, c + 1, ...
+  // pairs l, l + 1, ...; in each the rank of the half's parity first, then its pair's message
+  constexpr int B = N / 2;
+  const int h = c / B, l = c & (B - 1);
+  return 2 * (((r >> 1) - l) & (B - 1)) + ((r & 1) ^ h);
+}
+
+template <int N, int ORDER, int DT, int U, Starts S, int LD, int ST>
+__global__ __launch_bounds__(64 * N) void k_group_exchange(GroupArgs<N> a) {
   VR_GROUP_PROLOGUE;
-  const ParallelSinks<N, U> sk(lds, lane);
-  const int y = (int)blockIdx.y;
-  const auto at = span_of<S, U>(a, y, lane);
+  // A wave's share of the sums: an N-th of the message, but no less than 4 bytes a lane; waves
+  // without one wait.  (Shared out among all waves, 8 or 16 of 64 lanes with work to do, the
+  // additions of 16 ranks bound the launch: bisect, 16 x 12 MB bfloat16 82 us, so 67.)
+  constexpr int kMsg = U * 1024, kShare = kMsg / N >= 256 ? kMsg / N : 256;   // bytes
+  constexpr int W = kShare >= 1024 ? 16 : kShare / 64;                         // bytes a lane adds up at once
+  typedef _Float16 V __attribute__((ext_vector_type(W / 2)));
+  const int c = (int)blockIdx.y;
+  const auto at = span_of<S, U, 1024>(a, c, lane);
   Msg<U> v = load<U, LD>(src, at);
-  sk.ready();
-  poll.arm(a);
-  if (r != y) {
-    sk.put(r, v);
-    sk.publish();
-    sk.raise(r, 1);
-    poll.until([&] { return sk.look(N + r) != 0; });
-    v = sk.get(r);
-  } else {
-    sk.template await_others<N>(poll, 0, r);
-    Msg<U> m[N - 1];
+  u32x4 *const own = lds + operand_of<N, ORDER>(r, c) * (U * 64) + lane;
 #pragma unroll
-    for (int i = 0; i < N - 1; ++i) m[i] = sk.get((r + i + 1) % N);
+  for (int u = 0; u < U; ++u) own[u * 64] = v.d[u];
+  meet();
+  if (kShare * N <= kMsg || r < kMsg / kShare) {
+    char *const share = reinterpret_cast<char *>(lds) + r * kShare + lane * W;
 #pragma unroll
-    for (int i = 0; i < N - 1; ++i) add<DT, U>(v, m[i]);     // peers in order rank+1, rank+2, ...
+    for (int i = 0; i < kShare; i += 64 * W) {
+      V x[N];
 #pragma unroll
-    for (int i = 0; i < N - 1; ++i) sk.put((r + i + 1) % N, v);
-    sk.publish();
-    sk.template raise_others<N>(N, r);
+      for (int k = 0; k < N; ++k) x[k] = *reinterpret_cast<const V *>(share + i + k * kMsg);
+      // the received message is the left operand (rt64_128.hpp:947-957)
+      V sum;
+      if constexpr (ORDER == ORDER_ROTATED) {
+        sum = x[0];
+#pragma unroll
+        for (int k = 1; k < N; ++k) sum = vadd<DT>(x[k], sum);
+      } else {
+        sum = vadd<DT>(x[1], x[0]);
+#pragma unroll
+        for (int k = 2; k < N; k += 2) sum = vadd<DT>(vadd<DT>(x[k + 1], x[k]), sum);
+      }
+      *reinterpret_cast<V *>(share + i) = sum;
+    }
   }
+  meet();
+#pragma unroll
+  for (int u = 0; u < U; ++u) v.d[u] = lds[u * 64 + lane];
   store<U, ST>(dst, at, v);
 }
 
-// ---- SequentialTransmit, SimpleTransmit (sequential_transmit.hpp:83-207, simple_transmit.hpp:16-179) ----
-// One wave does everything its rank owes a column, peer after peer.  The slot of the
-// pair (owner, peer) carries the peer's message to the owner and then the owner's sum back.
-template <int N, int U>
-using SequentialSinks = Sinks<U, N * N, 2 * N * N>;
-
-template <int N, int DT, int U, Starts S, int LD, int ST>
-__global__ __launch_bounds__(64 * N) void k_group_sequential(GroupArgs<N> a) {
+// ---- all-gather (sequential_transmit.hpp:429-516 without the sums, its hops one) --------------------
+// Row p of the grid sweeps rank p's slice: p's wave sends the message, every wave stores it.
+template <int N, int U, Starts S, int LD, int ST>
+__global__ __launch_bounds__(64 * N) void k_group_allgather(GroupArgs<N> a) {
   VR_GROUP_PROLOGUE;
-  const SequentialSinks<N, U> sk(lds, lane);
-  Msg<U> x[N];                                             // x[i]: chunk of rank r + i
+  const int p = (int)blockIdx.y;
+  // Consecutive work-groups run on consecutive XCDs, so XCD k gets every eighth KiB.  With runs, the
+  // work-groups of each group of 8 * run are permuted so that it gets `run` KiB in a row (the
+  // ragged last group of a slice stays as it is).
+  uint32_t col = blockIdx.x;
+  const uint32_t run_log2 = a.run_log2(), group = 8u << run_log2, first = col & ~(group - 1u);
+  if (run_log2 && first + group <= a.run_cols()) {
+    const uint32_t k = col & (group - 1u);
+    col = first + ((k & 7u) << run_log2) + (k >> 3);
+  }
+  const auto at = span_of<S, U, 1024>(a, p, lane, col);
+  // the input is one slice long: the same bytes of it as of the own slot
+  const char *slot0 = src - (size_t)r * a.pitch();
+  Msg<U> v;
+  if (r == p) {
+    v = load<U, LD>(slot0, at);
 #pragma unroll
-  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<S, U>(a, (r + i) % N, lane));
-  sk.ready();
-  poll.arm(a);
+    for (int u = 0; u < U; ++u) lds[u * 64 + lane] = v.d[u];
+  }
+  meet();
+  if (r != p) {
 #pragma unroll
-  for (int i = 1; i < N; ++i) sk.put((r + i) % N * N + r, x[i]);
-  sk.publish();
-  sk.template raise_others<N>(r, r, N);                    // flag owner * N + r
-  Msg<U> v = x[0];
-  sk.template await_others<N>(poll, r * N, r);
-#pragma unroll
-  for (int i = 1; i < N; ++i) x[i] = sk.get(r * N + (r + i) % N);
-#pragma unroll
-  for (int i = 1; i < N; ++i) add<DT, U>(v, x[i]);         // peers in order rank+1, rank+2, ...
-#pragma unroll
-  for (int i = 1; i < N; ++i) sk.put(r * N + (r + i) % N, v);
-  sk.publish();
-  sk.template raise_others<N>(N * N + r * N, r);           // flag owner r, peer
-  store<U, ST>(dst, span_of<S, U>(a, r, lane), v);
-  sk.template await_others<N>(poll, N * N + r, r, N);
-#pragma unroll
-  for (int i = 1; i < N; ++i) x[i] = sk.get((r + i) % N * N + r);
-#pragma unroll
-  for (int i = 1; i < N; ++i) store<U, ST>(dst, span_of<S, U>(a, (r + i) % N, lane), x[i]);
+    for (int u = 0; u < U; ++u) v.d[u] = lds[u * 64 + lane];
+  } else if (slot0 == dst) {
+    return;   // the own slot needs no store when it is the input (sequential_transmit.hpp:496-497)
+  }
+  store<U, ST>(dst, at, v);
 }
 
 // ---- RingTransmit (sequential_transmit.hpp:429-516) --------------------------------------
@@ -309,12 +327,13 @@ struct Ring {
 template <int N, int DT, int U, Starts S, int LD, int ST>
 __global__ __launch_bounds__(64 * N) void k_group_ring(GroupArgs<N> a) {
   VR_GROUP_PROLOGUE;
+  Poll poll;
   const RingSinks<N, U> sk(lds, lane);
   Msg<U> x[N];                                             // x[i]: chunk of rank r - i
 #pragma unroll
-  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<S, U>(a, (r + N - i) % N, lane));
+  for (int i = 0; i < N; ++i) x[i] = load<U, LD>(src, span_of<S, U, 128>(a, (r + N - i) % N, lane));
   const Ring<N, U> ring{sk, poll, r, (r + 1) % N};
-  sk.ready();
+  meet();   // all waves' flag words are zero from here on
   poll.arm(a);
   ring.send(0, x[0]);
 #pragma unroll
@@ -322,85 +341,13 @@ __global__ __launch_bounds__(64 * N) void k_group_ring(GroupArgs<N> a) {
     add<DT, U>(x[i], ring.recv(i - 1));
     ring.send(i, x[i]);
   }
-  store<U, ST>(dst, span_of<S, U>(a, (r + 1) % N, lane), x[N - 1]);
+  store<U, ST>(dst, span_of<S, U, 128>(a, (r + 1) % N, lane), x[N - 1]);
 #pragma unroll
   for (int i = 1; i < N; ++i) {                            // write back, forward except on the last hop
     const Msg<U> v = ring.recv(N - 2 + i);
     if (i < N - 1) ring.send(N - 1 + i, v);
-    store<U, ST>(dst, span_of<S, U>(a, (r + 1 + N - i) % N, lane), v);
+    store<U, ST>(dst, span_of<S, U, 128>(a, (r + 1 + N - i) % N, lane), v);
   }
-}
-
-template <int N, int DT, int U, Starts S, int LD, int ST>
-__global__ __launch_bounds__(64 * N) void k_group_allgather(GroupArgs<N> a) {
-  VR_GROUP_PROLOGUE;
-  const RingSinks<N, U> sk(lds, lane);
-  const auto own = span_of<S, U>(a, r, lane);
-  // the input is one slice long: the same bytes of it as of the own slot
-  const char *slot0 = src - (size_t)r * a.pitch();
-  Msg<U> v = load<U, LD>(slot0, own);
-  const Ring<N, U> ring{sk, poll, r, (r + 1) % N};
-  sk.ready();
-  poll.arm(a);
-  ring.send(0, v);
-  // the own slot needs no store when it is the input (sequential_transmit.hpp:496-497)
-  if (slot0 != dst) store<U, ST>(dst, own, v);
-#pragma unroll
-  for (int i = 1; i < N; ++i) {
-    v = ring.recv(i - 1);
-    if (i < N - 1) ring.send(i, v);
-    store<U, ST>(dst, span_of<S, U>(a, (r + N - i) % N, lane), v);
-  }
-}
-
-// ---- BisectPTransmit (bisect_transmit.hpp:286-424) -----------------------------------------
-// Row y of the grid sweeps chunk y of both halves.  Slot r (far): the pair's message to
-// rank r, then r's sum back to the pair.  Slot N + r (close): r's pair sum to the owner,
-// then the owner's sum back.
-template <int N, int U>
-using BisectSinks = Sinks<U, 2 * N, 4 * N>;
-
-template <int N, int DT, int U, Starts S, int LD, int ST>
-__global__ __launch_bounds__(64 * N) void k_group_bisect(GroupArgs<N> a) {
-  constexpr int B = N / 2;
-  VR_GROUP_PROLOGUE;
-  const BisectSinks<N, U> sk(lds, lane);
-  const int y = (int)blockIdx.y, h = r & 1, l = r >> 1, pair = r ^ 1;
-  const auto close = span_of<S, U>(a, h * B + y, lane),
-             far = span_of<S, U>(a, (1 - h) * B + y, lane);
-  const Msg<U> f = load<U, LD>(src, far);
-  Msg<U> v = load<U, LD>(src, close);
-  sk.ready();
-  poll.arm(a);
-  sk.put(pair, f);                                         // scatterFar
-  sk.publish();
-  sk.raise(pair, 1);
-  poll.until([&] { return sk.look(r) != 0; });
-  add<DT, U>(v, sk.get(r));                                // pair sum
-  if (y != l) {
-    sk.put(N + r, v);                                      // scatterClose to the owner, rank 2y + h
-    sk.publish();
-    sk.raise(N + r, 1);
-    poll.until([&] { return sk.look(2 * N + r) != 0; });
-    v = sk.get(N + r);
-  } else {
-    sk.template await_others<B>(poll, N + h, l, 2);
-    Msg<U> m[B - 1];
-#pragma unroll
-    for (int i = 0; i < B - 1; ++i) m[i] = sk.get(N + (r + 2 * i + 2) % N);
-#pragma unroll
-    for (int i = 0; i < B - 1; ++i) add<DT, U>(v, m[i]);   // pair sums in order l+1, l+2, ...
-#pragma unroll
-    for (int i = 0; i < B - 1; ++i) sk.put(N + (r + 2 * i + 2) % N, v);
-    sk.publish();
-    sk.template raise_others<B>(2 * N + h, l, 2);
-  }
-  sk.put(r, v);                                            // forward to the pair
-  sk.publish();
-  sk.raise(3 * N + pair, 1);
-  store<U, ST>(dst, close, v);
-  poll.until([&] { return sk.look(3 * N + r) != 0; });     // pollFarGatherOutput
-  store<U, ST>(dst, far, sk.get(pair));
 }
 
 #undef VR_GROUP_PROLOGUE
@@ -413,43 +360,56 @@ struct Pick {
 template <int N, int DT, int LD, int ST, int U, bool LINED>
 Pick pick_flow(WireFlow flow) {
   constexpr Starts kWhole = LINED ? ON_LINES : ON_VECTORS, kAny = LINED ? ON_LINES : ON_HALVES;
+  constexpr uint32_t kSlots = N * U * 1024u;
   if constexpr (N <= 8) {
     switch (flow) {
-      case WIRE_PARALLEL: return {reinterpret_cast<const void *>(&k_group_parallel<N, DT, U, kAny, LD, ST>), N, ParallelSinks<N, U>::kBytes};
-      case WIRE_SEQUENTIAL: return {reinterpret_cast<const void *>(&k_group_sequential<N, DT, U, kWhole, LD, ST>), 1, SequentialSinks<N, U>::kBytes};
-      case WIRE_SIMPLE: return {reinterpret_cast<const void *>(&k_group_sequential<N, DT, U, kAny, LD, ST>), 1, SequentialSinks<N, U>::kBytes};
-      case WIRE_RING: return {reinterpret_cast<const void *>(&k_group_ring<N, DT, U, kWhole, LD, ST>), 1, RingSinks<N, U>::kBytes};
-      case WIRE_ALLGATHER:   // no adds: one instantiation serves both element types
-        if constexpr (U == 1)
-          return {reinterpret_cast<const void *>(&k_group_allgather<N, DT_F16, U, kWhole, LD, ST>), 1, RingSinks<N, U>::kBytes};
+      case WIRE_PARALLEL:
+      case WIRE_SEQUENTIAL:
+      case WIRE_SIMPLE:
+        if constexpr (U <= (N == 8 ? 4 : 2))
+          return {reinterpret_cast<const void *>(&k_group_exchange<N, ORDER_ROTATED, DT, U, kAny, LD, ST>), N, kSlots};
         break;
+      case WIRE_RING:
+        if constexpr (U <= (N == 8 ? 2 : 1))
+          return {reinterpret_cast<const void *>(&k_group_ring<N, DT, U, kWhole, LD, ST>), 1, RingSinks<N, U>::kBytes};
+        break;
+      case WIRE_ALLGATHER:   // no adds: one instantiation serves both element types
+        return {reinterpret_cast<const void *>(&k_group_allgather<N, U, kWhole, LD, ST>), N, U * 1024u};
       default: break;
     }
   }
-  if constexpr (N >= 4) {
-    if (flow == WIRE_BISECT) return {reinterpret_cast<const void *>(&k_group_bisect<N, DT, U, kAny, LD, ST>), N / 2, BisectSinks<N, U>::kBytes};
+  if constexpr (N >= 4 && U <= (N == 8 ? 4 : 2)) {
+    if (flow == WIRE_BISECT)
+      return {reinterpret_cast<const void *>(&k_group_exchange<N, ORDER_BISECT, DT, U, kAny, LD, ST>), N, kSlots};
   }
   return {nullptr, 0, 0};
 }
 
-template <int DT, int LD, int ST, bool LINED>
-Pick pick_ranks(WireFlow flow, int nranks, int unroll) {
+template <int DT, int LD, int ST, bool LINED, int U>
+Pick pick_ranks(WireFlow flow, int nranks) {
   switch (nranks) {
-    case 2: return pick_flow<2, DT, LD, ST, 1, LINED>(flow);
-    case 4: return pick_flow<4, DT, LD, ST, 1, LINED>(flow);
-    case 8: return unroll == 2 ? pick_flow<8, DT, LD, ST, 2, LINED>(flow) : pick_flow<8, DT, LD, ST, 1, LINED>(flow);
-    case 16: return unroll == 2 ? pick_flow<16, DT, LD, ST, 2, LINED>(flow) : pick_flow<16, DT, LD, ST, 1, LINED>(flow);
+    case 2: return pick_flow<2, DT, LD, ST, U, LINED>(flow);
+    case 4: return pick_flow<4, DT, LD, ST, U, LINED>(flow);
+    case 8: return pick_flow<8, DT, LD, ST, U, LINED>(flow);
+    case 16: return pick_flow<16, DT, LD, ST, U, LINED>(flow);
     default: return {nullptr, 0, 0};
   }
+}
+
+template <int DT, int LD, int ST, bool LINED>
+Pick pick_unroll(WireFlow flow, int nranks, int unroll) {
+  return unroll == 4   ? pick_ranks<DT, LD, ST, LINED, 4>(flow, nranks)
+         : unroll == 2 ? pick_ranks<DT, LD, ST, LINED, 2>(flow, nranks)
+                       : pick_ranks<DT, LD, ST, LINED, 1>(flow, nranks);
 }
 
 template <int LD, int ST>
 Pick pick_type(WireFlow flow, int nranks, DType dtype, int unroll, bool lined) {
   if (lined)
-    return dtype == DT_BF16 ? pick_ranks<DT_BF16, LD, ST, true>(flow, nranks, unroll)
-                            : pick_ranks<DT_F16, LD, ST, true>(flow, nranks, unroll);
-  return dtype == DT_BF16 ? pick_ranks<DT_BF16, LD, ST, false>(flow, nranks, unroll)
-                          : pick_ranks<DT_F16, LD, ST, false>(flow, nranks, unroll);
+    return dtype == DT_BF16 ? pick_unroll<DT_BF16, LD, ST, true>(flow, nranks, unroll)
+                            : pick_unroll<DT_F16, LD, ST, true>(flow, nranks, unroll);
+  return dtype == DT_BF16 ? pick_unroll<DT_BF16, LD, ST, false>(flow, nranks, unroll)
+                          : pick_unroll<DT_F16, LD, ST, false>(flow, nranks, unroll);
 }
 
 }  // namespace
@@ -457,24 +417,26 @@ Pick pick_type(WireFlow flow, int nranks, DType dtype, int unroll, bool lined) {
 hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow, int nranks, DType dtype,
                              const PtrTable &in, const PtrTable &out, size_t chunk_bytes, const GroupPlan &plan,
                              uint32_t spin_limit, uint32_t *status) {
-  const bool lined = (((uintptr_t)out.p[0] | chunk_bytes) & 127u) == 0;
+  // what wires are laid on (span_of)
+  const uint32_t grain = flow == WIRE_RING ? 128u : 1024u;
+  const bool lined = (((uintptr_t)out.p[0] | chunk_bytes) & (grain - 1u)) == 0;
   const Pick k =
       plan.policy == GROUP_STREAM     ? pick_type<kStreamLoad, kStreamStore>(flow, nranks, dtype, plan.unroll, lined)
       : plan.policy == GROUP_RESIDENT ? pick_type<0, 0>(flow, nranks, dtype, plan.unroll, lined)
                                       : pick_type<0, kStreamStore>(flow, nranks, dtype, plan.unroll, lined);
   if (!k.fn) return hipErrorInvalidValue;
-  const size_t wire = 1024u * (size_t)(nranks >= 8 ? plan.unroll : 1);   // payload of one wave
+  const size_t wire = 1024u * (size_t)plan.unroll;   // payload of one wave
   uint32_t lds = k.lds;
   const uint32_t cap = lds_cap_bytes(dev, plan.wgs_per_cu);
   if (cap > lds) lds = cap;
   if (hipError_t e = allow_dynamic_lds(k.fn, dev, lds); e != hipSuccess) return e;
   // (0 where every chunk starts on a line: those kernels take GroupArgs::seg as it is)
   const uint32_t head_mask =
-      !lined && (flow == WIRE_PARALLEL || flow == WIRE_BISECT || flow == WIRE_SIMPLE) ? head_mask_of(nranks, in, out) : 0u;
+      !lined && (flow != WIRE_RING && flow != WIRE_ALLGATHER) ? head_mask_of(nranks, in, out) : 0u;
   const size_t seg_max = plan.segment_bytes;
   for (size_t off = 0; off < chunk_bytes; off += seg_max) {
     const size_t seg = chunk_bytes - off < seg_max ? chunk_bytes - off : seg_max;
-    const dim3 grid((uint32_t)((seg + (lined ? 0 : 120) + wire - 1) / wire), k.rows), block(64u * (uint32_t)nranks);
+    const dim3 grid((uint32_t)((seg + (lined ? 0 : grain - 8) + wire - 1) / wire), k.rows), block(64u * (uint32_t)nranks);
     hipEvent_t ev0 = off == 0 ? tl_kernel_events.start : nullptr;
     hipEvent_t ev1 = off + seg >= chunk_bytes ? tl_kernel_events.stop : nullptr;
     hipError_t e = hipErrorInvalidValue;
@@ -482,6 +444,7 @@ hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow
 #define VR_CASE(NN)                                                                                            \
   case NN: {                                                                                                   \
     GroupArgs<NN> a = group_args<NN>(in.p, out.p, chunk_bytes, off, seg, head_mask, spin_limit, status);       \
+    if (flow == WIRE_ALLGATHER) a.rest = (a.rest & 0x1ffffu) | run_code(plan.run, grid.x);                     \
     void *kargs[] = {&a};                                                                                      \
     e = launch_kernel(k.fn, grid, block, kargs, lds, s, ev0, ev1);                                             \
     break;                                                                                                     \

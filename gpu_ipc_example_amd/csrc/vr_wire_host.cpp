@@ -102,65 +102,79 @@ static uint32_t spin_limit_of(const vr_ctx *c) {
   return limit > 0xffffffffull ? 0xffffffffu : (uint32_t)limit;
 }
 
-// Launch shape of the work-group form.  `reads` = bytes of all ranks' inputs.
+// Launch shape of the work-group form.  `reads` = bytes of all ranks' inputs.  Lines lie where
+// calls that take three sets of buffers in turn change sides, us per call with each:
 static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_place) {
   const size_t MiB = (size_t)1 << 20;
   GroupPlan p = {GROUP_MIXED, 1, 0};
-  // Cache policies, us per pass on one / three / ten sets of buffers in turn:
-  //  * in place up to 72 MiB everything stays cacheable: what else a caller's program touches
+  // Cache policies:
+  //  * in place up to 80 MiB everything stays cacheable: what else a caller's program touches
   //    between two calls is not known here, so room is left for twice as much again (three sets
-  //    fit the memory-side cache) (8 x 4 MiB 9.1 / 12.9 / 16.0, streamed 13.9 / 15.9 / 15.9; 9 MiB per rank on 8, one
-  //    and three sets: parallel 23.4 / 23.8, streamed 27.6 / 27.9, ring 8 x 8 MiB + 16 B
-  //    20.7 / 20.5, streamed 27.2 / 27.3), beyond it streaming wins as soon as the buffers do
-  //    not all fit (8 x 10 MiB: simple 26.3 / 33.5, streamed 30.4 / 30.5; 8 x 16 MiB
-  //    39.5 / 50.5 / 53.2, streamed 49.9 / 48.9 / 49.4).  (The direct transport, which stays
-  //    cacheable up to 255 MiB, takes 41.5 there on one set and 52.0 with inputs that change, parallel 53.4
-  //    and 49.3.)
-  //  * out of place up to half the memory-side cache of inputs: results are streamed past
-  //    inputs that may stay (8 x 16 MiB 41.3 / 49.3 / 50.5, everything streamed
-  //    50.2 / 50.2 / 49.4), beyond it everything streams (8 x 128 MiB 355, 351 us);
+  //    fit the memory-side cache); beyond it streaming wins as soon as the buffers do not all fit
+  //    (2 / 4 / 8 / 16 ranks, 73 MiB 22.1 / 24.1 / 25.0 / 25.7 cacheable, 24.0 / 26.2 / 27.4 / 30.6
+  //    streamed; 79 to 86 MiB even at 2 and 4 ranks, at 8 and 16 ranks cacheable is 2 to 5 % ahead up to
+  //    91);
+  //  * out of place up to 100 MiB of inputs results are streamed past inputs that may stay (4 x 14
+  //    MiB 17.7, everything streamed 21.2), beyond it everything streams (4 x 28 MiB 39.3 / 38.6,
+  //    2 x 58 39.5 / 38.3);
   //  * all-gather: results are streamed past the inputs at every size, they are N times as
-  //    long (2 x 64 MiB 58.2 / 65.9, everything streamed 68.0 / 66.9; 8 x 16 MiB 193 / 222, streamed
-  //    238 / 230; with inputs that change, 256 and 512 MiB of them: 8 x 32 MiB 399, streamed 416, 8 x 64
-  //    810, 821, 2 x 128 and 4 x 128 even).
-  if (in_place) p.policy = reads <= 72 * MiB ? GROUP_RESIDENT : GROUP_STREAM;
-  else if (reads > 128 * MiB && flow != WIRE_ALLGATHER) p.policy = GROUP_STREAM;
-  // Two vectors per lane at 8 and 16 ranks, where that is the faster (fewer waves for the
-  // same bytes where the caches feed them quicker than waves start; at 2 and 4 ranks one vector
-  // is 10 to 40 % faster at every size):
+  //    long (8 x 19 MiB 256, everything streamed 264; 4 x 32 112, 116).
+  if (in_place) p.policy = reads <= 80 * MiB ? GROUP_RESIDENT : GROUP_STREAM;
+  else if (reads > 100 * MiB && flow != WIRE_ALLGATHER) p.policy = GROUP_STREAM;
+  // Vectors per lane: fewer and larger work-groups where caches feed them quicker than they
+  // start, one vector where HBM does.
   switch (flow) {
     case WIRE_PARALLEL:
-      // 8 x 4 MiB 16.6 -> 12.9 us, 8 x 8 MiB 27.4 -> 23.0; 8 x 16 MiB is better off with one
-      // (50.5, two: 55.5).  From 512 MiB on with three work-groups per CU, 48 KiB of loads
-      // in flight: 8 x 64 MiB 173.9 -> 168.7 us, 8 x 256 MiB 720 -> 689; 8 x 48 MiB 132.2, two: 133.1.
-      if (nranks == 8 && reads <= 64 * MiB) p.unroll = 2;
-      if (nranks == 8 && reads >= 512 * MiB) p.unroll = 2, p.wgs_per_cu = 3;
-      break;
     case WIRE_BISECT:
-      // 8 x 4 MiB 15.2 -> 11.8 us, 8 x 2 and 8 x 8 MiB even; 16 x 4 MiB 29.8 -> 22.0 us,
-      // 16 x 8 MiB 53.8, two: 57.4
-      // Four ranks, streaming, from 192 MiB on: five work-groups per CU (40 KiB of loads in
-      // flight, uncapped 64).  4 x 64 MiB 91.7 -> 84.1 us, 4 x 128 MiB 165.5 -> 163.2.  (Eight
-      // ranks with three: from 5 % faster to 11 % slower.)
-      p.unroll = nranks == 8 ? (reads >= 16 * MiB && reads < 64 * MiB ? 2 : 1) : nranks == 16 && reads <= 96 * MiB ? 2 : 1;
-      if (nranks == 4 && reads >= 192 * MiB) p.wgs_per_cu = 5;
-      break;
-    case WIRE_RING:
     case WIRE_SEQUENTIAL:
     case WIRE_SIMPLE:
-      // ring 8 x 16 MiB 65.1 -> 48.9 us, sequential 65.6 -> 46.8; 8 x 4 MiB even, 8 x 2 MiB
-      // 8.4, two: 9.9; 8 x 32 MiB 97.7, two: 108.8
+      if (nranks <= 4) {
+        // 2 ranks in place 10 MiB 4.59, two vectors 4.03; 12 MiB 5.23 / 4.82; 17 MiB 6.81 / 7.04; 4 ranks 10
+        // MiB 4.41 / 4.09, 17 MiB 7.32 / 6.12, 20 MiB 7.83 / 8.24
+        p.unroll = reads >= 9 * MiB && reads < 16 * MiB ? 2 : 1;
+      } else if (nranks == 8) {
+        // In place two / four vectors: 8 MiB 3.83 / 4.05, 12 MiB 5.03 / 5.36, 14 MiB 6.31 / 5.92, 40 MiB
+        // 14.4 / 13.9; one / four: 50 MiB out of place 16.9 / 16.3, 64 MiB 21.2 / 22.1, out of place 20.1 / 22.0,
+        // 120 MiB 43.9 / 47.2 (three work-groups a CU 45.6 with one vector)
+        p.unroll = reads < 13 * MiB ? 2 : reads < 56 * MiB ? 4 : 1;
+        // Chunks of 24 MiB and more that are multiples of 1 MiB start all streams on one channel: two
+        // vectors with three work-groups a CU 668 us at 8 x 256 MiB, one 681; on other lengths 665, 653.
+        if (reads >= 1536 * MiB && reads % (64 * MiB) == 0) p.unroll = 2, p.wgs_per_cu = 3;
+      } else {
+        // 16 ranks, one / two: 6 MiB in place 4.89 / 4.74, 24 MiB 10.1 / 9.9, 64 MiB 22.3 / 25.3, 192 MiB 68.0 /
+        // 70.0, out of place 68.9 / 70.7 (bfloat16 73.0 / 72.0)
+        p.unroll = reads < 56 * MiB ? 2 : 1;
+      }
+      break;
+    case WIRE_RING:
+      // 8 x 16 MiB 65.1 -> 48.9 us; 8 x 4 MiB even, 8 x 2 MiB 8.4, two: 9.9; 8 x 32 MiB 97.7, two: 108.8
       if (nranks == 8 && reads >= 32 * MiB && reads <= 192 * MiB) p.unroll = 2;
-      // Ring, four ranks, streaming: 48 KiB of loads per CU in flight instead of 128.
+      // Four ranks, streaming: 48 KiB of loads per CU in flight instead of 128.
       // 4 x 64 MiB 106 -> 94 us, 4 x 128 MiB 190.5 -> 169.5; 4 x 32 MiB 50.7, capped 50.9.  (Eight
       // ranks with one vector: their 64 KiB of slots hold a compute unit at two work-groups anyway;
       // with two vectors no cap was timed.)
-      if (flow == WIRE_RING && nranks == 4 && reads >= 192 * MiB) p.wgs_per_cu = 3;
+      if (nranks == 4 && reads >= 192 * MiB) p.wgs_per_cu = 3;
       break;
-    case WIRE_ALLGATHER:   // one vector: 8 x 4 MiB 49.0, two: 59.1 us
-      // Four ranks with four work-groups per CU: 4 x 4 MiB 14.5 -> 13.6 us, 4 x 16 MiB 52.9 -> 48.6,
-      // 4 x 32 MiB 121.6 -> 109.2; 4 x 2 MiB 6.7, capped 6.5
-      if (nranks == 4 && reads >= 8 * MiB) p.wgs_per_cu = 4;
+    case WIRE_ALLGATHER:
+      // One vector per lane, so that the N waves of a work-group each write one KiB, and 64 KiB of a
+      // slice in a row on an XCD, where the inputs of three calls fit the memory-side cache (one /
+      // two / four vectors, R = 1: every XCD every eighth KiB; 8 ranks 24 MiB 32.3 / 34.3 / 35.6, R = 1 32.1,
+      // 48 MiB 60.0 / 67.6 / 67.8, 64 MiB 80.3 / 90.0 / 89.6; 4 ranks 32 MiB 23.9 / 25.1 / 24.3, R = 1 24.2, 64 MiB
+      // 46.1 / 47.6 / 47.4; 2 ranks 24 MiB 11.8 / 12.0 / 11.7, 64 MiB 28.8 / 28.8 / 27.9).  Beyond, one
+      // KiB loaded by a work-group is too little in flight: two vectors, R = 1 (8 ranks 80 MiB 119 / 113, 128 MiB
+      // 251 / 185; 4 ranks 96 MiB 84.0 / 76.2, 200 MiB 195 / 163; 2 ranks 128 MiB 62.1 / 63.0).  Below, where
+      // the start of a launch counts: two vectors (8 ranks 6 MiB 9.45 / 9.26; 4 ranks 6 MiB 5.58 / 5.26).
+      if (nranks == 8) {
+        p.unroll = reads >= 7 * MiB && reads < 72 * MiB ? 1 : 2;
+        p.run = reads < 7 * MiB ? 16 : reads < 72 * MiB ? 64 : 1;
+      } else if (nranks == 4) {
+        p.unroll = reads >= 10 * MiB && reads < 88 * MiB ? 1 : 2;
+        p.run = reads < 88 * MiB ? 64 : 1;
+      } else {
+        p.unroll = reads < 14 * MiB ? 2 : 1;
+        if (reads >= 20 * MiB && reads < 88 * MiB) p.unroll = 4, p.wgs_per_cu = 3;
+        p.run = reads < 88 * MiB ? 64 : 1;
+      }
       break;
   }
   return p;

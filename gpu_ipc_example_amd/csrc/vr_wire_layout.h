@@ -123,13 +123,14 @@ struct Span {
   VR_HD uint32_t first_load() const { return half() ? 8u : off; }
 };
 // The chunk's bytes [base, base + seg_bytes) of each buffer; `lines` = place of the first output
-// in its line and, in the second byte, 8 where a chunk that starts in the middle of 16 bytes does
-// so in every buffer, else 0; `off` = the lane's place counted from the start of the first wire.
-// `lined` = every chunk starts on a line.
-VR_HD Span wire_span(bool lined, size_t base, uint32_t seg_bytes, uint32_t lines, uint32_t off, bool first_wire) {
+// in its KiB and, as 8 << 8, whether a chunk that starts in the middle of 16 bytes does so in
+// every buffer; `off` = the lane's place counted from the start of the first wire.  `lined` =
+// every chunk starts on a multiple of `grain` bytes, on which wires are laid: a line, or a KiB.
+VR_HD Span wire_span(bool lined, size_t base, uint32_t seg_bytes, uint32_t lines, uint32_t off, bool first_wire,
+                     uint32_t grain = 128) {
   if (lined) return Span{base, seg_bytes, off, false};
-  const uint32_t addr = (lines & 0xffu) + (uint32_t)base, head = addr & (lines >> 8);
-  return Span{base - head, seg_bytes + head, off - ((addr - head) & 112u), first_wire && head != 0};
+  const uint32_t addr = (lines & 0x3ffu) + (uint32_t)base, head = addr & (lines >> 8 & 8u);
+  return Span{base - head, seg_bytes + head, off - ((addr - head) & (grain - 16u)), first_wire && head != 0};
 }
 
 // ---- flag values ----------------------------------------------------------------------------

@@ -93,12 +93,11 @@ typedef enum vr_algo {
  *          except VR_ALGO_PARALLEL.
  *  WIRE  : the reference's stage structure — every rank's waves load their own input
  *          only, scatter into the owner's sink, reduce, gather into every peer's sink
- *          and store their own output only; receivers learn of a message from a flag.
- *          Default for VR_ALGO_PARALLEL.  Two forms:
+ *          and store their own output only.  Default for VR_ALGO_PARALLEL.  Two forms:
  *          - a call that holds all ranks and leaves every "wire_*" setting and the grid
  *            to the library: the N waves of a wire column (one per rank) are one
- *            work-group and the sinks lie in its compute unit's LDS, flag words at
- *            work-group scope;
+ *            work-group and the sinks lie in its compute unit's LDS; its barrier says
+ *            that messages are there, in the ring protocols a flag word for each rank;
  *          - everything else (launches that hold some of the ranks, a user grid, any
  *            "wire_*" setting): sinks in scratch memory, one persistent kernel whose
  *            work-groups are partitioned between the ranks.  Flags are the reference's,
@@ -313,8 +312,8 @@ int vr_allgather_grid(vr_ctx *ctx, void *stream, int algo, int transport, const 
  * scratch has been zeroed again; sinks a caller handed to the rank-group launches
  * are the caller's to zero. */
 int vr_ctx_check(vr_ctx *ctx, void *stream);
-/* Poll budget of the wire transport's bounded spin (0 = library default).  Launches that hold
- * all ranks take it rounded up to 10 significant bits. */
+/* Poll budget of the wire transport's bounded spin (0 = library default).  Ring launches that hold
+ * all ranks take it rounded up to 10 significant bits; the others of that form wait for no flag. */
 int vr_ctx_set_spin_limit(vr_ctx *ctx, uint64_t polls);
 
 /* Tuning knobs for the direct kernels (benchmark sweeps).  Unknown keys are

@@ -43,7 +43,7 @@ static void check(uint64_t in_base, uint64_t out_base, size_t pitch, size_t off,
       EXPECT(g.rank[k].out() == (uintptr_t)out[k] + off);
     }
     EXPECT(g.pitch() == pitch && (g.seg & 0x7fffffffu) == seg && (head || g.seg == seg));
-    EXPECT(g.lines() == ((((uintptr_t)out[0] + off) & 127u) | head << 8));
+    EXPECT(g.lines() == ((((uintptr_t)out[0] + off) & 1023u) | head << 8));
     EXPECT(g.status_address(g.rest, g.status_lo) == status);
     const uint32_t got = g.spin_limit(g.rest);
     // rounded up to 10 significant bits, at most the largest that 32 bits hold
@@ -67,6 +67,14 @@ int main() {
               check<8>(b, o, pitch, off, seg, head, spin);
               check<16>(b, o, pitch, off, seg, head, spin);
             }
+  for (int run : {1, 2, 64, 128, 256})
+    for (uint32_t cols : {1u, 7u, 8u, 1023u, 1024u, 1025u, 4194304u}) {
+      GroupArgs<2> g = {};
+      g.rest = 0x1ffffu | run_code(run, cols);
+      EXPECT(1 << g.run_log2() == (run > 128 ? 128 : run));
+      const uint32_t group = 8u << g.run_log2();
+      EXPECT(g.run_cols() % group == 0 && g.run_cols() <= cols && (g.run_cols() + group > cols || g.run_cols() == 4095u * group));
+    }
   EXPECT(sizeof(DirectArgs<8>) == kCheapArgBytes && sizeof(GroupArgs<8>) == kCheapArgBytes);
   if (failures) {
     printf("%d failures\n", failures);

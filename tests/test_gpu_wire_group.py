@@ -1,8 +1,7 @@
 """Wire-transport launches that hold all ranks (messages through LDS) at the sizes where
 the work-group form can go wrong, bit for bit against the oracle.  A wave's wire is 1 KiB
-of a chunk, 2 KiB where a lane carries two vectors (parallel at 8 ranks up to 64 MiB and
-from 512 MiB of inputs, bisect at 16, ring and sequential at 8 from 32 MiB); a chunk of
-8-byte messages may end inside a lane's 16 bytes."""
+of a chunk, 2 or 4 KiB where a lane carries two or four vectors (as the sizes of inputs given
+below make it); a chunk of 8-byte messages may end inside a lane's 16 bytes."""
 import numpy as np
 import pytest
 
@@ -65,6 +64,20 @@ def test_ragged_sizes_of_the_larger_launches(oracle, algo, mib):
     ctx.close()
 
 
+@pytest.mark.parametrize("nranks,algo,kib", [(2, "simple", 12 * 1024), (4, "bisect", 12 * 1024), (8, "parallel", 8 * 1024),
+                                             (8, "small_pcie", 14 * 1024), (8, "bisect", 80 * 1024),
+                                             (8, "simple_transmit", 20 * 1024), (16, "bisect", 90 * 1024)])
+def test_vectors_per_lane(oracle, nranks, algo, kib):
+    """Two and four vectors per lane: messages of 2 and 4 KiB whose last ends early, and a wave's
+    share of the sums in each width."""
+    msg = 16 if algo == "small_pcie" else 8
+    ctx = vr.VirtualRanks(nranks)
+    chunk = kib * 1024 // nranks ** 2 // 4096 * 4096
+    for k, tail in enumerate((0, msg, 1024 - msg, 3072 + msg)):
+        run(oracle, ctx, algo, nranks * (chunk + tail) // 2, BF16 if k % 2 else F16, k < 2, 0, 46_000 + 100 * k)
+    ctx.close()
+
+
 @pytest.mark.parametrize("nranks", [2, 8])
 def test_allgather_edges(oracle, nranks):
     ctx = vr.VirtualRanks(nranks)
@@ -87,6 +100,21 @@ def test_capped_and_resident_launches(oracle, nranks, algo, mib, inplace):
     msg = 16 if algo == "simple_ring" else 8
     chunk = (mib << 20) // nranks ** 2 // 16 * 16 + 3 * msg
     run(oracle, ctx, algo, nranks * chunk // 2, F16, inplace, 0, 70_000)
+    ctx.close()
+
+
+@pytest.mark.parametrize("nranks,kib", [(8, 512), (8, 1024), (4, 700), (4, 3 * 1024), (2, 6 * 1024), (2, 12 * 1024),
+                                        (8, 10 * 1024)])
+def test_runs_of_a_gather(oracle, nranks, kib):
+    """KiB of input per rank at which work-groups are permuted (in runs of 16 and 64 KiB, with one,
+    two and four vectors per lane) and at which they are not: a last group that is whole, and ragged ones."""
+    ctx = vr.VirtualRanks(nranks)
+    for tail in (0, 16, 9 * 1024 + 1008):
+        n = (kib * 1024 + tail) // 2
+        ins = [oracle.generate_dt(F16, n, 72_000 + r, DIST_NORMAL, 0.0, 1.0) for r in range(nranks)]
+        want = oracle.allgather(ins)
+        for r, got in enumerate(run_allgather_wire(ctx, "allgather_simple", ins, tail == 16)):
+            assert (got == want).all(), (n, r)
     ctx.close()
 
 
