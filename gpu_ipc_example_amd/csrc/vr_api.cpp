@@ -599,6 +599,43 @@ static int resolve_transport(const AlgoInfo *a, int transport, int *out) {
   return VR_OK;
 }
 
+// The direct transport has a second kernel: one pass over the same bytes in which a
+// work-group's waves load one rank's input each, hand the data to each other through LDS and
+// store one rank's output each (the wire transport's, vr_wire_group.hip).  Its waves have two
+// streams each instead of 2N (all-gather: N + 1), which the caches like better, and hardly a
+// prologue.  This says for which calls it is the faster; calls with a grid or a tuning key of the
+// direct kernels take those.  us per call with three sets of buffers in turn, register kernel / through LDS:
+//   in place   2 ranks 16 MiB 6.0 / 6.8, 24 11.0 / 8.7, 65 22.2 / 20.3, 161 63.8 / 51.8, 1007 334 / 309
+//              4 ranks 50 MiB 16.2 / 16.6, 79 24.7 / 25.2, 100 38.5 / 34.8, 164 62.2 / 54.5, 391 125 / 124
+//              8 ranks 4 MiB 3.43 / 3.32, 8 3.89 / 3.51, 10 5.01 / 4.11, 16 7.05 / 7.15, 67 21.7 / 22.5, 81 32.9 /
+//              31.8, 130 54.7 / 46.7, 224 101 / 79, 335 113.6 / 112.5, 1963 639 / 662
+//              16 ranks 2 MiB 4.99 / 3.33, 16 8.4 / 6.7, 39 15.4 / 14.3, 63 22.4 / 23.7, 100 39.3 / 37.4, 196 90 / 72,
+//              501 184 / 178, 718 250 / 255; bfloat16 40 MiB 16.0 / 15.5, 90 34.7 / 35.0, 192 85.8 / 72.3, 512 176 / 184
+//   out of     2 ranks 12 MiB 5.4 / 7.0, 19 8.6 / 7.0, 66 20.3 / 19.9, 113 41.6 / 37.5, 309 99.6 / 97.4, 1019 331 / 315
+//   place      4 ranks 17 MiB 6.40 / 6.43, 24 9.3 / 8.8, 66 20.8 / 20.2, 113 45.7 / 38.6, 233 76.1 / 75.4, 697 222 / 220
+//              8 ranks 4 MiB 3.27 / 3.35, 8 3.89 / 3.33, 33 11.8 / 11.6, 63 20.5 / 20.2, 80 25.5 / 26.7, 107 44.9 /
+//              38.0, 228 79.8 / 78.2, 256 81.8 / 85.5, 686 227 / 228
+//              16 ranks 40 MiB 14.7 / 13.9, 64 22.0 / 22.6, 99 40.2 / 37.0, 128 52 / 47, 190 70.1 / 69.9
+//   all-gather 2 ranks 12 MiB 5.8 / 6.3, 16 8.6 / 8.4, 64 29.2 / 27.9, 96 45.8 / 46.5, 200 101 / 97
+//              4 ranks 8 MiB 7.0 / 7.0, 12 11.4 / 9.8, 32 24.3 to 27.4 / 23.9, 64 51.0 / 46.2, 200 171 / 164
+//              8 ranks 6 MiB 9.9 / 9.7, 12 18.7 / 17.5, 32 43.2 to 50.0 / 43.0, 64 96.7 / 81.5, 200 310 / 301
+static bool faster_through_lds(const vr_ctx *ctx, const AlgoInfo *a, size_t read_bytes, bool in_place) {
+  const TuningOverrides &o = ctx->tune;
+  if (o.block != -1 || o.waves_per_cu != -1 || o.unroll != -1 || o.nt_load != -1 || o.nt_store != -1 || o.oneshot != -1 ||
+      o.segment_kib != -1 || o.f16_wide != -1 || o.wgs_per_cu != -1 || o.deal != -1 || o.run != -1)
+    return false;
+  const size_t MiB = (size_t)1 << 20;
+  const auto within = [&](size_t from, size_t to) { return read_bytes >= from * MiB && read_bytes < to * MiB; };
+  const size_t any = (size_t)-1 / MiB;
+  if (a->allgather) return read_bytes >= (ctx->nranks == 2 ? 14 : ctx->nranks == 4 ? 10 : 6) * MiB;
+  switch (ctx->nranks) {
+    case 2: return within(18, any);
+    case 4: return in_place ? within(88, 256) : within(20, 256);
+    case 8: return in_place ? within(4, 15) || within(80, 256) : within(5, 64) || within(88, 256);
+    default: return within(0, 40) || (in_place ? within(96, 256) : within(88, 129));   // 16
+  }
+}
+
 // Runs one all-reduce starting at sequence number `seq_no`; *next_seq receives
 // the sequence number the following launch should start at.
 static int run_allreduce(vr_ctx *ctx, hipStream_t s, const Prepared &p, int transport,
@@ -616,6 +653,8 @@ static int run_allreduce(vr_ctx *ctx, hipStream_t s, const Prepared &p, int tran
     if (*next_seq == 0) *next_seq = 1;
     return VR_OK;
   }
+  if (!t.force_blocks_per_rank && faster_through_lds(ctx, p.a, p.bytes_all_ranks, p.in_place))
+    return group_launch(ctx, s, p.a->order == ORDER_BISECT ? WIRE_BISECT : WIRE_PARALLEL, p.in, p.out, p.chunk_elems * 2);
   hipError_t e = launch_direct_allreduce(s, ctx->dev, t, ctx->nranks, p.a->order, ctx->dtype, p.in,
                                          p.out, p.chunk_elems);
   if (e != hipSuccess) return fail_hip(e, "launch_direct_allreduce");
@@ -738,8 +777,12 @@ static int run_allgather(vr_ctx *ctx, hipStream_t s, const PreparedGather &p, in
     return VR_OK;
   }
   if (transport != VR_TRANSPORT_DEFAULT && transport != VR_TRANSPORT_DIRECT) return fail(VR_ERR_INVALID, "bad transport");
-  hipError_t e = launch_direct_allgather(s, ctx->dev, t, ctx->nranks, p.in, p.out, nelems);
-  if (e != hipSuccess) return fail_hip(e, "launch_direct_allgather");
+  if (!t.force_blocks_per_rank && faster_through_lds(ctx, p.a, (size_t)ctx->nranks * nelems * 2, false)) {
+    if (int rc = group_launch(ctx, s, WIRE_ALLGATHER, p.in, p.out, nelems * 2)) return rc;
+  } else {
+    hipError_t e = launch_direct_allgather(s, ctx->dev, t, ctx->nranks, p.in, p.out, nelems);
+    if (e != hipSuccess) return fail_hip(e, "launch_direct_allgather");
+  }
   *next_seq = seq_no + p.geom.steps;
   if (*next_seq == 0) *next_seq = 1;
   return VR_OK;

@@ -180,19 +180,19 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
   return p;
 }
 
-static int group_launch(vr_ctx *c, hipStream_t s, const AlgoInfo *a, const PtrTable &in, const PtrTable &out,
-                        size_t chunk_bytes) {
+namespace vr {
+int group_launch(vr_ctx *c, hipStream_t s, WireFlow flow, const PtrTable &in, const PtrTable &out, size_t chunk_bytes) {
   const int N = c->nranks;
-  const WireFlow flow = a->wire_flow();
-  bool in_place = !a->allgather;
+  bool in_place = flow != WIRE_ALLGATHER;
   for (int r = 0; r < N; ++r) in_place = in_place && in.p[r] == out.p[r];
-  const size_t reads = (size_t)N * chunk_bytes * (a->allgather ? 1 : N);
+  const size_t reads = (size_t)N * chunk_bytes * (flow == WIRE_ALLGATHER ? 1 : N);
   GroupPlan plan = group_plan(flow, N, reads, in_place);
   if (c->tune.segment_kib != -1) plan.segment_bytes = (size_t)c->tune.segment_kib << 10;
   const hipError_t e = launch_wire_group(s, c->dev, flow, N, c->dtype, in, out, chunk_bytes, plan, spin_limit_of(c),
                                          c->status);
   return e == hipSuccess ? VR_OK : fail_hip(e, "launch_wire_group");
 }
+}  // namespace vr
 
 struct WireLaunch {
   const WireSinks *sinks;
@@ -344,7 +344,7 @@ static int wire_launch(vr_ctx *c, hipStream_t s, const AlgoInfo *a, const PtrTab
   if ((wlch.hist || wlch.always_clear) && takes_group_form(c, user_wires)) {
     *flags_used = chunk_bytes ? 1u : 0u;
     if (seq + *flags_used == 0) *seq_io = 1;   // 0 is never handed out
-    return group_launch(c, s, a, in, out, chunk_bytes);
+    return group_launch(c, s, a->wire_flow(), in, out, chunk_bytes);
   }
   WirePlan plan;
   if (int rc = plan_wire(c, a, chunk_bytes, vec_halves, user_wires, k, &plan)) return rc;

@@ -90,7 +90,8 @@ typedef enum vr_algo {
  *  DIRECT: the workgroups of the rank that owns a chunk read every rank's input
  *          in place, add in the protocol's order, and write every rank's output.
  *          One pass over HBM; no scratch, no flags.  Default for every algo
- *          except VR_ALGO_PARALLEL.
+ *          except VR_ALGO_PARALLEL.  The data meets in registers or, at sizes where
+ *          that is the faster, in a compute unit's LDS.
  *  WIRE  : the reference's stage structure — every rank's waves load their own input
  *          only, scatter into the owner's sink, reduce, gather into every peer's sink
  *          and store their own output only.  Default for VR_ALGO_PARALLEL.  Two forms:
@@ -361,7 +362,9 @@ int vr_ctx_set_spin_limit(vr_ctx *ctx, uint64_t polls);
  * -1 restores the library's own choice. */
 /* The launch the direct transport gives a collective of this shape when nothing
  * is overridden: pure host arithmetic, no device needed (nelems per rank; in_place
- * is ignored for an all-gather).  No counterpart in the reference, whose launch
+ * is ignored for an all-gather): the launch of the kernels whose data meets in registers,
+ * the ones that the tuning keys and a grid are for.  A call that sets none of them may
+ * take the kernel that goes through LDS instead.  No counterpart in the reference, whose launch
  * shape is the user's -g / -w / -s (main.cpp:181-198). */
 typedef struct vr_launch_plan {
   int one_trip;      /* 1: one tile per work-group, started in index order; 0: persistent grid-stride grid */
