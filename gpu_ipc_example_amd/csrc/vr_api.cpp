@@ -604,21 +604,26 @@ static int resolve_transport(const AlgoInfo *a, int transport, int *out) {
 // store one rank's output each (the wire transport's, vr_wire_group.hip).  Its waves have two
 // streams each instead of 2N (all-gather: N + 1), which the caches like better, and hardly a
 // prologue.  This says for which calls it is the faster; calls with a grid or a tuning key of the
-// direct kernels take those.  us per call with three sets of buffers in turn, register kernel / through LDS:
-//   in place   2 ranks 16 MiB 6.0 / 6.8, 24 11.0 / 8.7, 65 22.2 / 20.3, 161 63.8 / 51.8, 1007 334 / 309
-//              4 ranks 50 MiB 16.2 / 16.6, 79 24.7 / 25.2, 100 38.5 / 34.8, 164 62.2 / 54.5, 391 125 / 124
-//              8 ranks 4 MiB 3.43 / 3.32, 8 3.89 / 3.51, 10 5.01 / 4.11, 16 7.05 / 7.15, 67 21.7 / 22.5, 81 32.9 /
-//              31.8, 130 54.7 / 46.7, 224 101 / 79, 335 113.6 / 112.5, 1963 639 / 662
-//              16 ranks 2 MiB 4.99 / 3.33, 16 8.4 / 6.7, 39 15.4 / 14.3, 63 22.4 / 23.7, 100 39.3 / 37.4, 196 90 / 72,
-//              501 184 / 178, 718 250 / 255; bfloat16 40 MiB 16.0 / 15.5, 90 34.7 / 35.0, 192 85.8 / 72.3, 512 176 / 184
-//   out of     2 ranks 12 MiB 5.4 / 7.0, 19 8.6 / 7.0, 66 20.3 / 19.9, 113 41.6 / 37.5, 309 99.6 / 97.4, 1019 331 / 315
-//   place      4 ranks 17 MiB 6.40 / 6.43, 24 9.3 / 8.8, 66 20.8 / 20.2, 113 45.7 / 38.6, 233 76.1 / 75.4, 697 222 / 220
-//              8 ranks 4 MiB 3.27 / 3.35, 8 3.89 / 3.33, 33 11.8 / 11.6, 63 20.5 / 20.2, 80 25.5 / 26.7, 107 44.9 /
-//              38.0, 228 79.8 / 78.2, 256 81.8 / 85.5, 686 227 / 228
-//              16 ranks 40 MiB 14.7 / 13.9, 64 22.0 / 22.6, 99 40.2 / 37.0, 128 52 / 47, 190 70.1 / 69.9
-//   all-gather 2 ranks 12 MiB 5.8 / 6.3, 16 8.6 / 8.4, 64 29.2 / 27.9, 96 45.8 / 46.5, 200 101 / 97
-//              4 ranks 8 MiB 7.0 / 7.0, 12 11.4 / 9.8, 32 24.3 to 27.4 / 23.9, 64 51.0 / 46.2, 200 171 / 164
-//              8 ranks 6 MiB 9.9 / 9.7, 12 18.7 / 17.5, 32 43.2 to 50.0 / 43.0, 64 96.7 / 81.5, 200 310 / 301
+// register kernels take those.  us per call, register kernels / through LDS, with three sets of buffers
+// in turn, and as many as no cache holds where a ratio follows (there 5 to 30 % faster nearly throughout):
+//   in place   2 ranks 24 MiB 12.3 / 13.4, 40 18.3 / 18.6, 65 22.2 / 20.3, 100 38.2 / 33.9, 161 63.8 / 51.8 (1.21), 1007 334 / 309
+//              4 ranks 50 MiB 16.2 / 16.6, 79 24.7 / 25.2, 100 38.5 / 34.8 (1.17), 164 62.2 / 54.5, 391 125 / 124, 2048 647 / 643
+//              8 ranks 8 MiB 3.89 / 3.51 (1.16), 10 5.01 / 4.11, 12 (1.09), 16 7.05 / 7.15, 67 21.7 / 22.5, 81 to 100
+//              mixed (0.90 to 1.08; 1.17), 120 51.3 / 49.1 (1.14), 130 54.7 / 46.7, 224 101 / 79, 512 164 / 162, 1024
+//              327 / 323, 1963 639 / 662
+//              16 ranks 2 MiB 4.99 / 3.33, 16 8.4 / 6.7, 39 15.4 / 14.3, 63 22.4 / 23.7, 100 39.3 / 37.4, 196 90 / 72 (1.33),
+//              718 250 / 255; bfloat16 40 MiB 16.0 / 15.5, 90 34.7 / 35.0, 192 85.8 / 72.3, 512 176 / 184
+//   out of     2 ranks 12 MiB 5.4 / 7.0, 24 10.5 / 10.9, 32 14.8 / 13.0 (1.09), 66 20.3 / 19.9, 113 41.6 / 37.5, 1019 331 / 315
+//   place      4 ranks 24 MiB 10.8 / 11.4, 32 18.1 / 13.7 (1.19), 66 20.8 / 20.2 (1.15), 113 45.7 / 38.6, 697 222 / 220
+//              8 ranks 4 MiB 3.27 / 3.35, 8 3.89 / 3.33 (1.17), 33 11.8 / 11.6 (1.08), 63 20.5 / 20.2, 80 25.5 / 26.7,
+//              90 to 107 mixed (0.84 to 1.18), 120 (1.09), 228 79.8 / 78.2, 256 82.2 / 81.4, 512 163.6 / 162.3, 686 227 / 228
+//              16 ranks 40 MiB 14.7 / 13.9, 64 22.0 / 22.6, 99 40.2 / 37.0 (1.15), 128 52 / 47, 190 70.1 / 69.9
+//   all-gather 2 ranks 12 MiB 5.8 / 6.3, 16 8.7 / 8.3, 64 29.4 / 28.8, 128 65.5 / 62.9
+//              4 ranks 8 MiB 7.0 / 6.9, 12 11.0 / 10.0, 32 25.8 / 24.6 (1.07), 64 50.9 / 48.2, 128 104 / 102
+//              8 ranks 8 MiB 12.4 / 12.0 (0.97), 12 19.3 / 18.6 (0.98), 24 36.3 / 35.1 (1.03), 32 52.2 / 46.7, 64 98.1 / 87.3,
+//              128 190 / 194
+// One set over and over, which the memory-side cache then holds, is up to 10 % slower through LDS from 96
+// to 250 MiB in place, where it streams: what lies between two calls of a caller is not known here.
 static bool faster_through_lds(const vr_ctx *ctx, const AlgoInfo *a, size_t read_bytes, bool in_place) {
   const TuningOverrides &o = ctx->tune;
   if (o.block != -1 || o.waves_per_cu != -1 || o.unroll != -1 || o.nt_load != -1 || o.nt_store != -1 || o.oneshot != -1 ||
@@ -627,11 +632,11 @@ static bool faster_through_lds(const vr_ctx *ctx, const AlgoInfo *a, size_t read
   const size_t MiB = (size_t)1 << 20;
   const auto within = [&](size_t from, size_t to) { return read_bytes >= from * MiB && read_bytes < to * MiB; };
   const size_t any = (size_t)-1 / MiB;
-  if (a->allgather) return read_bytes >= (ctx->nranks == 2 ? 14 : ctx->nranks == 4 ? 10 : 6) * MiB;
+  if (a->allgather) return ctx->nranks == 2 ? within(14, any) : ctx->nranks == 4 ? within(10, any) : within(14, 90);
   switch (ctx->nranks) {
-    case 2: return within(18, any);
-    case 4: return in_place ? within(88, 256) : within(20, 256);
-    case 8: return in_place ? within(4, 15) || within(80, 256) : within(5, 64) || within(88, 256);
+    case 2: return in_place ? within(60, any) : within(28, any);
+    case 4: return in_place ? within(96, any) : within(28, any);
+    case 8: return in_place ? within(4, 15) || within(112, 1200) : within(5, 64) || within(112, 640);
     default: return within(0, 40) || (in_place ? within(96, 256) : within(88, 129));   // 16
   }
 }

@@ -156,25 +156,24 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
       if (nranks == 4 && reads >= 192 * MiB) p.wgs_per_cu = 3;
       break;
     case WIRE_ALLGATHER:
-      // One vector per lane, so that the N waves of a work-group each write one KiB, and 64 KiB of a
-      // slice in a row on an XCD, where the inputs of three calls fit the memory-side cache (one /
-      // two / four vectors, R = 1: every XCD every eighth KiB; 8 ranks 24 MiB 32.3 / 34.3 / 35.6, R = 1 32.1,
-      // 48 MiB 60.0 / 67.6 / 67.8, 64 MiB 80.3 / 90.0 / 89.6; 4 ranks 32 MiB 23.9 / 25.1 / 24.3, R = 1 24.2, 64 MiB
-      // 46.1 / 47.6 / 47.4; 2 ranks 24 MiB 11.8 / 12.0 / 11.7, 64 MiB 28.8 / 28.8 / 27.9).  Beyond, one
-      // KiB loaded by a work-group is too little in flight: two vectors, R = 1 (8 ranks 80 MiB 119 / 113, 128 MiB
-      // 251 / 185; 4 ranks 96 MiB 84.0 / 76.2, 200 MiB 195 / 163; 2 ranks 128 MiB 62.1 / 63.0).  Below, where
-      // the start of a launch counts: two vectors (8 ranks 6 MiB 9.45 / 9.26; 4 ranks 6 MiB 5.58 / 5.26).
-      if (nranks == 8) {
-        p.unroll = reads >= 7 * MiB && reads < 72 * MiB ? 1 : 2;
-        p.run = reads < 7 * MiB ? 16 : reads < 72 * MiB ? 64 : 1;
-      } else if (nranks == 4) {
-        p.unroll = reads >= 10 * MiB && reads < 88 * MiB ? 1 : 2;
-        p.run = reads < 88 * MiB ? 64 : 1;
-      } else {
-        p.unroll = reads < 14 * MiB ? 2 : 1;
-        if (reads >= 20 * MiB && reads < 88 * MiB) p.unroll = 4, p.wgs_per_cu = 3;
-        p.run = reads < 88 * MiB ? 64 : 1;
-      }
+      // Vectors per lane, work-groups per CU and KiBs of a slice in a row on an XCD (run), us with three sets
+      // of buffers in turn (inputs cached) / with as many as no cache holds.  One vector, one KiB loaded
+      // by N waves, is the best there is for cached inputs and the worst for others: 8 ranks 32 MiB 41.4 /
+      // 63.1, 4 ranks 24.0 / 32.3.
+      //   4 ranks  two, run 64: 12 MiB 10.0 / 12.5, 32 MiB 25.2 / 27.5; four, four per CU, run 64: 12 MiB 10.9 / 12.6,
+      //            16 MiB 13.1 / 15.3, 32 MiB 24.6 / 27.0, 64 MiB 48.2 / 52.0, 128 MiB 101.7; uncapped 32 MiB 24.6 /
+      //            28.2, 128 MiB 114.7
+      //   8 ranks  two, run 64: 12 MiB 18.6 / 21.7, 32 MiB 46.7 / 50.1, 64 MiB 87.3 / 97.2, 128 MiB 194; no run (200 MiB)
+      //            301, run 64 302; four, three per CU: 12 MiB 21.5 / 23.4, 32 MiB 44.7 / 50.1, 64 MiB 97.3 / 102.4
+      //   2 ranks  four, six per CU, run 64: 16 MiB 8.3 / 10.0, 64 MiB 28.8 / 32.7, 128 MiB 63.8; two 8.4 / 10.3, 29.3 /
+      //            32.9, 65.0; one, no run 8.7 / 10.6, 29.4 / 33.2, 62.9
+      p.run = 64;
+      if (nranks == 4 && reads >= 14 * MiB) p.unroll = 4, p.wgs_per_cu = 4;
+      else if (nranks == 2 && reads >= 96 * MiB) p.unroll = 1, p.run = 1;
+      else if (nranks == 2 && reads >= 14 * MiB) p.unroll = 4, p.wgs_per_cu = 6;
+      else p.unroll = 2;
+      if (nranks != 4 && reads < 7 * MiB) p.run = 16;
+      if (nranks == 8 && reads >= 90 * MiB) p.run = 1;
       break;
   }
   return p;

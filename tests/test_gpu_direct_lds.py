@@ -41,8 +41,8 @@ def call(oracle, ctx, algo, ins, form, registers):
     return got
 
 
-@pytest.mark.parametrize("nranks,algo,mib", [(2, "simple", 19), (2, "small_ring", 66), (4, "bisect", 21), (4, "small_pcie", 89),
-                                             (8, "small", 6), (8, "simple_ring", 14), (8, "bisect", 40), (8, "simple_transmit", 90),
+@pytest.mark.parametrize("nranks,algo,mib", [(2, "simple", 62), (2, "small_ring", 66), (4, "bisect", 29), (4, "small_pcie", 97),
+                                             (8, "small", 6), (8, "simple_ring", 14), (8, "bisect", 40), (8, "simple_transmit", 113),
                                              (16, "bisect", 1), (16, "bisect", 30), (16, "bisect", 100)])
 def test_same_as_through_registers(oracle, nranks, algo, mib):
     ctx = vr.VirtualRanks(nranks)
@@ -67,7 +67,7 @@ def test_same_as_through_registers(oracle, nranks, algo, mib):
     ctx.close()
 
 
-@pytest.mark.parametrize("nranks,mib", [(2, 15), (4, 11), (8, 7), (8, 75)])
+@pytest.mark.parametrize("nranks,mib", [(2, 15), (2, 97), (4, 11), (4, 15), (8, 15)])
 @pytest.mark.parametrize("form", ["apart", "own slot", "the next rank's slot"])
 def test_gather_same_as_through_registers(oracle, nranks, mib, form):
     """Inputs of their own, and inputs that already are their slot of an output."""
