@@ -154,9 +154,11 @@ enum GroupPolicy : int {
 };
 struct GroupPlan {
   GroupPolicy policy;
-  int unroll;       // 16-byte vectors per lane and message: 1 or 2, or 4 for all-to-all flows at 8 ranks
+  int unroll;       // 16-byte vectors per lane and message: 1; 2 at 8 and 16 ranks; 4 at 8 ranks, not for the ring;
+                    // all-gather: 1, 2 or 4
   int wgs_per_cu;   // residency cap, 0 = none
   int run = 1;      // all-gather: work-groups in a row on an XCD (Tuning::run), a power of two up to 128
+  bool columns = false;   // ring: a work-group has all N chunks of a column, not one
   size_t segment_bytes = (size_t)1 << 30;   // bytes of a chunk one launch covers (32-bit offsets); multiple of 16
 };
 hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow, int nranks, DType dtype,

@@ -20,7 +20,7 @@
 // times the algorithmic bytes at the L2 / fabric boundary, which carries about
 // 8 TB/s however much of it the memory-side cache serves; here only inputs and
 // outputs cross it.  ParallelTransmit, 8 ranks in place: 256 MiB per rank 2196 us through memory,
-// 670 us (6.4 TB/s); RingTransmit, 4 x 8 MB: 39.4, 10.8 us; all-gather, 8 x 1 MB: 51.6, 11.6 us.
+// 670 us (6.4 TB/s); RingTransmit, 4 x 8 MB: 39.4, 10.7 us; all-gather, 8 x 1 MB: 51.6, 11.8 us.
 // Small launches are bound by the chain from a wave's load to its store.  With flag words for
 // every message, the owner's N - 1 additions in one wave and a copy of the sum for each peer it was
 // longer: parallel, 8 x 1 MiB bfloat16 4.62 us, now 3.72, of 64 bytes less 5.51, now 3.93; 8 x 8 MiB less
@@ -84,9 +84,9 @@ struct Msg {
 };
 
 // Where a chunk lies in every rank's buffer (wl::wire_span), by what chunks are known to start
-// on.  GRAIN: what wires are laid on, 128-byte lines or, where a row of the grid sweeps one chunk,
-// KiBs (parallel, 8 x 8 MiB less 64 bytes 28.6 -> 27.1 us, bisect 8 x 16 MiB less 64 56.2 -> 54.7; ring and
-// all-gather, which have a wire more then, lose 1 %).  ON_LINES: none of the arithmetic for other starts (the extra scalar instructions of eight
+// on.  GRAIN: what wires are laid on, KiBs (parallel, 8 x 8 MiB less 64 bytes on 128-byte lines 28.6 us, now
+// 27.1, bisect 8 x 16 MiB less 64 56.2, 54.7) or, in the ring by columns, which would have N more wires
+// then, lines (4 x 8 MB 10.9 us, on KiBs 11.0).  ON_LINES: none of the arithmetic for other starts (the extra scalar instructions of eight
 // waves per 8 KiB cost 7 % at 8 x 32 MiB).  ON_VECTORS: messages of 16 bytes, no vector straddles
 // a start.
 enum Starts : int { ON_LINES, ON_VECTORS, ON_HALVES };
@@ -284,21 +284,45 @@ __global__ __launch_bounds__(64 * N) void k_group_allgather(GroupArgs<N> a) {
 }
 
 // ---- RingTransmit (sequential_transmit.hpp:429-516) --------------------------------------
+// Row c of the grid sweeps chunk c.  Rank c sends its message, ranks c + 1, c + 2, ... each add theirs
+// and send on; the last one's sum lies in a slot that all ranks gather from (the reference
+// forwards it rank by rank).  Slot k holds what the rank of place k sent, flag k says so.
+// For sizes where a launch is bound by its start or by HBM (group_plan).
+template <int N, int DT, int U, Starts S, int LD, int ST>
+__global__ __launch_bounds__(64 * N) void k_group_ring(GroupArgs<N> a) {
+  VR_GROUP_PROLOGUE;
+  Poll poll;
+  const Sinks<U, N, N> sk(lds, lane);
+  const int c = (int)blockIdx.y, place = operand_of<N, ORDER_ROTATED>(r, c);
+  const auto at = span_of<S, U, 1024>(a, c, lane);
+  Msg<U> v = load<U, LD>(src, at);
+  meet();   // all flag words are zero from here on
+  poll.arm(a);
+  if (place > 0) {
+    poll.until([&] { return sk.look(place - 1) != 0; });
+    add<DT, U>(v, sk.get(place - 1));
+  }
+  sk.put(place, v);
+  sk.publish();
+  sk.raise(place, 1);
+  if (place < N - 1) {
+    poll.until([&] { return sk.look(N - 1) != 0; });
+    v = sk.get(N - 1);
+  }
+  store<U, ST>(dst, at, v);
+}
+
+// The same with all N chunks of a column in one work-group: the hops of the N rings overlap.
 // A rank's sink is a ring of slots fed by its predecessor; flag r counts the messages
-// delivered to rank r.  With N slots nothing more is needed: message k + N comes into the
-// slot of message k, and it is sent after message k + N - 1 was received, which was sent
-// after ..., N - 1 ranks back, message k + 1 of the slot's own rank, and that one is made of
-// (or sent after) message k, read from the slot.  Where N slots of U KiB a rank would take
-// the room of too many work-groups, two slots, and flag N + r counts the messages rank r has
-// taken out, which its predecessor looks at before it reuses one.  A hop is a chain of LDS
-// round trips, and the count and the look at it were two of five: with two slots
-// throughout, 8 x 256 KiB 7.3 us, now 5.9, 8 x 2 MiB 11.6, now 9.8, 4 x 2 MiB 5.2, now 4.6 (14
-// and 6 hops); all-gather 8 x 1 MiB 13.1, now 11.9, 8 x 2 MiB 25.1, now 22.9 (there the 64 KiB of
-// slots also hold a compute unit at two work-groups, which suits its 8 write streams).
+// delivered to rank r, N - 1 of them; finished sums lie in one slot each.  With N slots a rank no
+// message comes into a used slot, and the last is the sum's.  Where N slots of U KiB a rank would
+// take the room of too many work-groups, two slots, and flag N + r counts the messages rank r has
+// taken out, which its predecessor looks at before it reuses one: two LDS round trips more of
+// three a hop (8 x 256 KiB 7.3 us with two slots, 5.9 with N; without forwarding the sums 5.5).
 template <int N, int U>
-struct RingSinks : Sinks<U, N * (N * U <= 8 ? N : 2), 2 * N> {
+struct RingSinks : Sinks<U, N * (N * U <= 8 ? N : 3), 3 * N> {
   static constexpr int kDepth = N * U <= 8 ? N : 2;
-  using Sinks<U, N * kDepth, 2 * N>::Sinks;
+  using Sinks<U, N * (N * U <= 8 ? N : 3), 3 * N>::Sinks;
 };
 
 template <int N, int U>
@@ -322,10 +346,20 @@ struct Ring {
     }
     return m;
   }
+  static __device__ __forceinline__ int sum_slot(int q) { return kDepth == N ? q * N + N - 1 : N * kDepth + q; }
+  __device__ __forceinline__ void send_sum(const Msg<U> &m) const {
+    sk.put(sum_slot(r), m);
+    sk.publish();
+    sk.raise(2 * N + r, 1);
+  }
+  __device__ __forceinline__ Msg<U> recv_sum(int q) const {
+    poll.until([&] { return sk.look(2 * N + q) != 0; });
+    return sk.get(sum_slot(q));
+  }
 };
 
 template <int N, int DT, int U, Starts S, int LD, int ST>
-__global__ __launch_bounds__(64 * N) void k_group_ring(GroupArgs<N> a) {
+__global__ __launch_bounds__(64 * N) void k_group_ring_columns(GroupArgs<N> a) {
   VR_GROUP_PROLOGUE;
   Poll poll;
   const RingSinks<N, U> sk(lds, lane);
@@ -337,17 +371,15 @@ __global__ __launch_bounds__(64 * N) void k_group_ring(GroupArgs<N> a) {
   poll.arm(a);
   ring.send(0, x[0]);
 #pragma unroll
-  for (int i = 1; i < N; ++i) {                            // reduce and forward; the last add starts the gather ring
+  for (int i = 1; i < N; ++i) {                            // reduce and forward; the last is the sum
     add<DT, U>(x[i], ring.recv(i - 1));
-    ring.send(i, x[i]);
+    if (i < N - 1) ring.send(i, x[i]);
   }
+  ring.send_sum(x[N - 1]);
   store<U, ST>(dst, span_of<S, U, 128>(a, (r + 1) % N, lane), x[N - 1]);
 #pragma unroll
-  for (int i = 1; i < N; ++i) {                            // write back, forward except on the last hop
-    const Msg<U> v = ring.recv(N - 2 + i);
-    if (i < N - 1) ring.send(N - 1 + i, v);
-    store<U, ST>(dst, span_of<S, U, 128>(a, (r + 1 + N - i) % N, lane), v);
-  }
+  for (int i = 1; i < N; ++i)                              // the others' sums, the neighbour's first
+    store<U, ST>(dst, span_of<S, U, 128>(a, (r + 1 + N - i) % N, lane), ring.recv_sum((r + N - i) % N));
 }
 
 #undef VR_GROUP_PROLOGUE
@@ -358,7 +390,7 @@ struct Pick {
 };
 
 template <int N, int DT, int LD, int ST, int U, bool LINED>
-Pick pick_flow(WireFlow flow) {
+Pick pick_flow(WireFlow flow, bool columns) {
   constexpr Starts kWhole = LINED ? ON_LINES : ON_VECTORS, kAny = LINED ? ON_LINES : ON_HALVES;
   constexpr uint32_t kSlots = N * U * 1024u;
   if constexpr (N <= 8) {
@@ -366,19 +398,23 @@ Pick pick_flow(WireFlow flow) {
       case WIRE_PARALLEL:
       case WIRE_SEQUENTIAL:
       case WIRE_SIMPLE:
-        if constexpr (U <= (N == 8 ? 4 : 2))
+        if constexpr (U <= (N == 8 ? 4 : 1))
           return {reinterpret_cast<const void *>(&k_group_exchange<N, ORDER_ROTATED, DT, U, kAny, LD, ST>), N, kSlots};
         break;
       case WIRE_RING:
-        if constexpr (U <= (N == 8 ? 2 : 1))
-          return {reinterpret_cast<const void *>(&k_group_ring<N, DT, U, kWhole, LD, ST>), 1, RingSinks<N, U>::kBytes};
+        if (columns) {
+          if constexpr (N >= 4 && U <= (N == 8 ? 2 : 1))
+            return {reinterpret_cast<const void *>(&k_group_ring_columns<N, DT, U, LINED ? ON_LINES : ON_VECTORS, LD, ST>), 1, RingSinks<N, U>::kBytes};
+        } else if constexpr (U <= (N >= 4 ? 2 : 1)) {
+          return {reinterpret_cast<const void *>(&k_group_ring<N, DT, U, kWhole, LD, ST>), N, kSlots + N * 4u};
+        }
         break;
       case WIRE_ALLGATHER:   // no adds: one instantiation serves both element types
         return {reinterpret_cast<const void *>(&k_group_allgather<N, U, kWhole, LD, ST>), N, U * 1024u};
       default: break;
     }
   }
-  if constexpr (N >= 4 && U <= (N == 8 ? 4 : 2)) {
+  if constexpr (N >= 4 && U <= (N == 8 ? 4 : N == 16 ? 2 : 1)) {
     if (flow == WIRE_BISECT)
       return {reinterpret_cast<const void *>(&k_group_exchange<N, ORDER_BISECT, DT, U, kAny, LD, ST>), N, kSlots};
   }
@@ -386,30 +422,30 @@ Pick pick_flow(WireFlow flow) {
 }
 
 template <int DT, int LD, int ST, bool LINED, int U>
-Pick pick_ranks(WireFlow flow, int nranks) {
+Pick pick_ranks(WireFlow flow, int nranks, bool columns) {
   switch (nranks) {
-    case 2: return pick_flow<2, DT, LD, ST, U, LINED>(flow);
-    case 4: return pick_flow<4, DT, LD, ST, U, LINED>(flow);
-    case 8: return pick_flow<8, DT, LD, ST, U, LINED>(flow);
-    case 16: return pick_flow<16, DT, LD, ST, U, LINED>(flow);
+    case 2: return pick_flow<2, DT, LD, ST, U, LINED>(flow, columns);
+    case 4: return pick_flow<4, DT, LD, ST, U, LINED>(flow, columns);
+    case 8: return pick_flow<8, DT, LD, ST, U, LINED>(flow, columns);
+    case 16: return pick_flow<16, DT, LD, ST, U, LINED>(flow, columns);
     default: return {nullptr, 0, 0};
   }
 }
 
 template <int DT, int LD, int ST, bool LINED>
-Pick pick_unroll(WireFlow flow, int nranks, int unroll) {
-  return unroll == 4   ? pick_ranks<DT, LD, ST, LINED, 4>(flow, nranks)
-         : unroll == 2 ? pick_ranks<DT, LD, ST, LINED, 2>(flow, nranks)
-                       : pick_ranks<DT, LD, ST, LINED, 1>(flow, nranks);
+Pick pick_unroll(WireFlow flow, int nranks, int unroll, bool columns) {
+  return unroll == 4   ? pick_ranks<DT, LD, ST, LINED, 4>(flow, nranks, columns)
+         : unroll == 2 ? pick_ranks<DT, LD, ST, LINED, 2>(flow, nranks, columns)
+                       : pick_ranks<DT, LD, ST, LINED, 1>(flow, nranks, columns);
 }
 
 template <int LD, int ST>
-Pick pick_type(WireFlow flow, int nranks, DType dtype, int unroll, bool lined) {
+Pick pick_type(WireFlow flow, int nranks, DType dtype, int unroll, bool lined, bool columns) {
   if (lined)
-    return dtype == DT_BF16 ? pick_unroll<DT_BF16, LD, ST, true>(flow, nranks, unroll)
-                            : pick_unroll<DT_F16, LD, ST, true>(flow, nranks, unroll);
-  return dtype == DT_BF16 ? pick_unroll<DT_BF16, LD, ST, false>(flow, nranks, unroll)
-                          : pick_unroll<DT_F16, LD, ST, false>(flow, nranks, unroll);
+    return dtype == DT_BF16 ? pick_unroll<DT_BF16, LD, ST, true>(flow, nranks, unroll, columns)
+                            : pick_unroll<DT_F16, LD, ST, true>(flow, nranks, unroll, columns);
+  return dtype == DT_BF16 ? pick_unroll<DT_BF16, LD, ST, false>(flow, nranks, unroll, columns)
+                          : pick_unroll<DT_F16, LD, ST, false>(flow, nranks, unroll, columns);
 }
 
 }  // namespace
@@ -418,12 +454,12 @@ hipError_t launch_wire_group(hipStream_t s, const DeviceInfo &dev, WireFlow flow
                              const PtrTable &in, const PtrTable &out, size_t chunk_bytes, const GroupPlan &plan,
                              uint32_t spin_limit, uint32_t *status) {
   // what wires are laid on (span_of)
-  const uint32_t grain = flow == WIRE_RING ? 128u : 1024u;
+  const uint32_t grain = plan.columns ? 128u : 1024u;
   const bool lined = (((uintptr_t)out.p[0] | chunk_bytes) & (grain - 1u)) == 0;
   const Pick k =
-      plan.policy == GROUP_STREAM     ? pick_type<kStreamLoad, kStreamStore>(flow, nranks, dtype, plan.unroll, lined)
-      : plan.policy == GROUP_RESIDENT ? pick_type<0, 0>(flow, nranks, dtype, plan.unroll, lined)
-                                      : pick_type<0, kStreamStore>(flow, nranks, dtype, plan.unroll, lined);
+      plan.policy == GROUP_STREAM     ? pick_type<kStreamLoad, kStreamStore>(flow, nranks, dtype, plan.unroll, lined, plan.columns)
+      : plan.policy == GROUP_RESIDENT ? pick_type<0, 0>(flow, nranks, dtype, plan.unroll, lined, plan.columns)
+                                      : pick_type<0, kStreamStore>(flow, nranks, dtype, plan.unroll, lined, plan.columns);
   if (!k.fn) return hipErrorInvalidValue;
   const size_t wire = 1024u * (size_t)plan.unroll;   // payload of one wave
   uint32_t lds = k.lds;

@@ -128,32 +128,32 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
     case WIRE_BISECT:
     case WIRE_SEQUENTIAL:
     case WIRE_SIMPLE:
-      if (nranks <= 4) {
-        // 2 ranks in place 10 MiB 4.59, two vectors 4.03; 12 MiB 5.23 / 4.82; 17 MiB 6.81 / 7.04; 4 ranks 10
-        // MiB 4.41 / 4.09, 17 MiB 7.32 / 6.12, 20 MiB 7.83 / 8.24
-        p.unroll = reads >= 9 * MiB && reads < 16 * MiB ? 2 : 1;
-      } else if (nranks == 8) {
-        // In place two / four vectors: 8 MiB 3.83 / 4.05, 12 MiB 5.03 / 5.36, 14 MiB 6.31 / 5.92, 40 MiB
-        // 14.4 / 13.9; one / four: 50 MiB out of place 16.9 / 16.3, 64 MiB 21.2 / 22.1, out of place 20.1 / 22.0,
-        // 120 MiB 43.9 / 47.2 (three work-groups a CU 45.6 with one vector)
-        p.unroll = reads < 13 * MiB ? 2 : reads < 56 * MiB ? 4 : 1;
+      // (Single sizes differ by up to 30 % either way, with the lengths' place among the channels; means of
+      // 30 lengths and two placements each, ratios of times.  Two vectors / one at 2 ranks 0.94 from 13 MiB on,
+      // at 4 ranks 0.99 in place, 0.91 out of place; below 13 MiB even.)
+      if (nranks == 8) {
+        // two / four, in place and out of place: 6 to 9 MiB 0.98, 0.99; 13 to 20 MiB 1.07, 1.07; 20 to 56 MiB
+        // 1.05, 1.01; 56 to 100 MiB 1.05, 1.01 (one / four 1.02, 1.00); one / four at 120 MiB 0.93
+        p.unroll = reads < 13 * MiB ? 2 : reads < 96 * MiB ? 4 : 1;
         // Chunks of 24 MiB and more that are multiples of 1 MiB start all streams on one channel: two
         // vectors with three work-groups a CU 668 us at 8 x 256 MiB, one 681; on other lengths 665, 653.
         if (reads >= 1536 * MiB && reads % (64 * MiB) == 0) p.unroll = 2, p.wgs_per_cu = 3;
-      } else {
-        // 16 ranks, one / two: 6 MiB in place 4.89 / 4.74, 24 MiB 10.1 / 9.9, 64 MiB 22.3 / 25.3, 192 MiB 68.0 /
-        // 70.0, out of place 68.9 / 70.7 (bfloat16 73.0 / 72.0)
-        p.unroll = reads < 56 * MiB ? 2 : 1;
+      } else if (nranks == 16) {
+        // one / two: 6 to 9 MiB 1.03, 9 to 13 MiB 1.09, 13 to 35 MiB 1.02, 35 to 56 MiB 0.98; 192 MiB 68.0 / 70.0 us,
+        // out of place 68.9 / 70.7 (bfloat16 73.0 / 72.0)
+        p.unroll = reads < 35 * MiB ? 2 : 1;
       }
       break;
     case WIRE_RING:
-      // 8 x 16 MiB 65.1 -> 48.9 us; 8 x 4 MiB even, 8 x 2 MiB 8.4, two: 9.9; 8 x 32 MiB 97.7, two: 108.8
-      if (nranks == 8 && reads >= 32 * MiB && reads <= 192 * MiB) p.unroll = 2;
-      // Four ranks, streaming: 48 KiB of loads per CU in flight instead of 128.
-      // 4 x 64 MiB 106 -> 94 us, 4 x 128 MiB 190.5 -> 169.5; 4 x 32 MiB 50.7, capped 50.9.  (Eight
-      // ranks with one vector: their 64 KiB of slots hold a compute unit at two work-groups anyway;
-      // with two vectors no cap was timed.)
-      if (nranks == 4 && reads >= 192 * MiB) p.wgs_per_cu = 3;
+      // By columns / one chunk a work-group (8 and 4 ranks with two vectors, 2 ranks one), ratios of times where
+      // single lengths scatter: 8 ranks 2 MiB 5.25 / 4.23 us, 6 MiB 5.8 / 5.2, 9 MiB 0.98, out of place 1.05, 12 MiB 0.87,
+      // 0.98, 13 to 90 MiB 0.90, 0.98, 110 MiB 48.3 / 46.6, 220 MiB 91.8 / 81.5, 1000 MiB 419 / 346; 4 ranks 7 to 90 MiB
+      // 0.97, 0.96, 105 MiB 1.10, 1.08, 420 MiB 151 / 141, 1000 MiB 349 / 336; 2 ranks 9 MiB 4.3 / 4.2 to 4.8, 18 MiB
+      // 7.9 / 7.8, 76 MiB 28.4 / 27.1, 600 MiB 200 / 190.
+      p.columns = nranks == 8 ? reads >= 10 * MiB && reads < 100 * MiB : nranks == 4 && reads < 100 * MiB;
+      p.unroll = p.columns || nranks == 2 ? 1 : 2;
+      // columns, one / two vectors: 8 x 2 MiB 8.4 / 9.9, 8 x 4 MiB even
+      if (p.columns && nranks == 8 && reads >= 32 * MiB) p.unroll = 2;
       break;
     case WIRE_ALLGATHER:
       // Vectors per lane, work-groups per CU and KiBs of a slice in a row on an XCD (run), us with three sets

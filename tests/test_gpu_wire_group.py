@@ -66,11 +66,12 @@ def test_ragged_sizes_of_the_larger_launches(oracle, algo, mib):
 
 @pytest.mark.parametrize("nranks,algo,kib", [(2, "simple", 12 * 1024), (4, "bisect", 12 * 1024), (8, "parallel", 8 * 1024),
                                              (8, "small_pcie", 14 * 1024), (8, "bisect", 80 * 1024),
-                                             (8, "simple_transmit", 20 * 1024), (16, "bisect", 90 * 1024)])
+                                             (8, "simple_transmit", 20 * 1024), (16, "bisect", 30 * 1024),
+                                             (8, "simple_ring", 14 * 1024), (8, "small_ring", 110 * 1024)])
 def test_vectors_per_lane(oracle, nranks, algo, kib):
-    """Two and four vectors per lane: messages of 2 and 4 KiB whose last ends early, and a wave's
-    share of the sums in each width."""
-    msg = 16 if algo == "small_pcie" else 8
+    """One, two and four vectors per lane: messages of 1, 2 and 4 KiB whose last ends early, and a wave's
+    share of the sums in each width; rings by columns and by chunks."""
+    msg = 16 if algo.endswith(("pcie", "ring")) else 8
     ctx = vr.VirtualRanks(nranks)
     chunk = kib * 1024 // nranks ** 2 // 4096 * 4096
     for k, tail in enumerate((0, msg, 1024 - msg, 3072 + msg)):
