@@ -606,24 +606,28 @@ static int resolve_transport(const AlgoInfo *a, int transport, int *out) {
 // prologue.  This says for which calls it is the faster; calls with a grid or a tuning key of the
 // register kernels take those.  us per call, register kernels / through LDS, with three sets of buffers
 // in turn, and as many as no cache holds where a ratio follows (there 5 to 30 % faster nearly throughout):
-//   in place   2 ranks 24 MiB 12.3 / 13.4, 40 18.3 / 18.6, 65 22.2 / 20.3, 100 38.2 / 33.9, 161 63.8 / 51.8 (1.21), 1007 334 / 309
-//              4 ranks 50 MiB 16.2 / 16.6, 79 24.7 / 25.2, 100 38.5 / 34.8 (1.17), 164 62.2 / 54.5, 391 125 / 124, 2048 647 / 643
-//              8 ranks 8 MiB 3.89 / 3.51 (1.16), 10 5.01 / 4.11, 12 (1.09), 16 7.05 / 7.15, 67 21.7 / 22.5, 81 to 100
-//              mixed (0.90 to 1.08; 1.17), 120 51.3 / 49.1 (1.14), 130 54.7 / 46.7, 224 101 / 79, 512 164 / 162, 1024
-//              327 / 323, 1963 639 / 662
-//              16 ranks 2 MiB 4.99 / 3.33, 16 8.4 / 6.7, 39 15.4 / 14.3, 63 22.4 / 23.7, 100 39.3 / 37.4, 196 90 / 72 (1.33),
-//              718 250 / 255; bfloat16 40 MiB 16.0 / 15.5, 90 34.7 / 35.0, 192 85.8 / 72.3, 512 176 / 184
-//   out of     2 ranks 12 MiB 5.4 / 7.0, 24 10.5 / 10.9, 32 14.8 / 13.0 (1.09), 66 20.3 / 19.9, 113 41.6 / 37.5, 1019 331 / 315
-//   place      4 ranks 24 MiB 10.8 / 11.4, 32 18.1 / 13.7 (1.19), 66 20.8 / 20.2 (1.15), 113 45.7 / 38.6, 697 222 / 220
-//              8 ranks 4 MiB 3.27 / 3.35, 8 3.89 / 3.33 (1.17), 33 11.8 / 11.6 (1.08), 63 20.5 / 20.2, 80 25.5 / 26.7,
-//              90 to 107 mixed (0.84 to 1.18), 120 (1.09), 228 79.8 / 78.2, 256 82.2 / 81.4, 512 163.6 / 162.3, 686 227 / 228
-//              16 ranks 40 MiB 14.7 / 13.9, 64 22.0 / 22.6, 99 40.2 / 37.0 (1.15), 128 52 / 47, 190 70.1 / 69.9
+//   in place   2 ranks 24 MiB 12.3 / 13.4, 40 12.1 / 12.0, 50 16.0 / 14.4, 70 20.5 / 18.8, 112 42.5 / 39.7, 250 92.5 / 85.7,
+//              1007 334 / 309; one set over and over 70 MiB 21.1 / 18.9, 160 42.6 / 38.9
+//              4 ranks 50 MiB 16.2 / 16.6, 79 24.7 / 25.2, 96 34.5 / 32.1, 160 59.6 / 58.1, 391 125 / 124, 2048 647 / 643;
+//              one set 96 to 250 MiB even
+//              8 ranks 8 MiB 3.89 / 3.51 (1.16), 10 5.01 / 4.11, 12 (1.09), 16 7.05 / 7.15, 67 21.7 / 22.5, 81 to 108
+//              three sets 1.03 to 1.31 times as fast, one set 0.87 to 0.98; 112 50.6 / 40.2, 160 67.5 / 59.1, 250 102.8 / 86.4 (one
+//              set even, lengths that are no whole KiBs 2 to 9 % slower); 512 164 / 162, 1024 327 / 323, 1963 639 / 662
+//              16 ranks 2 MiB 4.99 / 3.33, 16 8.4 / 6.7, 39 15.4 / 14.3, 63 22.4 / 23.7, 93 to 109 MiB 0.93 to 0.97 times as
+//              fast, 122 to 167 1.10 to 1.14, 192 80.8 / 69.3; one set 1.12 to 1.20; 718 250 / 255; bfloat16 512 176 / 184
+//   out of     2 ranks 12 MiB 5.4 / 7.0, 24 10.5 / 10.9, 32 14.8 / 13.0 (1.09), 66 20.3 / 19.9, 96 to 126 MiB 1.02 to 1.07
+//   place      times as fast, one set too; 1019 331 / 315
+//              4 ranks 24 MiB 10.8 / 11.4, 32 18.1 / 13.7 (1.19), 66 20.8 / 20.2 (1.15), 96 to 127 MiB 1.09 to 1.14 times as
+//              fast, one set 1.00 to 1.03; 697 222 / 220
+//              8 ranks 4 MiB 3.27 / 3.35, 8 3.89 / 3.33 (1.17), 33 11.8 / 11.6 (1.08), 55 to 85 MiB 0.99 to 1.09 times as fast,
+//              one set 0.99 to 1.03; 90 to 125 MiB 1.00 to 1.17, one set 0.96 to 1.05; 256 82.2 / 81.4, 512 163.6 / 162.3,
+//              686 227 / 228
+//              16 ranks 40 MiB 14.7 / 13.9, 64 22.0 / 22.6, 75 to 130 MiB 1.01 to 1.15 times as fast, one set 1.04 to 1.08;
+//              190 70.1 / 69.9
 //   all-gather 2 ranks 12 MiB 5.8 / 6.3, 16 8.7 / 8.3, 64 29.4 / 28.8, 128 65.5 / 62.9
 //              4 ranks 8 MiB 7.0 / 6.9, 12 11.0 / 10.0, 32 25.8 / 24.6 (1.07), 64 50.9 / 48.2, 128 104 / 102
 //              8 ranks 8 MiB 12.4 / 12.0 (0.97), 12 19.3 / 18.6 (0.98), 24 36.3 / 35.1 (1.03), 32 52.2 / 46.7, 64 98.1 / 87.3,
 //              128 190 / 194
-// One set over and over, which the memory-side cache then holds, is up to 10 % slower through LDS from 96
-// to 250 MiB in place, where it streams: what lies between two calls of a caller is not known here.
 static bool faster_through_lds(const vr_ctx *ctx, const AlgoInfo *a, size_t read_bytes, bool in_place) {
   const TuningOverrides &o = ctx->tune;
   if (o.block != -1 || o.waves_per_cu != -1 || o.unroll != -1 || o.nt_load != -1 || o.nt_store != -1 || o.oneshot != -1 ||
@@ -636,8 +640,8 @@ static bool faster_through_lds(const vr_ctx *ctx, const AlgoInfo *a, size_t read
   switch (ctx->nranks) {
     case 2: return in_place ? within(60, any) : within(28, any);
     case 4: return in_place ? within(96, any) : within(28, any);
-    case 8: return in_place ? within(4, 15) || within(112, 1200) : within(5, 64) || within(112, 640);
-    default: return within(0, 40) || (in_place ? within(96, 256) : within(88, 129));   // 16
+    case 8: return in_place ? within(4, 15) || within(112, 1200) : within(5, 640);
+    default: return within(0, 40) || (in_place ? within(120, 256) : within(70, 129));   // 16
   }
 }
 
@@ -659,7 +663,8 @@ static int run_allreduce(vr_ctx *ctx, hipStream_t s, const Prepared &p, int tran
     return VR_OK;
   }
   if (!t.force_blocks_per_rank && faster_through_lds(ctx, p.a, p.bytes_all_ranks, p.in_place))
-    return group_launch(ctx, s, p.a->order == ORDER_BISECT ? WIRE_BISECT : WIRE_PARALLEL, p.in, p.out, p.chunk_elems * 2);
+    return group_launch(ctx, s, p.a->order == ORDER_BISECT ? WIRE_BISECT : WIRE_PARALLEL, p.in, p.out, p.chunk_elems * 2,
+                        true);
   hipError_t e = launch_direct_allreduce(s, ctx->dev, t, ctx->nranks, p.a->order, ctx->dtype, p.in,
                                          p.out, p.chunk_elems);
   if (e != hipSuccess) return fail_hip(e, "launch_direct_allreduce");
@@ -783,7 +788,7 @@ static int run_allgather(vr_ctx *ctx, hipStream_t s, const PreparedGather &p, in
   }
   if (transport != VR_TRANSPORT_DEFAULT && transport != VR_TRANSPORT_DIRECT) return fail(VR_ERR_INVALID, "bad transport");
   if (!t.force_blocks_per_rank && faster_through_lds(ctx, p.a, (size_t)ctx->nranks * nelems * 2, false)) {
-    if (int rc = group_launch(ctx, s, WIRE_ALLGATHER, p.in, p.out, nelems * 2)) return rc;
+    if (int rc = group_launch(ctx, s, WIRE_ALLGATHER, p.in, p.out, nelems * 2, true)) return rc;
   } else {
     hipError_t e = launch_direct_allgather(s, ctx->dev, t, ctx->nranks, p.in, p.out, nelems);
     if (e != hipSuccess) return fail_hip(e, "launch_direct_allgather");

@@ -137,6 +137,7 @@ int wire_launch_ctx(vr_ctx *c, hipStream_t s, const AlgoInfo *a, const PtrTable 
                     uint32_t *flags_used);
 
 // A launch whose messages travel through LDS (vr_wire_group.hip); it needs no scratch.
-int group_launch(vr_ctx *c, hipStream_t s, WireFlow flow, const PtrTable &in, const PtrTable &out, size_t chunk_bytes);
+int group_launch(vr_ctx *c, hipStream_t s, WireFlow flow, const PtrTable &in, const PtrTable &out, size_t chunk_bytes,
+                 bool direct);
 
 }  // namespace vr

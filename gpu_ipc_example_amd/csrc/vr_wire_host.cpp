@@ -104,7 +104,7 @@ static uint32_t spin_limit_of(const vr_ctx *c) {
 
 // Launch shape of the work-group form.  `reads` = bytes of all ranks' inputs.  Lines lie where
 // calls that take three sets of buffers in turn change sides, us per call with each:
-static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_place) {
+static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_place, bool direct) {
   const size_t MiB = (size_t)1 << 20;
   GroupPlan p = {GROUP_MIXED, 1, 0};
   // Cache policies:
@@ -113,14 +113,17 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
   //    fit the memory-side cache); beyond it streaming wins as soon as the buffers do not all fit
   //    (2 / 4 / 8 / 16 ranks, 73 MiB 22.1 / 24.1 / 25.0 / 25.7 cacheable, 24.0 / 26.2 / 27.4 / 30.6
   //    streamed; 79 to 86 MiB even at 2 and 4 ranks, at 8 and 16 ranks cacheable is 2 to 5 % ahead up to
-  //    91);
+  //    91).  Calls of the direct transport stay cacheable as long as one set of buffers fits, as its register kernels
+  //    do: one set over and over 8 x 14 MiB 29.2 us, streamed 38.6, 8 x 28 MiB 54.8, 72.2, 2 x 96 MiB 47.0,
+  //    60.0; three sets 39.9 / 38.4, 80.9 / 71.7, 68.2 / 59.9;
   //  * out of place up to 100 MiB of inputs results are streamed past inputs that may stay (4 x 14
   //    MiB 17.7, everything streamed 21.2), beyond it everything streams (4 x 28 MiB 39.3 / 38.6,
-  //    2 x 58 39.5 / 38.3);
+  //    2 x 58 39.5 / 38.3; the direct transport beyond 128 MiB, as its register kernels: 8 x 16 MiB on one
+  //    set 32.5, streamed 46.2);
   //  * all-gather: results are streamed past the inputs at every size, they are N times as
   //    long (8 x 19 MiB 256, everything streamed 264; 4 x 32 112, 116).
-  if (in_place) p.policy = reads <= 80 * MiB ? GROUP_RESIDENT : GROUP_STREAM;
-  else if (reads > 100 * MiB && flow != WIRE_ALLGATHER) p.policy = GROUP_STREAM;
+  if (in_place) p.policy = reads <= 80 * MiB || (direct && reads < 256 * MiB) ? GROUP_RESIDENT : GROUP_STREAM;
+  else if (reads > (direct ? 128 : 100) * MiB && flow != WIRE_ALLGATHER) p.policy = GROUP_STREAM;
   // Vectors per lane: fewer and larger work-groups where caches feed them quicker than they
   // start, one vector where HBM does.
   switch (flow) {
@@ -133,8 +136,9 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
       // at 4 ranks 0.99 in place, 0.91 out of place; below 13 MiB even.)
       if (nranks == 8) {
         // two / four, in place and out of place: 6 to 9 MiB 0.98, 0.99; 13 to 20 MiB 1.07, 1.07; 20 to 56 MiB
-        // 1.05, 1.01; 56 to 100 MiB 1.05, 1.01 (one / four 1.02, 1.00); one / four at 120 MiB 0.93
-        p.unroll = reads < 13 * MiB ? 2 : reads < 96 * MiB ? 4 : 1;
+        // 1.05, 1.01; 56 to 100 MiB in place 1.05 (one / four 1.02); one / four at 120 MiB 0.93.  Out of place one / four,
+        // one set over and over and three: 42 MiB 0.99, 0.98, 55 to 70 MiB 0.93, 0.90, 80 to 125 MiB 0.94, 0.93
+        p.unroll = reads < 13 * MiB ? 2 : reads < (in_place ? 96 : 42) * MiB ? 4 : 1;
         // Chunks of 24 MiB and more that are multiples of 1 MiB start all streams on one channel: two
         // vectors with three work-groups a CU 668 us at 8 x 256 MiB, one 681; on other lengths 665, 653.
         if (reads >= 1536 * MiB && reads % (64 * MiB) == 0) p.unroll = 2, p.wgs_per_cu = 3;
@@ -180,12 +184,13 @@ static GroupPlan group_plan(WireFlow flow, int nranks, size_t reads, bool in_pla
 }
 
 namespace vr {
-int group_launch(vr_ctx *c, hipStream_t s, WireFlow flow, const PtrTable &in, const PtrTable &out, size_t chunk_bytes) {
+int group_launch(vr_ctx *c, hipStream_t s, WireFlow flow, const PtrTable &in, const PtrTable &out, size_t chunk_bytes,
+                 bool direct) {
   const int N = c->nranks;
   bool in_place = flow != WIRE_ALLGATHER;
   for (int r = 0; r < N; ++r) in_place = in_place && in.p[r] == out.p[r];
   const size_t reads = (size_t)N * chunk_bytes * (flow == WIRE_ALLGATHER ? 1 : N);
-  GroupPlan plan = group_plan(flow, N, reads, in_place);
+  GroupPlan plan = group_plan(flow, N, reads, in_place, direct);
   if (c->tune.segment_kib != -1) plan.segment_bytes = (size_t)c->tune.segment_kib << 10;
   const hipError_t e = launch_wire_group(s, c->dev, flow, N, c->dtype, in, out, chunk_bytes, plan, spin_limit_of(c),
                                          c->status);
@@ -343,7 +348,7 @@ static int wire_launch(vr_ctx *c, hipStream_t s, const AlgoInfo *a, const PtrTab
   if ((wlch.hist || wlch.always_clear) && takes_group_form(c, user_wires)) {
     *flags_used = chunk_bytes ? 1u : 0u;
     if (seq + *flags_used == 0) *seq_io = 1;   // 0 is never handed out
-    return group_launch(c, s, a->wire_flow(), in, out, chunk_bytes);
+    return group_launch(c, s, a->wire_flow(), in, out, chunk_bytes, false);
   }
   WirePlan plan;
   if (int rc = plan_wire(c, a, chunk_bytes, vec_halves, user_wires, k, &plan)) return rc;

@@ -43,7 +43,7 @@ def call(oracle, ctx, algo, ins, form, registers):
 
 @pytest.mark.parametrize("nranks,algo,mib", [(2, "simple", 62), (2, "small_ring", 66), (4, "bisect", 29), (4, "small_pcie", 97),
                                              (8, "small", 6), (8, "simple_ring", 14), (8, "bisect", 40), (8, "simple_transmit", 113),
-                                             (16, "bisect", 1), (16, "bisect", 30), (16, "bisect", 100)])
+                                             (8, "bisect", 98), (16, "bisect", 1), (16, "bisect", 30), (16, "bisect", 125)])
 def test_same_as_through_registers(oracle, nranks, algo, mib):
     ctx = vr.VirtualRanks(nranks)
     msg = 16 if algo in ("small_ring", "simple_ring", "small_pcie") else 8
