@@ -20,6 +20,9 @@
 // binary16 adds per half2, and N dwordx4 stores; nothing is staged in LDS
 // because no datum is used twice.
 //
+// At the sizes where it is the faster, a call takes the LDS kernels of vr_wire_group.hip instead
+// (faster_through_lds in vr_api.cpp, with both sides measured).
+//
 // Memory is addressed through buffer resources (one per rank and direction,
 // built in scalar registers from the chunk's base pointer and byte length): a
 // lane supplies a 32-bit byte offset, the hardware drops every access at or
