@@ -27,8 +27,8 @@ HBM_PEAK_GBPS = 8000.0
 # (workload, transport) -> (bytes, the summary under profiles/ that derives the
 # figure; a CPU test checks that the file states this very number).
 MEASURED_TRAFFIC_BYTES = {
-    ("cfg3", "direct"): (536914021, "direct_allreduce_bisect_8x32MiB_hbm_traffic.md"),
-    ("cfg4", "direct"): (167799218, "direct_allreduce_bisect_8x32MiB_hbm_traffic.md"),
+    ("cfg3", "direct"): (536886310, "direct_through_lds_kernel_trace.md"),
+    ("cfg4", "direct"): (167802116, "direct_through_lds_kernel_trace.md"),
     ("cfg5_32MiB", "wire"): (536903576, "wire_allreduce_through_lds_8x32MiB.md"),
     ("cfg3", "wire"): (536909720, "wire_allreduce_through_lds_8x32MiB.md"),
 }
@@ -70,7 +70,7 @@ KERNEL_SAMPLE_LAUNCHES = 200
 KERNEL_SAMPLE_MIN_PAIRS = 20
 # p50 kernel execution time of cfg2 in a rocprofv3 kernel trace (microseconds), and the
 # summary under profiles/ that states it; printed beside the in-process figures.
-CFG2_KERNEL_TRACE = (4.20, "direct_allreduce_small_8x1MiB_kernel_trace.md")
+CFG2_KERNEL_TRACE = (3.36, "direct_through_lds_kernel_trace.md")
 
 # --transport: how the virtual ranks exchange data (0 = the protocol's default).
 TRANSPORT = 0
